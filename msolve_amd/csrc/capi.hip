@@ -820,10 +820,13 @@ int band_setup(msa_batch *b, ClassHost &C, bool *changed, bool shared = false)
     }
     const size_t per = (size_t)C.dev.bn * C.dev.bW;
     const size_t need = shared ? per : (size_t)C.nsamp * per;
+    const size_t lper = (size_t)((C.dev.bn + kBandNB - 1) / kBandNB) * 2 * kBandNB * kBandNB;
     if (C.band_cap < need) {
         void *p = nullptr;
         MSA_TRY(dalloc(b, &p, need * sizeof(double)));
         C.dev.band = (double *)p;
+        MSA_TRY(dalloc(b, &p, (shared ? 1 : C.nsamp) * lper * sizeof(double)));
+        C.dev.linv = (double *)p;
         C.band_cap = need;
         upload = true;
     }
@@ -831,9 +834,10 @@ int band_setup(msa_batch *b, ClassHost &C, bool *changed, bool shared = false)
         void *p = nullptr;
         MSA_TRY(dalloc(b, &p, (size_t)C.nsamp * C.dev.bn * sizeof(double)));
         C.dev.by = (double *)p;
-        const int nchunk = (C.dev.bW + kBandChunkRows - 1) / kBandChunkRows;
-        MSA_TRY(dalloc(b, &p, (size_t)C.nsamp * nchunk * kBandNB * sizeof(double)));
-        C.dev.bpart = (double *)p;
+        if (!band_one_launch(C.dev.bn, C.dev.bW)) {
+            MSA_TRY(dalloc(b, &p, (size_t)C.nsamp * C.dev.bn * sizeof(double)));
+            C.dev.bx = (double *)p;
+        }
         MSA_TRY(dalloc(b, &p, (size_t)C.nsamp * sizeof(int)));
         C.dev.bfail = (int *)p;
         upload = true;
@@ -841,6 +845,7 @@ int band_setup(msa_batch *b, ClassHost &C, bool *changed, bool shared = false)
     const long long ss = shared ? 0 : (long long)per;
     if (C.dev.band_ss != ss) {
         C.dev.band_ss = ss;
+        C.dev.linv_ss = shared ? 0 : (long long)lper;
         upload = true;
     }
     if (upload) *changed = true;
@@ -855,34 +860,47 @@ int prepare_band(msa_batch *b)
     return MSA_OK;
 }
 
-int band_backward(msa_batch *b, const ClassDev *cp, int n, int W, int ns, int mode);
-
-// Forward and backward sweeps with the band factor of every sample (in
-// place on by): one launch for bands of at most kBandOneMax rows, else two
-// launch pairs per 64-column block.  mode >= 0: coarsest multigrid level,
-// samples selected by the cycle's mode.
-int band_sweeps(msa_batch *b, const ClassDev *cp, int n, int W, int ns, int mode)
+// Band Cholesky factors of ns samples and the inverses of their diagonal
+// blocks, which the sweeps read.
+int band_factor(msa_batch *b, const ClassDev *cp, int n, int W, int ns)
 {
     hipStream_t s = b->ctx->stream;
-    if (n <= kBandOneMax)
-        return timed(b, KK_OTHER, [&] { return launch_band_solve_one(s, cp, ns, n, mode); });
     for (int k0 = 0; k0 < n; k0 += kBandNB) {
         const int nk = std::min(kBandNB, n - k0), r0 = k0 + nk, m = std::min(n - r0, W - kBandNB);
-        MSA_TRY(timed(b, KK_OTHER, [&] { return launch_band_fwd(s, cp, ns, k0, nk, r0, m, mode); }));
+        MSA_TRY(timed(b, KK_ASSEMBLE, [&] { return launch_chol_diag(s, cp, ns, k0, nk); }));
+        MSA_TRY(timed(b, KK_ASSEMBLE, [&] { return launch_chol_panel(s, cp, ns, k0, nk, r0, m); }));
+        MSA_TRY(timed(b, KK_ASSEMBLE, [&] { return launch_chol_update(s, cp, ns, k0, nk, r0, m); }));
     }
-    return band_backward(b, cp, n, W, ns, mode);
+    return timed(b, KK_ASSEMBLE, [&] { return launch_band_linv(s, cp, ns, n); });
 }
 
-// The backward sweep L^T x = y alone (in place on by), block by block.
+// Backward sweep L^T x = y alone: from `by` (narrow bands, in place) or
+// `bx` (wide ones) into `by`.
 int band_backward(msa_batch *b, const ClassDev *cp, int n, int W, int ns, int mode)
 {
     hipStream_t s = b->ctx->stream;
-    const int last = ((n - 1) / kBandNB) * kBandNB;
-    for (int k0 = last; k0 >= 0; k0 -= kBandNB) {
-        const int nk = std::min(kBandNB, n - k0), r0 = k0 + nk, m = std::min(n - r0, W - kBandNB);
-        MSA_TRY(timed(b, KK_OTHER, [&] { return launch_band_bwd(s, cp, ns, k0, nk, r0, m, mode); }));
-    }
+    if (band_one_launch(n, W))
+        return timed(b, KK_OTHER, [&] { return launch_band_sweep_one(s, cp, ns, n, W, mode, 2); });
+    for (int k = (n - 1) / kBandNB; k >= 0; k--)
+        MSA_TRY(timed(b, KK_OTHER, [&] {
+            return launch_band_sweep_step(s, cp, ns, n, W, k, false, mode);
+        }));
     return MSA_OK;
+}
+
+// Forward and backward sweeps with the band factor of every sample (in
+// place on by): one launch, or one per 64-column block and sweep.  mode >= 0:
+// samples selected by the multigrid cycle's mode.
+int band_sweeps(msa_batch *b, const ClassDev *cp, int n, int W, int ns, int mode)
+{
+    hipStream_t s = b->ctx->stream;
+    if (band_one_launch(n, W))
+        return timed(b, KK_OTHER, [&] { return launch_band_sweep_one(s, cp, ns, n, W, mode, 3); });
+    for (int k = 0; k < (n + kBandNB - 1) / kBandNB; k++)
+        MSA_TRY(timed(b, KK_OTHER, [&] {
+            return launch_band_sweep_step(s, cp, ns, n, W, k, true, mode);
+        }));
+    return band_backward(b, cp, n, W, ns, mode);
 }
 
 // Zero-energy-mode buffers and switches of one class for the next
@@ -944,7 +962,8 @@ int zem_modes(msa_batch *b, size_t c)
     for (int v : cnt) most = std::max(most, std::min(v, zmax));
     const size_t row = (size_t)n * sizeof(double);
     for (int k = 0; k < most; k++) {
-        MSA_HIP(hipMemcpy2DAsync(C.dev.by, row, C.zv + (size_t)k * n, zmax * row, row, ns,
+        double *in = band_one_launch(n, C.dev.bW) ? C.dev.by : C.dev.bx;
+        MSA_HIP(hipMemcpy2DAsync(in, row, C.zv + (size_t)k * n, zmax * row, row, ns,
                                  hipMemcpyDeviceToDevice, s));
         MSA_TRY(band_backward(b, b->d_cls + c, n, C.dev.bW, ns, -1));
         MSA_HIP(hipMemcpy2DAsync(C.zv + (size_t)k * n, zmax * row, C.dev.by, row, row, ns,
@@ -1412,12 +1431,7 @@ int mg_values(msa_batch *b)
         ClassHost &C = tab(b, ci);
         const ClassDev *cp = b->d_cls + ci;
         const int n = C.dev.bn, W = C.dev.bW, ns = C.nsamp;
-        for (int k0 = 0; k0 < n; k0 += kBandNB) {
-            const int nk = std::min(kBandNB, n - k0), r0 = k0 + nk, m = std::min(n - r0, W - kBandNB);
-            MSA_TRY(timed(b, KK_ASSEMBLE, [&] { return launch_chol_diag(s, cp, ns, k0, nk); }));
-            MSA_TRY(timed(b, KK_ASSEMBLE, [&] { return launch_chol_panel(s, cp, ns, k0, nk, r0, m); }));
-            MSA_TRY(timed(b, KK_ASSEMBLE, [&] { return launch_chol_update(s, cp, ns, k0, nk, r0, m); }));
-        }
+        MSA_TRY(band_factor(b, cp, n, W, ns));
     }
     // a coarse operator that is not positive definite leaves the cycle undefined
     for (int ci : b->mg_coarsest) {
@@ -1483,12 +1497,7 @@ int first_values(msa_batch *b)
         ClassHost &C = b->cls[c];
         const ClassDev *cp = b->d_cls + c;
         const int n = C.dev.bn, W = C.dev.bW;
-        for (int k0 = 0; k0 < n; k0 += kBandNB) {
-            const int nk = std::min(kBandNB, n - k0), r0 = k0 + nk, m = std::min(n - r0, W - kBandNB);
-            MSA_TRY(timed(b, KK_ASSEMBLE, [&] { return launch_chol_diag(s, cp, 1, k0, nk); }));
-            MSA_TRY(timed(b, KK_ASSEMBLE, [&] { return launch_chol_panel(s, cp, 1, k0, nk, r0, m); }));
-            MSA_TRY(timed(b, KK_ASSEMBLE, [&] { return launch_chol_update(s, cp, 1, k0, nk, r0, m); }));
-        }
+        MSA_TRY(band_factor(b, cp, n, W, 1));
     }
     for (size_t c = 0; c < b->cls.size(); c++) {
         MSA_HIP(hipMemcpyAsync(b->ctx->h_pinned, b->cls[c].dev.bfail, sizeof(int),
@@ -2655,13 +2664,7 @@ int msa_batch_factorize(msa_batch *b)
         ClassHost &C = b->cls[c];
         const ClassDev *cp = b->d_cls + c;
         const int n = C.dev.bn, W = C.dev.bW, ns = C.nsamp;
-        for (int k0 = 0; k0 < n; k0 += kBandNB) {
-            const int nk = std::min(kBandNB, n - k0), r0 = k0 + nk,
-                      m = std::min(n - r0, W - kBandNB);
-            MSA_TRY(timed(b, KK_ASSEMBLE, [&] { return launch_chol_diag(s, cp, ns, k0, nk); }));
-            MSA_TRY(timed(b, KK_ASSEMBLE, [&] { return launch_chol_panel(s, cp, ns, k0, nk, r0, m); }));
-            MSA_TRY(timed(b, KK_ASSEMBLE, [&] { return launch_chol_update(s, cp, ns, k0, nk, r0, m); }));
-        }
+        MSA_TRY(band_factor(b, cp, n, W, ns));
         if (b->zem_tol > 0.0) MSA_TRY(zem_modes(b, c));
     }
     MSA_HIP(hipStreamSynchronize(s));

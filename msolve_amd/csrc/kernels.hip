@@ -211,18 +211,6 @@ __device__ __forceinline__ double fval(const ClassDev &C, size_t vb, int br, int
     return C.fs ? C.fs[vb + ((size_t)br * 3 + d) * T + s] : C.f[br * 3 + d];
 }
 
-// Samples a multigrid cycle serves: 0 every sample, 1 active, 2 due for a
-// residual replacement, 3 refining.
-__device__ __forceinline__ bool mg_act(const SampleState &S, int mode)
-{
-    switch (mode) {
-    case 0: return true;
-    case 1: return S.active;
-    case 2: return S.ir_active && S.ru_due;
-    default: return S.ir_active;
-    }
-}
-
 __device__ __forceinline__ double fnorm_of(const ClassDev &C, const SampleState &S)
 {
     return C.fs ? S.fnorm : C.fnorm;
@@ -2481,173 +2469,6 @@ __global__ void k_band_rhs(const ClassDev *__restrict__ cp, int from_fs)
     const int tile = smp / T, s = smp % T;
     C.by[(size_t)smp * C.bn + i] =
         from_fs ? C.fs[(size_t)tile * C.tile_vec + (size_t)row * T + s] : C.f[row];
-}
-
-// Forward step of L y = b for block k0: y_blk = L11^-1 y_blk (workgroup 0
-// of the x grid, 64 threads), then rows [r0, r0 + m) minus L21 y_blk.  Two
-// launches per block: `phase` 0 is the diagonal solve, 1 the update.
-__global__ __launch_bounds__(64) void k_band_fwd(const ClassDev *__restrict__ cp, int k0, int nk,
-                                                 int r0, int m, int phase, int mode)
-{
-    __shared__ double yb[kBandNB];
-    const ClassDev &C = *cp;
-    const int smp = blockIdx.y;
-    if (mode >= 0 && !mg_act(C.mg_st[smp], mode)) return;  // coarsest multigrid level
-    const int t = threadIdx.x;
-    const double *AB = C.band + (size_t)smp * C.band_ss;
-    double *y = C.by + (size_t)smp * C.bn;
-    if (phase == 0) {
-        if (t < nk) yb[t] = y[k0 + t];
-        __syncthreads();
-        for (int c = 0; c < nk; c++) {
-            if (t == c) yb[c] /= AB[(size_t)(k0 + c) * C.bW];
-            __syncthreads();
-            if (t > c && t < nk) yb[t] -= AB[(size_t)(k0 + c) * C.bW + (t - c)] * yb[c];
-            __syncthreads();
-        }
-        if (t < nk) y[k0 + t] = yb[t];
-        return;
-    }
-    if (t < nk) yb[t] = y[k0 + t];
-    __syncthreads();
-    const int i = r0 + blockIdx.x * 64 + t;
-    if (i >= r0 + m) return;
-    double acc = 0.0;
-    for (int c = 0; c < nk; c++) acc += AB[(size_t)(k0 + c) * C.bW + (i - k0 - c)] * yb[c];
-    y[i] -= acc;
-}
-
-// Backward step of L^T x = y for block k0: phase 0 writes partial sums
-// bpart[g][c] = sum over rows i of chunk g of L[i][k0+c] x[i]; phase 1
-// (one workgroup) sums them in chunk order and back-substitutes L11^T.
-__global__ __launch_bounds__(64) void k_band_bwd(const ClassDev *__restrict__ cp, int k0, int nk,
-                                                 int r0, int m, int phase, int mode)
-{
-    __shared__ double xb[kBandNB];
-    const ClassDev &C = *cp;
-    const int smp = blockIdx.y;
-    if (mode >= 0 && !mg_act(C.mg_st[smp], mode)) return;  // coarsest multigrid level
-    const int t = threadIdx.x;
-    const double *AB = C.band + (size_t)smp * C.band_ss;
-    double *x = C.by + (size_t)smp * C.bn;
-    const int nchunk = (C.bW + kBandChunkRows - 1) / kBandChunkRows;
-    double *part = C.bpart + (size_t)smp * nchunk * kBandNB;
-    if (phase == 0) {
-        const int g = blockIdx.x;
-        const int i0 = r0 + g * kBandChunkRows, i1 = min(r0 + m, i0 + kBandChunkRows);
-        if (t < nk) {
-            double acc = 0.0;
-            for (int i = i0; i < i1; i++) acc += AB[(size_t)(k0 + t) * C.bW + (i - k0 - t)] * x[i];
-            part[g * kBandNB + t] = acc;
-        }
-        return;
-    }
-    const int ng = m > 0 ? (m + kBandChunkRows - 1) / kBandChunkRows : 0;
-    if (t < nk) {
-        double v = x[k0 + t];
-        for (int g = 0; g < ng; g++) v -= part[g * kBandNB + t];
-        xb[t] = v;
-    }
-    __syncthreads();
-    for (int c = nk - 1; c >= 0; c--) {
-        if (t == c) xb[c] /= AB[(size_t)(k0 + c) * C.bW];
-        __syncthreads();
-        if (t < c) xb[t] -= AB[(size_t)(k0 + t) * C.bW + (c - t)] * xb[c];
-        __syncthreads();
-    }
-    if (t < nk) x[k0 + t] = xb[t];
-}
-
-// Both band sweeps (L y = b, then L^T x = y) of one sample in one
-// workgroup, for bands of at most kBandOneMax rows: the same 64-column
-// blocks and the same order of operations as k_band_fwd / k_band_bwd (so the
-// same results), without a launch per block.  y lives in LDS; each block's
-// diagonal triangle is staged in LDS (rows padded to 65 against bank
-// conflicts) and solved by wave 0 with the right-hand side in registers.
-__device__ __forceinline__ double readlane_f64(double v, int l)
-{
-    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
-    const unsigned lo = __builtin_amdgcn_readlane((unsigned)b, l);
-    const unsigned hi = __builtin_amdgcn_readlane((unsigned)(b >> 32), l);
-    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-}
-
-__global__ __launch_bounds__(256) void k_band_solve_one(const ClassDev *__restrict__ cp, int mode)
-{
-    __shared__ double yl[kBandOneMax];
-    __shared__ double Ld[kBandNB][kBandNB + 1];
-    __shared__ double part[kBandNB];
-    const ClassDev &C = *cp;
-    const int smp = blockIdx.x;
-    if (mode >= 0 && !mg_act(C.mg_st[smp], mode)) return;  // coarsest multigrid level
-    const int n = C.bn, W = C.bW;
-    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const double *AB = C.band + (size_t)smp * C.band_ss;
-    double *y = C.by + (size_t)smp * n;
-    for (int i = t; i < n; i += 256) yl[i] = y[i];
-    // Ld[c][j] = AB[(k0 + c) W + j] = L[k0 + c + j][k0 + c], j < nk - c
-    auto stage = [&](int k0, int nk) {
-        for (int e = t; e < kBandNB * kBandNB; e += 256) {
-            const int c = e >> 6, j = e & 63;
-            Ld[c][j] = (c < nk && j < nk - c) ? AB[(size_t)(k0 + c) * W + j] : 0.0;
-        }
-    };
-    __syncthreads();
-    for (int k0 = 0; k0 < n; k0 += kBandNB) {
-        const int nk = min(kBandNB, n - k0), r0 = k0 + nk, m = min(n - r0, W - kBandNB);
-        stage(k0, nk);
-        __syncthreads();
-        if (wave == 0) {
-            double v = lane < nk ? yl[k0 + lane] : 0.0;
-            for (int c = 0; c < nk; c++) {
-                const double yc = readlane_f64(v, c) / Ld[c][0];
-                if (lane == c) v = yc;
-                if (lane > c && lane < nk) v -= Ld[c][lane - c] * yc;
-            }
-            if (lane < nk) yl[k0 + lane] = v;
-        }
-        __syncthreads();
-        // (unrolled so that the loads of a group issue together; the sum
-        // keeps its order)
-        for (int i = r0 + t; i < r0 + m; i += 256) {
-            double acc = 0.0;
-#pragma unroll 16
-            for (int c = 0; c < nk; c++) acc += AB[(size_t)(k0 + c) * W + (i - k0 - c)] * yl[k0 + c];
-            yl[i] -= acc;
-        }
-        __syncthreads();
-    }
-    const int last = ((n - 1) / kBandNB) * kBandNB;
-    for (int k0 = last; k0 >= 0; k0 -= kBandNB) {
-        const int nk = min(kBandNB, n - k0), r0 = k0 + nk, m = min(n - r0, W - kBandNB);
-        stage(k0, nk);
-        // column partials of L21^T x in chunks of kBandChunkRows rows,
-        // subtracted chunk by chunk (the order of k_band_bwd)
-        if (wave == 1 && lane < nk) {
-            double v = yl[k0 + lane];
-            for (int i0 = r0; i0 < r0 + m; i0 += kBandChunkRows) {
-                const int i1 = min(r0 + m, i0 + kBandChunkRows);
-                double acc = 0.0;
-#pragma unroll 16
-                for (int i = i0; i < i1; i++)
-                    acc += AB[(size_t)(k0 + lane) * W + (i - k0 - lane)] * yl[i];
-                v -= acc;
-            }
-            part[lane] = v;
-        }
-        __syncthreads();
-        if (wave == 0) {
-            double v = lane < nk ? part[lane] : 0.0;
-            for (int c = nk - 1; c >= 0; c--) {
-                const double xc = readlane_f64(v, c) / Ld[c][0];
-                if (lane == c) v = xc;
-                if (lane < c) v -= Ld[lane][c - lane] * xc;
-            }
-            if (lane < nk) yl[k0 + lane] = v;
-        }
-        __syncthreads();
-    }
-    for (int i = t; i < n; i += 256) y[i] = yl[i];
 }
 
 // Solution back to the internal rows: x[row] = by[band(row)], constrained
@@ -5326,38 +5147,6 @@ hipError_t launch_band_rhs(hipStream_t s, int T, const ClassDev *cp, int nsamp, 
     if (bn <= 0) return hipSuccess;
     MSA_DISPATCH_T(T, hipLaunchKernelGGL((k_band_rhs<TT>), dim3((bn + 255) / 256, nsamp), dim3(256),
                                          0, s, cp, from_fs));
-    return hipGetLastError();
-}
-
-hipError_t launch_band_fwd(hipStream_t s, const ClassDev *cp, int nsamp, int k0, int nk, int r0,
-                           int m, int mode)
-{
-    hipLaunchKernelGGL(k_band_fwd, dim3(1, nsamp), dim3(64), 0, s, cp, k0, nk, r0, m, 0, mode);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess || m <= 0) return e;
-    hipLaunchKernelGGL(k_band_fwd, dim3((m + 63) / 64, nsamp), dim3(64), 0, s, cp, k0, nk, r0, m, 1,
-                       mode);
-    return hipGetLastError();
-}
-
-hipError_t launch_band_bwd(hipStream_t s, const ClassDev *cp, int nsamp, int k0, int nk, int r0,
-                           int m, int mode)
-{
-    if (m > 0) {
-        hipLaunchKernelGGL(k_band_bwd, dim3((m + kBandChunkRows - 1) / kBandChunkRows, nsamp),
-                           dim3(64), 0, s, cp, k0, nk, r0, m, 0, mode);
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-    }
-    hipLaunchKernelGGL(k_band_bwd, dim3(1, nsamp), dim3(64), 0, s, cp, k0, nk, r0, m, 1, mode);
-    return hipGetLastError();
-}
-
-hipError_t launch_band_solve_one(hipStream_t s, const ClassDev *cp, int nsamp, int bn, int mode)
-{
-    if (bn <= 0) return hipSuccess;
-    if (bn > kBandOneMax) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_band_solve_one, dim3(nsamp), dim3(256), 0, s, cp, mode);
     return hipGetLastError();
 }
 

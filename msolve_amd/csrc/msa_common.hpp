@@ -196,7 +196,9 @@ struct ClassDev {
     long long band_ss;    // doubles between two samples' factors: bn*bW, or 0 when every
                           // sample uses the one factor at band (first-sample preconditioner)
     double *by;           // [nsamp][bn] right-hand side / solution in band order
-    double *bpart;        // [nsamp][kBandChunks][64] partial sums of the backward solve
+    double *bx;           // [nsamp][bn] second buffer of the sweeps of wide bands (null: narrow)
+    double *linv;         // [nsamp][blocks][2][64*64] inverted diagonal blocks, by row and by column
+    long long linv_ss;    // doubles between two samples' (0: one shared factor)
     int *bfail;           // [nsamp] non-positive pivot met
     // zero-energy modes of the direct solver's factorization (zv null: off):
     // a pivot of magnitude under zem_tol is set to 1 and its row and column
@@ -257,11 +259,30 @@ struct ClassDev {
     double *mf_k64;       // [640] the same in FP64 (replacement residuals)
 };
 
+// Samples a multigrid cycle serves: 0 every sample, 1 active, 2 due for a
+// residual replacement, 3 refining.
+__device__ __forceinline__ bool mg_act(const SampleState &S, int mode)
+{
+    switch (mode) {
+    case 0: return true;
+    case 1: return S.active;
+    case 2: return S.ir_active && S.ru_due;
+    default: return S.ir_active;
+    }
+}
+
 constexpr int kLzMax = 16;         // Lanczos steps of the smoothing-interval estimate, at most
 constexpr int kBandNB = 64;        // block size of the band Cholesky
-constexpr int kBandChunkRows = 512;  // rows per partial of the backward solve
 constexpr int kDenseMax = 256;       // coarsest multigrid levels up to this size use a dense inverse
-constexpr int kBandOneMax = 2048;    // bands up to this many rows: both sweeps in one launch
+// Bands whose sweeps run in one launch, a workgroup of 8 waves per sample: a
+// panel of at most 7 x 64 rows (one wave each), a factor within 32-bit byte
+// offsets.  Wider ones take a launch per 64-column block, which spreads the
+// panel over workgroups.
+constexpr int kBandOneMax = 512;
+inline bool band_one_launch(long long n, long long W)
+{
+    return W <= kBandOneMax && (n + 128) * W * 8 < (1ll << 32);
+}
 constexpr int kKlTiles = 8;          // tiles per thread of the KL field evaluation
 constexpr int kNoallocMaxElem = 4096; // elements per call of msa_ke_packed_noalloc
 
@@ -384,12 +405,12 @@ hipError_t launch_chol_update(hipStream_t s, const ClassDev *cp, int nsamp, int 
                               int m);
 hipError_t launch_band_rhs(hipStream_t s, int T, const ClassDev *cp, int nsamp, int bn,
                            int from_fs);
-// mode >= 0: coarsest multigrid level, only the samples mg_act serves
-hipError_t launch_band_fwd(hipStream_t s, const ClassDev *cp, int nsamp, int k0, int nk, int r0,
-                           int m, int mode = -1);
-hipError_t launch_band_solve_one(hipStream_t s, const ClassDev *cp, int nsamp, int bn, int mode);
-hipError_t launch_band_bwd(hipStream_t s, const ClassDev *cp, int nsamp, int k0, int nk, int r0,
-                           int m, int mode = -1);
+// band.hip.  mode >= 0: only the samples mg_act serves
+hipError_t launch_band_linv(hipStream_t s, const ClassDev *cp, int nsamp, int bn);
+hipError_t launch_band_sweep_one(hipStream_t s, const ClassDev *cp, int nsamp, int bn, int bW,
+                                 int mode, int sweeps);
+hipError_t launch_band_sweep_step(hipStream_t s, const ClassDev *cp, int nsamp, int bn, int bW,
+                                  int k, bool forward, int mode);
 hipError_t launch_band_out(hipStream_t s, int T, const ClassDev *cp, int nsamp, int nrows);
 // multigrid preconditioner: items of one level of every hierarchy
 enum MgStep { MG_PRE = 0, MG_RESID = 1, MG_POST1 = 2, MG_POST2 = 3 };
