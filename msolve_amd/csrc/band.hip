@@ -1,6 +1,13 @@
-// Triangular sweeps with the band Cholesky factors (direct solver, first-
-// sample preconditioner, coarsest multigrid levels): the solve half of
-// SkylineMatrix2D.Factorize / Solve (SkylineMatrix2D.cs:160-212).
+// Band Cholesky factorization and triangular sweeps (direct solver, first-
+// sample preconditioner, coarsest multigrid levels): SkylineMatrix2D.
+// Factorize / Solve (SkylineMatrix2D.cs:63-212) in blocks of kBandNB = 64
+// columns.  Lower band storage band[j*bW + (i - j)], bW >= bandwidth + 64,
+// so every panel is a full rectangle (entries outside the true band stay
+// zero).  grid.y = sample of the class.
+//
+// A factorization runs k_chol_block, k_chol_panel_inv and k_chol_update_mfma
+// per block (zero-energy modes: k_chol_diag and k_chol_panel in their place,
+// and k_band_linv at the end).
 //
 // A sweep walks the factor in blocks of kBandNB = 64 columns, and a block
 // depends on the one before: the time is the number of blocks times the
@@ -11,7 +18,14 @@
 // below; backward: the rows above), so no block waits on a reduction over
 // rows that another workgroup holds.
 //
-// Measured (MI355X, factor and all): the first-sample preconditioner on 8
+// Measured, factorization (MI355X, one 16^3 sample, 217 blocks of width 960):
+// 218 -> 43 us per block, 47 -> 9.3 ms: the diagonal block 137 -> 27 us (the
+// chain of 64 pivots; it was a 64-step loop with two barriers a step), the
+// panel 58 -> 5 us (a product with the inverse instead of a column sweep),
+// the update 23 -> 10.6 us (matrix cores instead of 4 x 4 register tiles
+// through LDS).
+//
+// Measured, sweeps (with the factorization before that change): the first-sample preconditioner on 8
 // samples of 12^3 (6084 rows, width 576, 22 applications) 525 -> 37.5 ms,
 // the sweeps of a 16^3 direct solve (13872 rows) 48 -> 1.6 ms, against a
 // launch pair per block and sweep with 64-step substitutions.  Both sweeps
@@ -66,14 +80,18 @@ __device__ __forceinline__ double sum8(double v)
 
 // ---------------------------------------------------- diagonal block inverse
 
-// X = L^-1 of a 64 x 64 lower triangle in LDS by 256 threads: the four
-// 16 x 16 diagonal blocks by substitution (wave w, lane = column), then the
-// blocks below by distance d from the diagonal, X_ij = -X_ii sum_k L_ik X_kj,
-// one block per wave on the matrix cores.  v_mfma_f64_16x16x4: lane l holds
-// A[l % 16][l / 16], B[l / 16][l % 16] and, in register v, D[l / 16 + 4 v]
-// [l % 16], so a product's registers are the next one's B operands.
-__device__ __forceinline__ void invert_lower(double (*L)[kBandNB + 1], double (*X)[kBandNB + 1],
-                                             int t)
+// Register v of lane l in v_mfma_f64_16x16x4: the operands are A[l % 16][l / 16]
+// and B[l / 16][l % 16], the result D[l / 16 + 4 v][l % 16].  So a product's
+// registers v = 0..3 are the B operands of the next one's four steps.
+#define MFMA64(a, b, c) __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0)
+
+typedef double Tile64[kBandNB][kBandNB + 1];  // in LDS, a column apart per row
+
+// X = L^-1 of a 64 x 64 lower triangle in LDS by 256 threads, rd = 1 / diag:
+// the four 16 x 16 diagonal blocks by substitution (wave w, lane = column),
+// then the blocks below by distance d from the diagonal,
+// X_ij = -X_ii sum_k L_ik X_kj, one block per wave on the matrix cores.
+__device__ __forceinline__ void invert_lower(const Tile64 &L, Tile64 &X, const double *rd, int t)
 {
     const int lane = t & 63, w = t >> 6, o = 16 * w;
     for (int e = t; e < kBandNB * kBandNB; e += 256) X[e >> 6][e & 63] = 0.0;
@@ -81,11 +99,12 @@ __device__ __forceinline__ void invert_lower(double (*L)[kBandNB + 1], double (*
     if (lane < 16) {
         double x[16];
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
-            double s = i == lane ? 1.0 : 0.0;
+        for (int i = 0; i < 16; i++) x[i] = i == lane ? 1.0 : 0.0;
 #pragma unroll
-            for (int k = 0; k < i; k++) s -= L[o + i][o + k] * x[k];
-            x[i] = s / L[o + i][o + i];
+        for (int k = 0; k < 16; k++) {
+            x[k] *= rd[o + k];
+#pragma unroll
+            for (int i = k + 1; i < 16; i++) x[i] -= L[o + i][o + k] * x[k];
         }
 #pragma unroll
         for (int i = 0; i < 16; i++) X[o + i][o + lane] = x[i];
@@ -99,14 +118,10 @@ __device__ __forceinline__ void invert_lower(double (*L)[kBandNB + 1], double (*
             for (int k = j; k < i; k++)
 #pragma unroll
                 for (int q = 0; q < 4; q++)
-                    s = __builtin_amdgcn_mfma_f64_16x16x4f64(L[16 * i + r][16 * k + 4 * q + g],
-                                                             X[16 * k + 4 * q + g][16 * j + r], s,
-                                                             0, 0, 0);
+                    s = MFMA64(L[16 * i + r][16 * k + 4 * q + g], X[16 * k + 4 * q + g][16 * j + r], s);
             f64x4 p = {0, 0, 0, 0};
 #pragma unroll
-            for (int q = 0; q < 4; q++)
-                p = __builtin_amdgcn_mfma_f64_16x16x4f64(X[16 * i + r][16 * i + 4 * q + g], s[q], p,
-                                                         0, 0, 0);
+            for (int q = 0; q < 4; q++) p = MFMA64(X[16 * i + r][16 * i + 4 * q + g], s[q], p);
 #pragma unroll
             for (int v = 0; v < 4; v++) X[16 * i + g + 4 * v][16 * j + r] = -p[v];
         }
@@ -114,26 +129,200 @@ __device__ __forceinline__ void invert_lower(double (*L)[kBandNB + 1], double (*
     __syncthreads();
 }
 
-// Inverse of every diagonal block of every factor: grid (block, sample).
-// Columns past the band's end (a last, partial block) invert as identity.
-__global__ __launch_bounds__(256) void k_band_linv(const ClassDev *__restrict__ cp)
+__device__ __forceinline__ void store_inverse(const Tile64 &X, GLOB double *out, int t)
 {
-    __shared__ double L[kBandNB][kBandNB + 1], X[kBandNB][kBandNB + 1];
-    const ClassDev &C = *cp;
-    const int t = threadIdx.x, k0 = blockIdx.x * kBandNB, smp = blockIdx.y;
-    const int nk = min(kBandNB, C.bn - k0);
-    const GLOB double *AB = glob(C.band + (size_t)smp * C.band_ss);
-    for (int e = t; e < kBandNB * kBandNB; e += 256) {
-        const int c = e >> 6, r = e & 63;
-        L[r][c] = r >= c && r < nk ? AB[(size_t)(k0 + c) * C.bW + (r - c)] : (r == c ? 1.0 : 0.0);
-    }
-    __syncthreads();
-    invert_lower(L, X, t);
-    GLOB double *out = glob(C.linv + (size_t)smp * C.linv_ss + (size_t)blockIdx.x * kLinvBlock);
     for (int e = t; e < kBandNB * kBandNB; e += 256) {
         out[e] = X[e >> 6][e & 63];                      // by row
         out[kBandNB * kBandNB + e] = X[e & 63][e >> 6];  // by column
     }
+}
+
+// Lower triangle of the diagonal block at column k0 into LDS, zeros above;
+// rows past the band's end (a last, partial block) become identity rows.
+__device__ __forceinline__ void load_diag(const ClassDev &C, const GLOB double *AB, int k0, Tile64 &L,
+                                          int t)
+{
+    const int nk = min(kBandNB, C.bn - k0);
+    for (int e = t; e < kBandNB * kBandNB; e += 256) {
+        const int c = e >> 6, r = e & 63;
+        L[r][c] = r >= c && r < nk ? AB[(size_t)(k0 + c) * C.bW + (r - c)] : (r == c ? 1.0 : 0.0);
+    }
+}
+
+// Inverse of every diagonal block of every factor: grid (block, sample).
+__global__ __launch_bounds__(256) void k_band_linv(const ClassDev *__restrict__ cp)
+{
+    __shared__ Tile64 L, X;
+    __shared__ double rd[kBandNB];
+    const ClassDev &C = *cp;
+    const int t = threadIdx.x, smp = blockIdx.y;
+    load_diag(C, glob((const double *)C.band + (size_t)smp * C.band_ss), blockIdx.x * kBandNB, L, t);
+    __syncthreads();
+    if (t < kBandNB) rd[t] = 1.0 / L[t][t];
+    __syncthreads();
+    invert_lower(L, X, rd, t);
+    store_inverse(X, glob(C.linv + (size_t)smp * C.linv_ss + (size_t)blockIdx.x * kLinvBlock), t);
+}
+
+// ------------------------------------------------------------ factorization
+
+__device__ __forceinline__ double lane_f64(double v, int l)
+{
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = __builtin_amdgcn_readlane((unsigned)b, l);
+    const unsigned hi = __builtin_amdgcn_readlane((unsigned)(b >> 32), l);
+    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+
+// Cholesky of the diagonal block at column k0 and its inverse, one workgroup
+// per sample: columns in four groups of 16, each factored by wave 0 with
+// lane = row and the group in registers (a pivot's reciprocal root from
+// v_rsq_f64 and one cubic Newton step), then applied to the columns right of
+// it on the matrix cores.  The chain of 64 pivots is what takes the time.
+__global__ __launch_bounds__(256) void k_chol_block(const ClassDev *__restrict__ cp, int k0)
+{
+    __shared__ Tile64 L, X;
+    __shared__ double rd[kBandNB];
+    const ClassDev &C = *cp;
+    const int smp = blockIdx.y, t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int nk = min(kBandNB, C.bn - k0);
+    GLOB double *AB = glob(C.band + (size_t)smp * C.band_ss);
+    load_diag(C, AB, k0, L, t);
+    __syncthreads();
+    bool fail = false;
+    const int r = lane & 15, g = lane >> 4;
+    for (int b = 0; b < 4; b++) {
+        const int o = 16 * b;
+        if (wave == 0) {
+            double a[16];
+#pragma unroll
+            for (int c = 0; c < 16; c++) a[c] = L[lane][o + c];
+#pragma unroll
+            for (int c = 0; c < 16; c++) {
+                double d = lane_f64(a[c], o + c);
+                if (!(d > 0.0) || !isfinite(d)) {
+                    fail = true;
+                    d = 1.0;
+                }
+                double y = __builtin_amdgcn_rsq(d);
+                const double e = __builtin_fma(-(d * y), y, 1.0);
+                y = __builtin_fma(y * e, __builtin_fma(0.375, e, 0.5), y);
+                const double l = lane > o + c ? a[c] * y : 0.0;
+#pragma unroll
+                for (int c2 = c + 1; c2 < 16; c2++) a[c2] -= l * lane_f64(l, o + c2);
+                double s = d * y;
+                s = __builtin_fma(0.5 * y, __builtin_fma(-s, s, d), s);
+                a[c] = lane == o + c ? s : l;
+                if (lane == 0) rd[o + c] = y;
+            }
+#pragma unroll
+            for (int c = 0; c < 16; c++) L[lane][o + c] = a[c];
+        }
+        __syncthreads();
+        // columns right of the group: tiles (I, J), b < J <= I
+        for (int T = wave, I = b + 1, J = b + 1; I < 4; ) {
+            if (T == 0) {
+                f64x4 s = {0, 0, 0, 0};
+#pragma unroll
+                for (int q = 0; q < 4; q++)
+                    s = MFMA64(L[16 * I + r][o + 4 * q + g], L[16 * J + r][o + 4 * q + g], s);
+#pragma unroll
+                for (int v = 0; v < 4; v++) L[16 * I + g + 4 * v][16 * J + r] -= s[v];
+                T = 4;
+            }
+            T--;
+            if (++J > I) {
+                I++;
+                J = b + 1;
+            }
+        }
+        __syncthreads();
+    }
+    if (t == 0 && fail) C.bfail[smp] = 1;
+    for (int e = t; e < kBandNB * kBandNB; e += 256) {
+        const int c = e >> 6, rr = e & 63;
+        if (rr >= c && rr < nk) AB[(size_t)(k0 + c) * C.bW + (rr - c)] = L[rr][c];
+    }
+    invert_lower(L, X, rd, t);
+    store_inverse(X, glob(C.linv + (size_t)smp * C.linv_ss + (size_t)(k0 / kBandNB) * kLinvBlock), t);
+}
+
+// Panel rows [r0, r0 + m), r0 = k0 + 64: L21 = A21 L11^-T as a product with
+// the inverted block, 16 rows per wave, straight from and to global memory:
+// D[c][row] = sum_k Linv[c][k] A21[row][k], so that loads and stores run
+// along rows.  (Rows past the band's end hold zeros.)
+__global__ __launch_bounds__(256) void k_chol_panel_inv(const ClassDev *__restrict__ cp, int k0, int m)
+{
+    const ClassDev &C = *cp;
+    const int smp = blockIdx.y, lane = threadIdx.x & 63;
+    const int r = lane & 15, g = lane >> 4, W = C.bW;
+    const int i0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 16;  // row - r0
+    if (i0 >= m) return;
+    GLOB double *P = glob(C.band + (size_t)smp * C.band_ss) + (size_t)k0 * W + kBandNB + i0 + r;
+    const GLOB double *LI = glob((const double *)C.linv + (size_t)smp * C.linv_ss +
+                                 (size_t)(k0 / kBandNB) * kLinvBlock + kBandNB * kBandNB);
+    double a[16];  // A21[row][4 q + g]
+#pragma unroll
+    for (int q = 0; q < 16; q++) a[q] = P[(size_t)(4 * q + g) * (W - 1)];
+    f64x4 s[4];
+#pragma unroll
+    for (int ct = 0; ct < 4; ct++) {
+        s[ct] = f64x4{0, 0, 0, 0};
+#pragma unroll
+        for (int q = 0; q < 4 * (ct + 1); q++)
+            s[ct] = MFMA64(LI[(4 * q + g) * kBandNB + 16 * ct + r], a[q], s[ct]);
+    }
+    if (i0 + r >= m) return;
+#pragma unroll
+    for (int ct = 0; ct < 4; ct++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) P[(size_t)(16 * ct + g + 4 * v) * (W - 1)] = s[ct][v];
+}
+
+// Trailing update of the band window: A[i][j] -= sum_c L[i][k0+c] L[j][k0+c]
+// for r0 <= j <= i < r0 + m; one workgroup per 64 x 64 tile (I, J), J <= I,
+// a 32 x 32 part per wave: D[j][i], operands straight from the panel (each
+// load four 128-byte row pieces).
+__global__ __launch_bounds__(256) void k_chol_update_mfma(const ClassDev *__restrict__ cp, int k0, int m)
+{
+    const ClassDev &C = *cp;
+    const int smp = blockIdx.y, W = C.bW;
+    // tile index -> (I, J) with J <= I
+    const int tix = blockIdx.x;
+    int I = (int)((sqrt(8.0 * tix + 1.0) - 1.0) * 0.5);
+    while ((I + 1) * (I + 2) / 2 <= tix) I++;
+    while (I * (I + 1) / 2 > tix) I--;
+    const int J = tix - I * (I + 1) / 2;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int r = lane & 15, g = lane >> 4;
+    const int i0 = I * kBandNB + 32 * (wave & 1), j0 = J * kBandNB + 32 * (wave >> 1);
+    if (i0 + 31 < j0 || i0 >= m || j0 >= m) return;
+    GLOB double *AB = glob(C.band + (size_t)smp * C.band_ss);
+    const GLOB double *P = AB + (size_t)k0 * W + kBandNB + (size_t)g * (W - 1) + r;
+    f64x4 s[2][2];
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+        for (int v = 0; v < 2; v++) s[u][v] = f64x4{0, 0, 0, 0};
+#pragma unroll
+    for (int q = 0; q < 16; q++) {
+        const GLOB double *Pq = P + (size_t)(4 * q) * (W - 1);
+        const double a0 = Pq[j0], a1 = Pq[j0 + 16], b0 = Pq[i0], b1 = Pq[i0 + 16];
+        s[0][0] = MFMA64(a0, b0, s[0][0]);
+        s[0][1] = MFMA64(a0, b1, s[0][1]);
+        s[1][0] = MFMA64(a1, b0, s[1][0]);
+        s[1][1] = MFMA64(a1, b1, s[1][1]);
+    }
+    const int r0 = k0 + kBandNB;
+#pragma unroll
+    for (int u = 0; u < 2; u++)
+#pragma unroll
+        for (int w = 0; w < 2; w++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int j = j0 + 16 * u + g + 4 * v, i = i0 + 16 * w + r;
+                if (i >= j && i < m) AB[(size_t)(r0 + j) * W + (i - j)] -= s[u][w][v];
+            }
 }
 
 // ------------------------------------------------------------------- sweeps
@@ -251,8 +440,6 @@ __device__ __forceinline__ bool served(const ClassDev &C, int smp, int mode)
 {
     return mode < 0 || mg_act(C.mg_st[smp], mode);
 }
-
-}  // namespace
 
 // The sweeps of one sample in one workgroup of 8 waves (narrow bands and
 // batches of samples), in place on by.  The band window of the right-hand
@@ -401,6 +588,29 @@ __global__ __launch_bounds__(64 * kSweepWaves) void k_band_sweep_step(
         s = sum8(s);
         if ((lane & 7) == 0) src[i] -= s;
     }
+}
+
+}  // namespace
+
+hipError_t launch_chol_block(hipStream_t s, const ClassDev *cp, int nsamp, int k0)
+{
+    hipLaunchKernelGGL(k_chol_block, dim3(1, nsamp), dim3(256), 0, s, cp, k0);
+    return hipGetLastError();
+}
+
+hipError_t launch_chol_panel_inv(hipStream_t s, const ClassDev *cp, int nsamp, int k0, int m)
+{
+    if (m <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_chol_panel_inv, dim3((m + 63) / 64, nsamp), dim3(256), 0, s, cp, k0, m);
+    return hipGetLastError();
+}
+
+hipError_t launch_chol_update(hipStream_t s, const ClassDev *cp, int nsamp, int k0, int m)
+{
+    if (m <= 0) return hipSuccess;
+    const int T = (m + kBandNB - 1) / kBandNB;
+    hipLaunchKernelGGL(k_chol_update_mfma, dim3(T * (T + 1) / 2, nsamp), dim3(256), 0, s, cp, k0, m);
+    return hipGetLastError();
 }
 
 hipError_t launch_band_linv(hipStream_t s, const ClassDev *cp, int nsamp, int bn)

@@ -861,16 +861,22 @@ int prepare_band(msa_batch *b)
 }
 
 // Band Cholesky factors of ns samples and the inverses of their diagonal
-// blocks, which the sweeps read.
-int band_factor(msa_batch *b, const ClassDev *cp, int n, int W, int ns)
+// blocks, which the sweeps read.  zem: with zero-energy modes.
+int band_factor(msa_batch *b, const ClassDev *cp, int n, int W, int ns, bool zem = false)
 {
     hipStream_t s = b->ctx->stream;
     for (int k0 = 0; k0 < n; k0 += kBandNB) {
         const int nk = std::min(kBandNB, n - k0), r0 = k0 + nk, m = std::min(n - r0, W - kBandNB);
-        MSA_TRY(timed(b, KK_ASSEMBLE, [&] { return launch_chol_diag(s, cp, ns, k0, nk); }));
-        MSA_TRY(timed(b, KK_ASSEMBLE, [&] { return launch_chol_panel(s, cp, ns, k0, nk, r0, m); }));
-        MSA_TRY(timed(b, KK_ASSEMBLE, [&] { return launch_chol_update(s, cp, ns, k0, nk, r0, m); }));
+        MSA_TRY(timed(b, KK_ASSEMBLE, [&] {
+            return zem ? launch_chol_diag(s, cp, ns, k0, nk) : launch_chol_block(s, cp, ns, k0);
+        }));
+        MSA_TRY(timed(b, KK_ASSEMBLE, [&] {
+            return zem ? launch_chol_panel(s, cp, ns, k0, nk, r0, m)
+                       : launch_chol_panel_inv(s, cp, ns, k0, m);
+        }));
+        MSA_TRY(timed(b, KK_ASSEMBLE, [&] { return launch_chol_update(s, cp, ns, k0, m); }));
     }
+    if (!zem) return MSA_OK;
     return timed(b, KK_ASSEMBLE, [&] { return launch_band_linv(s, cp, ns, n); });
 }
 
@@ -2664,7 +2670,7 @@ int msa_batch_factorize(msa_batch *b)
         ClassHost &C = b->cls[c];
         const ClassDev *cp = b->d_cls + c;
         const int n = C.dev.bn, W = C.dev.bW, ns = C.nsamp;
-        MSA_TRY(band_factor(b, cp, n, W, ns));
+        MSA_TRY(band_factor(b, cp, n, W, ns, b->zem_tol > 0.0));
         if (b->zem_tol > 0.0) MSA_TRY(zem_modes(b, c));
     }
     MSA_HIP(hipStreamSynchronize(s));

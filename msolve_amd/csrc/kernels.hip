@@ -2227,14 +2227,8 @@ __global__ __launch_bounds__(256) void k_dyn_update(const ClassDev *__restrict__
 }
 
 // ------------------------------------------------------------ direct solver
-// Banded Cholesky K = L L^T of each sample's FP64 stiffness (the GPU
-// counterpart of SkylineMatrix2D.Factorize / Solve, SkylineMatrix2D.cs:
-// 63-212, used by SolverSkyline.cs:90-205), blocked by kBandNB = 64 columns:
-// per block the diagonal factor (k_chol_diag), the panel solve below it
-// within the band (k_chol_panel) and the trailing update of the band window
-// (k_chol_update).  Lower band storage band[j*bW + (i - j)], bW >= bandwidth
-// + 64, so every panel is a full rectangle (entries outside the true band
-// stay zero).  grid.y = sample of the class.
+// Band storage of the factorization (band.hip), and its block steps with
+// zero-energy modes.  grid.y = sample of the class.
 
 // Lower band entries of every sample's assembled K (FP64 batch values).
 template <typename real, int T>
@@ -2279,10 +2273,11 @@ __global__ __launch_bounds__(256) void k_band_scatter(const ClassDev *__restrict
     }
 }
 
-// In-place Cholesky of the nk x nk diagonal block at column k0; one
-// workgroup of 64 threads (thread = block row) per sample.
+// In-place Cholesky of the nk x nk diagonal block at column k0 with
+// zero-energy modes; one workgroup of 64 threads (thread = block row) per
+// sample.
 //
-// Zero-energy modes (C.zv set; SkylineMatrix2D.Factorize's kFix branch,
+// Zero-energy modes ( SkylineMatrix2D.Factorize's kFix branch,
 // SkylineMatrix2D.cs:110-130): a pivot d = K_nn - sum_k L_nk^2 with |d| <
 // zem_tol is the LDL^T pivot of a singular direction.  The factor then takes
 // L_nn = 1 and clears row n (saved first: w_n = 1, w_k = -L_nk; in LDL^T terms
@@ -2403,57 +2398,6 @@ __global__ __launch_bounds__(256) void k_chol_panel(const ClassDev *__restrict__
         const int i = row0 + r;
         if (c < nk && i < r0 + m) AB[(size_t)(k0 + c) * C.bW + (i - k0 - c)] = P[r][c];
     }
-}
-
-// Trailing update of the band window: A[i][j] -= sum_c L[i][k0+c] L[j][k0+c]
-// for r0 <= j <= i < r0 + m; one 256-thread workgroup per 64 x 64 tile (I, J),
-// J <= I, each thread a 4 x 4 sub-block; the panel columns are staged in LDS
-// in two halves of 32.
-__global__ __launch_bounds__(256) void k_chol_update(const ClassDev *__restrict__ cp, int k0, int nk,
-                                                     int r0, int m)
-{
-    __shared__ double Li[kBandNB][33], Lj[kBandNB][33];
-    const ClassDev &C = *cp;
-    const int smp = blockIdx.y;
-    double *AB = C.band + (size_t)smp * C.band_ss;
-    // tile index -> (I, J) with J <= I
-    const int tix = blockIdx.x;
-    int I = (int)((sqrt(8.0 * tix + 1.0) - 1.0) * 0.5);
-    while ((I + 1) * (I + 2) / 2 <= tix) I++;
-    while (I * (I + 1) / 2 > tix) I--;
-    const int J = tix - I * (I + 1) / 2;
-    const int ti = threadIdx.x >> 4, tj = threadIdx.x & 15;
-    double acc[4][4] = {};
-    for (int h = 0; h < 2; h++) {
-        for (int e = threadIdx.x; e < kBandNB * 32; e += 256) {
-            const int r = e >> 5, c = (e & 31) + 32 * h;
-            const int ir = r0 + I * kBandNB + r, jr = r0 + J * kBandNB + r;
-            Li[r][c & 31] = (c < nk && ir < r0 + m) ? AB[(size_t)(k0 + c) * C.bW + (ir - k0 - c)] : 0.0;
-            Lj[r][c & 31] = (c < nk && jr < r0 + m) ? AB[(size_t)(k0 + c) * C.bW + (jr - k0 - c)] : 0.0;
-        }
-        __syncthreads();
-#pragma unroll 4
-        for (int c = 0; c < 32; c++) {
-            double a[4], b[4];
-#pragma unroll
-            for (int u = 0; u < 4; u++) {
-                a[u] = Li[ti * 4 + u][c];
-                b[u] = Lj[tj * 4 + u][c];
-            }
-#pragma unroll
-            for (int u = 0; u < 4; u++)
-#pragma unroll
-                for (int v = 0; v < 4; v++) acc[u][v] += a[u] * b[v];
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int u = 0; u < 4; u++)
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-            const int i = r0 + I * kBandNB + ti * 4 + u, j = r0 + J * kBandNB + tj * 4 + v;
-            if (i < r0 + m && j < r0 + m && i >= j) AB[(size_t)j * C.bW + (i - j)] -= acc[u][v];
-        }
 }
 
 // by[s][i] = right-hand side of band row i (class load vector, or the
@@ -5128,16 +5072,6 @@ hipError_t launch_chol_panel(hipStream_t s, const ClassDev *cp, int nsamp, int k
     if (m <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_chol_panel, dim3((m + kBandNB - 1) / kBandNB, nsamp), dim3(256), 0, s, cp,
                        k0, nk, r0, m);
-    return hipGetLastError();
-}
-
-hipError_t launch_chol_update(hipStream_t s, const ClassDev *cp, int nsamp, int k0, int nk, int r0,
-                              int m)
-{
-    if (m <= 0) return hipSuccess;
-    const int T = (m + kBandNB - 1) / kBandNB;
-    hipLaunchKernelGGL(k_chol_update, dim3(T * (T + 1) / 2, nsamp), dim3(256), 0, s, cp, k0, nk,
-                       r0, m);
     return hipGetLastError();
 }
 

@@ -401,11 +401,12 @@ hipError_t launch_band_scatter(hipStream_t s, int T, const ClassDev *d_cls, cons
 hipError_t launch_chol_diag(hipStream_t s, const ClassDev *cp, int nsamp, int k0, int nk);
 hipError_t launch_chol_panel(hipStream_t s, const ClassDev *cp, int nsamp, int k0, int nk, int r0,
                              int m);
-hipError_t launch_chol_update(hipStream_t s, const ClassDev *cp, int nsamp, int k0, int nk, int r0,
-                              int m);
 hipError_t launch_band_rhs(hipStream_t s, int T, const ClassDev *cp, int nsamp, int bn,
                            int from_fs);
 // band.hip.  mode >= 0: only the samples mg_act serves
+hipError_t launch_chol_block(hipStream_t s, const ClassDev *cp, int nsamp, int k0);
+hipError_t launch_chol_panel_inv(hipStream_t s, const ClassDev *cp, int nsamp, int k0, int m);
+hipError_t launch_chol_update(hipStream_t s, const ClassDev *cp, int nsamp, int k0, int m);
 hipError_t launch_band_linv(hipStream_t s, const ClassDev *cp, int nsamp, int bn);
 hipError_t launch_band_sweep_one(hipStream_t s, const ClassDev *cp, int nsamp, int bn, int bW,
                                  int mode, int sweeps);
