@@ -46,6 +46,7 @@ METRIC = "MC solves/sec at 1e-8 rel. err, batched mixed vs plain FP64, 1 MI355X"
 HBM_PEAK_GBS = 8000.0
 FP32_PEAK_TFLOPS = 157.3      # MI355X published FP32 rate (packed / MFMA)
 FP32_VALU_NOPACK_TFLOPS = 78.65  # the same without packed FP32 (disabled in this build)
+FP64_PEAK_TFLOPS = 78.6  # FP64 VALU
 HOST_CORE_SHARE = 16          # host cores one GPU gets on the benchmark box
 
 
@@ -263,13 +264,13 @@ def kernel_a_bytes(b, rs, full=False):
     return total
 
 
-def mf_pcg_work(b, models):
-    """FP32 operations and algorithmic HBM bytes of all matrix-free PCG
-    product launches (k_pcg_p + k_pcg_a_mf) of one solve, None unless
+def mf_pcg_work(b, models, rs=4):
+    """Operations and algorithmic HBM bytes of all matrix-free PCG product
+    launches (k_pcg_p + k_pcg_a_mf / k_pcg_a_mf64) of one solve, None unless
     every class takes that product.  Per iteration and active sample: the
     same 150 flop per (free node, incident cell) pair as the matrix-free
     smoothing products; bytes: z and p_old read and p written by the p
-    pass, p gathered and q written by the product (5 vectors of 4*3*nb),
+    pass, p gathered and q written by the product (5 vectors of rs*3*nb),
     and the moduli (8 per element)."""
     flops = byts = 0.0
     for c, m in enumerate(models):
@@ -281,7 +282,7 @@ def mf_pcg_work(b, models):
         inc = float(free_node[conn].sum())
         nb = float(free_node.sum())
         flops += its * inc * 150.0
-        byts += its * (5 * 4 * 3 * nb + 8.0 * conn.shape[0])
+        byts += its * (5 * rs * 3 * nb + 8.0 * conn.shape[0])
     return flops, byts
 
 
@@ -296,18 +297,26 @@ def counters(name):
                                                      cj["algorithmic_write"])
 
 
-def back_to_back(roof, b, reps=20, rs=8):
+def back_to_back(roof, b, reps=20, rs=8, models=None):
     """Adds the SpMV+dot kernel timed over `reps` back-to-back launches with
     every sample active (no per-launch event overhead) to a roofline entry
     and makes it the entry's achieved figure; the per-launch HIP-event
     figure of the solve stays beside it.  Overwrites the batch's PCG
     iterates."""
+    work = mf_pcg_work(b, models, rs) if roof["bound"] == "valu" else None
+    its = sum(float(b.stats(c)["iters"].sum()) for c in range(len(b.meshes)))
     ms = b.time_spmv(reps)
     byts = b.spmv_bytes()["kernel"]
     roof["per_launch_events"] = dict(achieved=roof["achieved"], avg_launch_ms=roof["avg_launch_ms"],
                                      avg_bytes_per_launch=roof["avg_bytes_per_launch"])
-    roof["achieved"] = byts / (ms / 1e3) / 1e9
-    roof["frac"] = roof["achieved"] / HBM_PEAK_GBS
+    if roof["bound"] == "valu":  # matrix-free: one product of every sample
+        flop = work[0] * sum(b.n_samples) / its
+        roof["achieved"] = flop / (ms / 1e3) / 1e12
+        roof["avg_flop_per_launch"] = flop
+        roof["hbm_gbs"] = byts / (ms / 1e3) / 1e9
+    else:
+        roof["achieved"] = byts / (ms / 1e3) / 1e9
+    roof["frac"] = roof["achieved"] / roof["peak"]
     roof["avg_launch_ms"] = ms
     roof["avg_bytes_per_launch"] = byts
     roof["timing"] = f"{reps} back-to-back launches, every sample active, HIP events"
@@ -327,6 +336,10 @@ def back_to_back(roof, b, reps=20, rs=8):
 def spmv_name(b, real, tile):
     """Name of the SpMV+dot kernel entry, saying which product it runs."""
     if all(b.product_form(c) == "matrix_free" for c in range(len(b.meshes))):
+        if real == "double":
+            return ("k_pcg_p<double> + k_pcg_a_mf64 (p = z + beta p_old, then the matrix-free "
+                    "FP64 PCG product K p on box grids from the cell moduli, the corners' "
+                    "differences from the node's value, + p.q; time of both kernels)")
         return ("k_pcg_p + k_pcg_a_mf (p = z + beta p_old, then the matrix-free FP32 PCG "
                 "product K p on box grids from the cell moduli, the corners' differences from "
                 "the node's value, + p.q; time of both kernels)")
@@ -338,17 +351,18 @@ def spmv_name(b, real, tile):
 
 def spmv_roofline(b, kt, rs, name, counter_file, models=None):
     """Roofline entry of k_pcg_a from one kernel-timing solve (the
-    matrix-free product: FP32 VALU, like the smoothing products)."""
+    matrix-free product: FP32 or FP64 VALU)."""
     launches = kt["spmv_dot"]["launches"]
     a_s = kt["spmv_dot"]["ms"] / 1e3 / max(launches, 1)
-    mfw = mf_pcg_work(b, models) if models is not None else None
+    mfw = mf_pcg_work(b, models, rs) if models is not None else None
     if mfw is not None:
         flop, byts = mfw[0] / max(launches, 1), mfw[1] / max(launches, 1)
         ach = flop / a_s / 1e12 if a_s > 0 else 0.0
-        ratio = counters("k_pcg_a_mf_counters.json")
-        return dict(bound="valu", achieved=ach, peak=FP32_PEAK_TFLOPS, unit="TFLOP/s",
-                    frac=ach / FP32_PEAK_TFLOPS,
-                    frac_of_valu_without_packed_fp32=ach / FP32_VALU_NOPACK_TFLOPS,
+        ratio = counters("k_pcg_a_mf_counters.json") if rs == 4 else None
+        peak = FP32_PEAK_TFLOPS if rs == 4 else FP64_PEAK_TFLOPS
+        extra = dict(frac_of_valu_without_packed_fp32=ach / FP32_VALU_NOPACK_TFLOPS) if rs == 4 \
+            else {}
+        return dict(bound="valu", achieved=ach, peak=peak, unit="TFLOP/s", frac=ach / peak, **extra,
                     traffic=byts * ratio if ratio is not None else None,
                     traffic_over_algorithmic=ratio,
                     kernel=name, launches=launches, avg_launch_ms=1e3 * a_s,
@@ -474,10 +488,10 @@ def leg_c3(msa, ctx, args):
     kt = b.kernel_timing()
     b.set_kernel_timing(False)
     roof = spmv_roofline(b, kt, 8, spmv_name(b, "double", 1) + ", 256 x 32^3",
-                         "k_pcg_a_fp64_counters.json")
+                         "k_pcg_a_fp64_counters.json", [model])
     u = {s: b.solution(0, s) for s in (0, ns - 1)}
     pers = persistent_run(b, ctx, kw, u, args)
-    back_to_back(roof, b)
+    back_to_back(roof, b, models=[model])
     # independent check of two samples: the oracle's own CSR operator
     otab = O.kl_table([1.0, 1.0, 1.0], args.corr, args.terms)
     res = {}
@@ -494,7 +508,7 @@ def leg_c3(msa, ctx, args):
                oracle_true_residual=res, roofline=roof, persistent_launch=pers,
                kernel_timing_ms={k: v["ms"] for k, v in kt.items()})
     log(f"[bench] C3 256x32^3 FP64: {el:.2f} s -> {ns / el:.1f} solves/s, "
-        f"k_pcg_a<double> {roof['achieved']:.0f} GB/s, residuals {res}" +
+        f"PCG product {roof['achieved']:.0f} {roof['unit']}, residuals {res}" +
         (f"; persistent launch {pers['s_per_solve']:.2f} s (same bits: "
          f"{pers['same_bits_as_graph']})" if pers else ""))
     return out
@@ -523,10 +537,10 @@ def leg_c2(msa, ctx, args):
     kt = b.kernel_timing()
     b.set_kernel_timing(False)
     roof = spmv_roofline(b, kt, 8, spmv_name(b, "double", 1) + ", one 64^3 sample",
-                         "k_pcg_a_fp64_counters.json")
+                         "k_pcg_a_fp64_counters.json", [model])
     u = b.solution(0, 0)
     pers = persistent_run(b, ctx, kw, {0: u}, args)
-    back_to_back(roof, b)
+    back_to_back(roof, b, models=[model])
     res = oracle_true_residual(O, model, E, u)
     b.close()
     mesh.close()
@@ -535,8 +549,8 @@ def leg_c2(msa, ctx, args):
                ms_per_iteration=1e3 * el / max(int(st["iters"][0]), 1),
                oracle_true_residual=res, roofline=roof, persistent_launch=pers,
                kernel_timing_ms={k: v["ms"] for k, v in kt.items()})
-    log(f"[bench] C2 64^3 FP64: {el:.3f} s, {int(st['iters'][0])} its, k_pcg_a<double> "
-        f"{roof['achieved']:.0f} GB/s, oracle residual {res:.2e}" +
+    log(f"[bench] C2 64^3 FP64: {el:.3f} s, {int(st['iters'][0])} its, PCG product "
+        f"{roof['achieved']:.0f} {roof['unit']}, oracle residual {res:.2e}" +
         (f"; persistent launch {pers['s_per_solve']:.3f} s (same bits: "
          f"{pers['same_bits_as_graph']})" if pers else ""))
     return out

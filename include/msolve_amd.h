@@ -248,13 +248,20 @@ int msa_batch_layout_info(msa_batch *b, int cls, long long *info);
 int msa_batch_set_symmetric_product(msa_batch *b, int enable);
 
 /* The PCG product q = K p of box-grid classes computed matrix-free (enable
- * = 1, the default): MIXED batches of one-sample tiles with the multigrid
- * preconditioner, on the classes it coarsens (a class without coarser
- * levels keeps the stored product), whose finest smoothing products compute K v from
- * the cell moduli and the unit element matrix in FP32.  The product then
- * reads z, p_old and the moduli instead of the stored FP32 values; the
- * FP64 residual replacements (also matrix-free) fix the accuracy, and the
- * stored values are still assembled (export, coarse levels, warm starts).
+ * = 1, the default), in batches of one-sample tiles:
+ *   MIXED with the multigrid preconditioner, on the classes it coarsens (a
+ *   class without coarser levels keeps the stored product), whose finest
+ *   smoothing products compute K v from the cell moduli and the unit element
+ *   matrix in FP32; the FP64 residual replacements (also matrix-free) fix
+ *   the accuracy;
+ *   FP64 with any preconditioner, in FP64 throughout, on grids whose cells
+ *   are equal up to the rounding of the coordinates, in batches of at least
+ *   128 chunks of 256 block rows (below that the launches dominate and the
+ *   stored product needs one less), unless matrices were loaded
+ *   (msa_batch_set_matrix_csr) or the full image is selected
+ *   (msa_batch_set_symmetric_product).
+ * The product then reads z, p_old and the moduli instead of the stored
+ * values, which are still assembled (export, coarse levels, warm starts).
  * enable = 0: the stored-value product.  Takes effect at the next solve.
  * Replaces, for those classes, the role of SkylineMatrix2D.Multiply
  * (SkylineMatrix2D.cs:253-269) in SolverPCG.cs:120. */

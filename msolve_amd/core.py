@@ -401,8 +401,9 @@ class Batch:
 
     def set_matrix_free_product(self, enable: bool):
         """PCG product of box-grid classes matrix-free (True, the default:
-        MIXED, one-sample tiles, multigrid preconditioner) or from the
-        stored values (False); takes effect at the next solve."""
+        one-sample tiles; MIXED with the multigrid preconditioner, or FP64
+        batches of assembled matrices past a small size) or from the stored
+        values (False); takes effect at the next solve."""
         check(lib().msa_batch_set_matrix_free_product(self.h, 1 if enable else 0))
 
     def product_form(self, cls: int) -> str:

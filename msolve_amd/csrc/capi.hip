@@ -56,6 +56,7 @@ struct ClassHost {
     // slot within its row's slice of every adjacency entry (brow_ptr/bcol
     // order): its rank in the row, or its stencil slot on box grids
     std::vector<uint8_t> srank;
+    GridInfo grid;  // of a uniform-grid mesh (nx = 0: not one)
     int R = 64;  // block rows per slice
     int slot_of(const MeshHost &h, int br, int j) const
     {
@@ -206,18 +207,15 @@ int dalloc(msa_batch *b, void **p, size_t bytes)
 // strides in y and z; otherwise the entry's rank in the row, and false.
 // A box thinner than 3 points in x or y keeps the ranks: there the stencil
 // order is not the column order.
-bool stencil_ranks(const MeshHost &h, std::vector<uint8_t> &srank, int &sy, int &sz)
+bool stencil_ranks(const MeshHost &h, const GridInfo &g, std::vector<uint8_t> &srank, int &sy,
+                   int &sz)
 {
     srank.resize(h.bcol.size());
     for (int br = 0; br < h.nb; br++)
         for (int j = h.brow_ptr[br]; j < h.brow_ptr[br + 1]; j++)
             srank[j] = (uint8_t)(j - h.brow_ptr[br]);
     sy = sz = 0;
-    GridInfo g;
-    if (grid_info(h, g) != MSA_OK || !g.box) {
-        set_error("");
-        return false;
-    }
+    if (!g.box) return false;
     const int nx = g.box_hi[0] - g.box_lo[0] + 1, ny = g.box_hi[1] - g.box_lo[1] + 1;
     if (nx < 3 || ny < 3) return false;
     std::vector<uint8_t> st(h.bcol.size());
@@ -258,7 +256,11 @@ int setup_class(msa_batch *b, ClassHost &C, msa_mesh *mesh, int nsamp)
         C.nchunks = (C.nslices + C.chunk - 1) / C.chunk;
         C.R = R;
         int sy = 0, sz = 0;
-        const bool stencil = stencil_ranks(h, C.srank, sy, sz);
+        if (grid_info(h, C.grid) != MSA_OK) {
+            set_error("");
+            C.grid = GridInfo();
+        }
+        const bool stencil = stencil_ranks(h, C.grid, C.srank, sy, sz);
         C.slice_ptr.assign(C.nslices + 1, 0);
         for (int sl = 0; sl < C.nslices; sl++) {
             int wmax = 0;
@@ -502,7 +504,8 @@ hipError_t launch_product(msa_batch *b, int pbuf)
                             (int)b->items.size(), pbuf, b->d_counts);
     const hipError_t e = launch_pcg_a(s, is_mixed(b), b->T, b->unroll, b->d_cls, b->d_items_st,
                                       b->n_items_st, pbuf, b->d_counts);
-    return e != hipSuccess ? e : launch_pcg_a_mf(s, b->d_cls, b->d_items_mf, b->n_items_mf, pbuf);
+    return e != hipSuccess ? e : launch_pcg_a_mf(s, is_mixed(b), b->dyn, b->d_cls, b->d_items_mf,
+                                                     b->n_items_mf, pbuf);
 }
 
 // ru_tol > 0: reliable-update mode (inner test off, replacement triggers on).
@@ -688,7 +691,7 @@ int pcg_loop(msa_batch *b, int kind, double tol, int max_it, int graph_iters)
         int G = 0;
         MSA_HIP(launch_pcg_persist(b->ctx->stream, is_mixed(b), b->unroll, b->d_cls, b->d_items,
                                    (int)b->items.size(), b->d_tiles, (int)b->tiles.size(), ra, rb,
-                                   max_it + 1, &G));
+                                   max_it + 1, b->n_items_mf > 0, b->dyn, &G));
         b->persist_launches++;
         b->persist_grid = G;
         int active = 0;
@@ -1059,25 +1062,38 @@ void class_items(const ClassHost &C, int ci, std::vector<int4> &out)
 // Work items of the box-grid smoothing lists: runs of kMfRun chunks of one
 // tile, the run length in the item's w.
 constexpr int kMfRun = 4;
-void class_run_items(const ClassHost &C, int ci, std::vector<int4> &out)
+void class_run_items(const ClassHost &C, int ci, std::vector<int4> &out, int run = kMfRun)
 {
     for (int t = 0; t < C.ntiles; t++)
-        for (int k = 0; k < C.nchunks; k += kMfRun)
-            out.push_back(make_int4(ci, t, k, std::min(kMfRun, C.nchunks - k)));
+        for (int k = 0; k < C.nchunks; k += run)
+            out.push_back(make_int4(ci, t, k, std::min(run, C.nchunks - k)));
 }
 
-// Which box-grid classes take the matrix-free PCG product (the setting,
-// MIXED, one-sample tiles, the multigrid preconditioner set up: its unit
-// element matrix and grid tables serve the product), and their work items.
-// Called after the preconditioner values of a solve; a change re-uploads
-// the class table and drops the captured graphs (they hold the items).
+// Which box-grid classes take the matrix-free PCG product (sync_mf_pcg), and their work
+// items: with the setting on and one-sample tiles, MIXED batches with the
+// multigrid preconditioner set up (its unit element matrix and grid tables
+// serve the product), and FP64 batches of assembled matrices whose storage
+// was not switched to the full image.  Called after the preconditioner
+// values of a solve; a change re-uploads the class table and drops the
+// captured graphs (they hold the items).
+//
+// FP64, why: the stored product is bound by its values (64 x 32^3: 0.54 ms
+// per launch, 64^3: 65 us), the matrix-free one reads 24 bytes a node and
+// runs on the FP64 VALU (98 + 32 us with its p pass, 17.5 + 6 us).  Under
+// 128 chunks every kernel lasts as long as its launch, and the p pass is one
+// launch more: us per iteration, stored / matrix-free, 24^3 (60 chunks)
+// 21.9 / 24.6, 16 x 16^3 (304) 34.2 / 24.1, 32^3 (133) 27.2 / 20.1.
+bool mf64_large(const msa_batch *b) { return !is_mixed(b) && b->items.size() >= 128; }
+
 int sync_mf_pcg(msa_batch *b)
 {
     bool changed = false, any = false;
     for (auto &C : b->cls) {
-        const int want = b->mf_product && is_mixed(b) && b->T == 1 &&
-                         b->precond == MSA_PRECOND_MULTIGRID && b->mg_ready && C.dev.mf &&
-                         C.dev.mf_box;
+        const int want =
+            b->mf_product && b->T == 1 &&
+            (is_mixed(b) ? b->precond == MSA_PRECOND_MULTIGRID && b->mg_ready && C.dev.mf &&
+                               C.dev.mf_box
+                         : C.dev.mf64 && mf64_large(b) && !b->loaded && !b->full_storage);
         changed |= C.dev.mf_pcg != want;
         C.dev.mf_pcg = want;
         any |= want != 0;
@@ -1085,9 +1101,11 @@ int sync_mf_pcg(msa_batch *b)
     if (!changed) return MSA_OK;
     if (any) {
         std::vector<int4> st, mf;
+        // runs of up to kMfRun chunks while they leave 8 workgroups a CU
+        const int run = std::max(1, std::min(kMfRun, (int)(b->items.size() / 2048)));
         for (int c = 0; c < (int)b->cls.size(); c++) {
             if (b->cls[c].dev.mf_pcg)
-                class_run_items(b->cls[c], c, mf);
+                class_run_items(b->cls[c], c, mf, run);
             else
                 class_items(b->cls[c], c, st);
         }
@@ -1118,13 +1136,16 @@ int assemble_items(msa_batch *b, const int4 *items, int nitems, const int4 *gite
     });
 }
 
-// Matrix-free smoothing products for a class on a uniform structured grid
-// (mixed precision, one-sample tiles); other classes keep the stored values.
+// Tables of the matrix-free products for a class on a uniform structured
+// grid (one-sample tiles); other classes keep the stored values.  FP64
+// batches take box grids whose cells are equal up to the rounding of the
+// coordinates: the shared element matrix then is every element's to FP64
+// rounding (MIXED: cells equal to 1e-9, FP32 products).
 int mf_setup(msa_batch *b, ClassHost &C)
 {
-    if (!is_mixed(b) || b->T != 1 || C.dev.mf) return MSA_OK;
-    GridInfo g;
-    if (grid_info(C.mesh->h, g) != MSA_OK) return MSA_OK;
+    const GridInfo &g = C.grid;
+    if (b->T != 1 || C.dev.mf || C.dev.mf64 || g.nx == 0) return MSA_OK;
+    if (!is_mixed(b) && !(g.box && g.exact)) return MSA_OK;
     ClassDev &D = C.dev;
     MSA_TRY(upload_vec(b, g.gblock, &D.mf_gblock));
     MSA_TRY(upload_vec(b, g.cell_elem, &D.mf_cell));
@@ -1144,7 +1165,14 @@ int mf_setup(msa_batch *b, ClassHost &C)
         D.mf_box_lo[d] = g.box_lo[d];
         D.mf_box_hi[d] = g.box_hi[d];
     }
-    D.mf = 1;
+    const MeshHost &m = C.mesh->h;
+    D.mf_free = 1;
+    for (int bb = 0; bb < m.nb; bb++)
+        if (m.node_free[m.block_node[bb]] != 7) D.mf_free = 0;
+    if (is_mixed(b))
+        D.mf = 1;
+    else
+        D.mf64 = 1;
     return MSA_OK;
 }
 
@@ -2041,6 +2069,7 @@ int msa_batch_create(msa_ctx *ctx, int n_classes, msa_mesh *const *meshes, const
             for (int k = 0; k < C.nchunks; k++) b->items.push_back(make_int4(c, t, k, 0));
         }
     }
+    for (int c = 0; c < n_classes && rc == MSA_OK && mf64_large(b); c++) rc = mf_setup(b, b->cls[c]);
     if (rc != MSA_OK) return fail(rc);
     void *p = nullptr;
     rc = dalloc(b, &p, sizeof(ClassDev) * n_classes);
@@ -2224,6 +2253,8 @@ int msa_batch_assemble(msa_batch *b, double nu)
             MSA_TRY(timed(b, KK_ASSEMBLE, [&] {
                 return launch_khat_cache(s, b->d_cls + c, C.mesh->h.n_elem, nu, C.dev.dyn);
             }));
+            if (C.dev.mf64)
+                MSA_TRY(timed(b, KK_ASSEMBLE, [&] { return launch_mf_khat(s, b->d_cls + c); }));
             C.kc_nu = nu;
             C.kc_mass = C.dev.dyn;
         }

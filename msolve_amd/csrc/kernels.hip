@@ -1292,32 +1292,38 @@ __global__ __launch_bounds__(256) void k_pcg_a(const ClassDev *__restrict__ cls,
 }
 
 // The same step for box-grid classes whose product is matrix-free
-// (mf_pcg: MIXED, one-sample tiles, multigrid set up), in two passes over
-// an item's rows.  k_pcg_p writes p = z + beta p_old; k_pcg_a_mf then
-// computes q = K p from the cell moduli and the unit element matrix (the
-// operator of the finest smoothing products) with one gather per node,
-// and the p.q partials.  No stored value is read.  An item covers
-// max(1, it.w) consecutive chunks.
+// (mf_pcg: MIXED, one-sample tiles, multigrid set up; or FP64, one-sample
+// tiles), in two passes over an item's rows.  k_pcg_p writes p = z + beta
+// p_old; k_pcg_a_mf / k_pcg_a_mf64 then compute q = K p from the cell moduli
+// and the unit element matrix (the operator of the finest smoothing
+// products) with one gather per node, and the p.q partials.  No stored value
+// is read.  An item covers max(1, it.w) consecutive chunks.
+template <typename real>
+__device__ __forceinline__ void pcg_p_item(const ClassDev *__restrict__ cls, const int4 it, int pbuf)
+{
+    const ClassDev &C = cls[it.x];
+    const int tile = it.y, nch = max(1, it.w);
+    if (tile >= C.nsamp || !C.st[tile].active) return;  // one sample per tile
+    const real beta = (real)C.st[tile].beta;
+    const size_t vb = (size_t)tile * C.tile_vec;
+    const MSA_GLOBAL real *__restrict__ z = gbl((const real *)C.z + vb);
+    const MSA_GLOBAL real *__restrict__ po = gbl((const real *)(pbuf ? C.p1 : C.p0) + vb);
+    MSA_GLOBAL real *__restrict__ pn = gbl((real *)(pbuf ? C.p0 : C.p1) + vb);
+    const int r0 = it.z * C.chunk * 64, r1 = min((it.z + nch) * C.chunk * 64, C.nb);
+    for (int br = r0 + (int)threadIdx.x; br < r1; br += blockDim.x) {
+        const vec3<real> zc = ld3(z, br), pc = ld3(po, br);
+        st3(pn, br, zc.x + beta * pc.x, zc.y + beta * pc.y, zc.z + beta * pc.z);
+    }
+}
+
+template <typename real>
 __global__ __launch_bounds__(256) void k_pcg_p(const ClassDev *__restrict__ cls,
                                                const int4 *__restrict__ items, int nitems,
                                                int pbuf)
 {
     const int item = xcd_item(nitems);
     if (item < 0) return;
-    const int4 it = items[item];
-    const ClassDev &C = cls[it.x];
-    const int tile = it.y, nch = max(1, it.w);
-    if (tile >= C.nsamp || !C.st[tile].active) return;  // one sample per tile
-    const float beta = (float)C.st[tile].beta;
-    const size_t vb = (size_t)tile * C.tile_vec;
-    const MSA_GLOBAL float *__restrict__ z = gbl((const float *)C.z + vb);
-    const MSA_GLOBAL float *__restrict__ po = gbl((const float *)(pbuf ? C.p1 : C.p0) + vb);
-    MSA_GLOBAL float *__restrict__ pn = gbl((float *)(pbuf ? C.p0 : C.p1) + vb);
-    const int r0 = it.z * C.chunk * 64, r1 = min((it.z + nch) * C.chunk * 64, C.nb);
-    for (int br = r0 + (int)threadIdx.x; br < r1; br += blockDim.x) {
-        const vec3<float> zc = ld3(z, br), pc = ld3(po, br);
-        st3(pn, br, zc.x + beta * pc.x, zc.y + beta * pc.y, zc.z + beta * pc.z);
-    }
+    pcg_p_item<real>(cls, items[item], pbuf);
 }
 
 __global__ __launch_bounds__(256) void k_pcg_a_mf(const ClassDev *__restrict__ cls,
@@ -1362,6 +1368,56 @@ __global__ __launch_bounds__(256) void k_pcg_a_mf(const ClassDev *__restrict__ c
         // the next chunk's partials reuse the same LDS rows
         if (ck + 1 < chunk + nch) __syncthreads();
     }
+}
+
+// y = K v for block row br of a box-grid class in FP64 (defined with the
+// smoothing kernels below).
+template <bool DYN>
+__device__ __forceinline__ void mf64_product(const ClassDev &C, const MSA_GLOBAL double *v,
+                                             const double *Es, int br, double (&y)[3],
+                                             double (&own)[3]);
+
+template <bool DYN>
+__device__ __forceinline__ void pcg_a_mf64_item(const ClassDev *__restrict__ cls, const int4 it,
+                                                int pbuf)
+{
+    const ClassDev &C = cls[it.x];
+    const int tile = it.y, chunk = it.z, nch = max(1, it.w);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const bool act = tile < C.nsamp && C.st[tile].active;  // one sample per tile
+    const size_t vb = (size_t)tile * C.tile_vec;
+    const MSA_GLOBAL double *__restrict__ p = gbl((const double *)(pbuf ? C.p0 : C.p1) + vb);
+    MSA_GLOBAL double *__restrict__ q = gbl((double *)C.q + vb);
+    const double *Es = C.E + (size_t)tile * C.n_elem;
+    for (int ck = chunk; ck < chunk + nch; ck++) {
+        double pq = 0.0;
+        const int s0 = ck * C.chunk, s1 = min(s0 + C.chunk, C.nslices);
+        if (act) {
+            for (int slice = s0 + wave; slice < s1; slice += kWaves) {
+                const int br = slice * 64 + lane;
+                if (br >= C.nb) continue;
+                double y[3], own[3];
+                mf64_product<DYN>(C, p, Es, br, y, own);
+                st3(q, br, y[0], y[1], y[2]);
+                pq += own[0] * y[0] + own[1] * y[1] + own[2] * y[2];
+            }
+        }
+        double acc[1] = {pq};
+        block_partials<1, 1>(acc, C.partial + ((size_t)tile * C.nchunks + ck) * 3);
+        // the next chunk's partials reuse the same LDS rows
+        if (ck + 1 < chunk + nch) __syncthreads();
+    }
+}
+
+template <bool DYN>
+__global__ __launch_bounds__(256) void k_pcg_a_mf64(const ClassDev *__restrict__ cls,
+                                                    const int4 *__restrict__ items, int nitems,
+                                                    int pbuf)
+{
+    const int item = xcd_item(nitems);
+    if (item < 0) return;
+    pcg_a_mf64_item<DYN>(cls, items[item], pbuf);
 }
 
 // Update + preconditioner + stopping test (SolverPCG.cs:122-136):
@@ -2784,7 +2840,9 @@ __global__ __launch_bounds__(1024) void k_reduce(const ClassDev *__restrict__ cl
 // (so the same bits).  Work items go to XCDs in contiguous ranges, as
 // xcd_item does.  Every workgroup reads the active-sample count after the
 // same barrier, so all leave the loop together; `iters` bounds it.
-template <typename real, int T, int U>
+// MF (FP64 batches with matrix-free classes; 2: with the consistent mass):
+// the p pass and its barrier come first.
+template <typename real, int T, int U, int MF>
 __global__ __launch_bounds__(256) void k_pcg_persist(const ClassDev *__restrict__ cls,
                                                      const int4 *__restrict__ items, int nitems,
                                                      const int2 *__restrict__ tiles, int ntiles,
@@ -2807,8 +2865,19 @@ __global__ __launch_bounds__(256) void k_pcg_persist(const ClassDev *__restrict_
                                                              __HIP_MEMORY_SCOPE_AGENT)) <= 0)
             break;
         const int pbuf = (pbuf0 + k) & 1;
+        if constexpr (MF != 0) {
+            for (int i = i0; i < i1; i += gx)
+                if (cls[items[i].x].mf_pcg) pcg_p_item<real>(cls, items[i], pbuf);
+            barrier();
+        }
         for (int i = i0; i < i1; i += gx) {
-            pcg_a_item<real, T, U>(cls, items[i], pbuf);
+            bool mf = false;
+            if constexpr (MF != 0) mf = cls[items[i].x].mf_pcg != 0;
+            if (!mf) {
+                pcg_a_item<real, T, U>(cls, items[i], pbuf);
+            } else {
+                if constexpr (MF != 0) pcg_a_mf64_item<MF == 2>(cls, items[i], pbuf);
+            }
             __syncthreads();
         }
         barrier();
@@ -3258,6 +3327,14 @@ __global__ void k_mf_khat(const ClassDev *__restrict__ cp)
         C.mf_k[i] = (float)v;
         C.mf_k64[i] = v;
     }
+    if (i < 48) {
+        // the distinct values (mf_entry), from the row of grid corner 0
+        const int q = i >> 4, e = i & 15, p = e < 8 ? q : (e < 12 ? (q + 1) % 3 : (q + 2) % 3);
+        int o = e;  // corner of the entry
+        if (e >= 8) o = (e & 2 ? 1 << p : 0) | (e & 1 ? 1 << (3 - p - q) : 0);
+        const int a = C.mf_corner[0], b = C.mf_corner[o];
+        C.mf_k64[kMfK64S + i] = C.kc[(a * 8 + b) * 9 + 3 * p + q];
+    }
 }
 
 // FP64 residual r64 -= (cK E K + cM M) u64 of the samples due for a
@@ -3371,6 +3448,169 @@ __device__ __forceinline__ cdouble *mf_khat64(const ClassDev &C)
     return (cdouble *)kp;
 }
 
+// Entry (p, q) of the unit element matrix of an axis-aligned cell between its
+// corners a (row) and o, from the 16 distinct values of input component q:
+// with d = a xor o and s = the corner's sign per axis, Khat_qq depends on d
+// only (values 0..7), and Khat_pq = s_p(a) s_q(a) c m(d_r) (lambda sigma(d_q)
+// + mu sigma(d_p)), r the third axis, sigma(0) = 1, sigma(1) = -1: up to the
+// sign one of the values 8 + (p = q + 1 ? 0 : 4) + 2 [d_p != d_q] + d_r (the
+// quadrature is a product rule, so the factors separate for any cell
+// lengths).  All indices are compile-time constants: 16 scalar values per
+// component serve its 168 products, where the full matrix took 24 scalar
+// loads of 48 registers per row.
+struct MfEntry {
+    int idx, neg;
+};
+__device__ __forceinline__ constexpr MfEntry mf_entry(int a, int o, int p, int q)
+{
+    const int d = a ^ o;
+    if (p == q) return {d, 0};
+    const int r = 3 - p - q, dp = (d >> p) & 1, dq = (d >> q) & 1;
+    const int minus = (((a >> p) & 1) ^ ((a >> q) & 1)) ^ dq;
+    return {8 + (p == (q + 1) % 3 ? 0 : 4) + 2 * (dp ^ dq) + ((d >> r) & 1), minus};
+}
+
+// y = K v for block row br of a box-grid class in FP64, one input component
+// at a time as k_residual64_mf_box, summed over the corners' differences
+// from the node's own value (a translation stores no energy, so the node's
+// own corner drops out: 7 of 8 corners per cell); own receives v's value at
+// the node.  DYN adds the consistent mass.  Rows of constrained components
+// are zero, as in the stored matrix.
+template <bool DYN>
+__device__ __forceinline__ void mf64_product(const ClassDev &C, const MSA_GLOBAL double *v,
+                                             const double *Es, int br, double (&y)[3],
+                                             double (&own)[3])
+{
+    const int lane = threadIdx.x & 63;
+    const int nx = __builtin_amdgcn_readfirstlane(C.mf_nx);
+    const int ny = __builtin_amdgcn_readfirstlane(C.mf_ny);
+    const int nz = __builtin_amdgcn_readfirstlane(C.mf_nz);
+    const int nb = __builtin_amdgcn_readfirstlane(C.nb);
+    const int b0x = __builtin_amdgcn_readfirstlane(C.mf_box_lo[0]);
+    const int b0y = __builtin_amdgcn_readfirstlane(C.mf_box_lo[1]);
+    const int b0z = __builtin_amdgcn_readfirstlane(C.mf_box_lo[2]);
+    const int b1x = __builtin_amdgcn_readfirstlane(C.mf_box_hi[0]);
+    const int b1y = __builtin_amdgcn_readfirstlane(C.mf_box_hi[1]);
+    const int b1z = __builtin_amdgcn_readfirstlane(C.mf_box_hi[2]);
+    const int sy = b1x - b0x + 1, sz = sy * (b1y - b0y + 1);
+    const int ne = __builtin_amdgcn_readfirstlane(C.n_elem);
+    const __amdgpu_buffer_rsrc_t ub = wave_buffer((const void *)v, (unsigned)nb * 24u);
+    const __amdgpu_buffer_rsrc_t eb = wave_buffer((const void *)Es, (unsigned)ne * 8u);
+    const unsigned uout = (unsigned)nb * 24u, eout = (unsigned)ne * 8u;
+    const int g = gbl(C.mf_bpos)[br];
+    const int i = g & 1023, j = (g >> 10) & 1023, k = g >> 20;
+    const bool blo[3] = {i > b0x, j > b0y, k > b0z}, bhi[3] = {i < b1x, j < b1y, k < b1z};
+    unsigned off[9];
+#pragma unroll
+    for (int m = 0; m < 9; m++) {
+        const int dy = m % 3, dz = m / 3;
+        const bool in = (dy != 0 || blo[1]) && (dy != 2 || bhi[1]) && (dz != 0 || blo[2]) &&
+                        (dz != 2 || bhi[2]);
+        off[m] = in ? (unsigned)br * 24u + (unsigned)(24 * ((dy - 1) * sy + (dz - 1) * sz)) : uout;
+    }
+    // the 8 cells' moduli (cells outside the grid: 0)
+    const double cK = DYN ? C.cK : 1.0;
+    double Ec[8];
+    bool cin[8];
+    {
+        const bool lo[3] = {i > 0, j > 0, k > 0}, hi[3] = {i < nx - 1, j < ny - 1, k < nz - 1};
+        const int cy1 = nx - 1, cz1 = (nx - 1) * (ny - 1);
+        const int c0 = (i - 1) + cy1 * (j - 1) + cz1 * (k - 1);
+        int ce[8];
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+            const int cx = c & 1, cy = (c >> 1) & 1, cz = c >> 2;
+            cin[c] = (cx ? hi[0] : lo[0]) && (cy ? hi[1] : lo[1]) && (cz ? hi[2] : lo[2]);
+            ce[c] = cin[c] ? c0 + cx + cy * cy1 + cz * cz1 : 0;
+        }
+        if (!__builtin_amdgcn_readfirstlane(C.mf_cell_id)) {  // element numbers from the table
+            const MSA_GLOBAL int *cell = gbl(C.mf_cell);
+#pragma unroll
+            for (int c = 0; c < 8; c++) ce[c] = cell[ce[c]];
+        }
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+            Ec[c] = buffer_load_f64(eb, (int)(cin[c] ? (unsigned)ce[c] * 8u : eout), 0, 0);
+            if constexpr (DYN) Ec[c] *= cK;
+        }
+    }
+    // x - 1 / x + 1 values count where the neighbour is in the box
+    const double fm = blo[0] ? 1.0 : 0.0, fp = bhi[0] ? 1.0 : 0.0;
+    y[0] = y[1] = y[2] = 0.0;
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+        double xq[9], xm[9], xp[9], ym = 0.0;
+#pragma unroll
+        for (int m = 0; m < 9; m++)
+            xq[m] = buffer_load_f64(ub, (int)(off[m] + 8u * q), 0, 0);
+        // lane 0: the column at x - 1, lane 63: at x + 1 (the other lanes'
+        // values are replaced by the shifts)
+#pragma unroll
+        for (int m = 0; m < 9; m++) xm[m] = 0.0;
+        if (lane == 0 || lane == 63) {
+            const bool okx = lane == 0 ? blo[0] : bhi[0];
+            const unsigned sh = lane == 0 ? (unsigned)-24 : 24u;
+#pragma unroll
+            for (int m = 0; m < 9; m++)
+                xm[m] = buffer_load_f64(
+                    ub, (int)((okx && off[m] != uout) ? off[m] + sh + 8u * q : uout), 0, 0);
+        }
+        cdouble *ks = mf_khat64(C) + kMfK64S + 16 * q;
+        double kv[16];
+#pragma unroll
+        for (int e = 0; e < 16; e++) kv[e] = ks[e];
+        const double o0 = xq[4];
+#pragma unroll
+        for (int m = 0; m < 9; m++) {
+            xp[m] = __builtin_fma(fp, dpp_wave<kDppWaveShl1>(xm[m], xq[m]), -o0);
+            xm[m] = __builtin_fma(fm, dpp_wave<kDppWaveShr1>(xm[m], xq[m]), -o0);
+        }
+#pragma unroll
+        for (int m = 0; m < 9; m++)
+            if (m != 4) xq[m] -= o0;
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+            const int cx = c & 1, cy = (c >> 1) & 1, cz = c >> 2;
+            const int a = (1 - cx) + 2 * (1 - cy) + 4 * (1 - cz);  // the node's corner
+            double t[3] = {0.0, 0.0, 0.0}, mq = 0.0, ms = 0.0;
+            cdouble *mh = mf_khat64(C) + 576 + a * 8;
+#pragma unroll
+            for (int o = 0; o < 8; o++) {
+                if constexpr (DYN) ms += mh[o];
+                if (o == a) continue;  // no difference at the node itself
+                const int ox = o & 1, oy = (o >> 1) & 1, oz = o >> 2;
+                const int m = (cy + oy) + 3 * (cz + oz), dx = cx + ox;
+                const double d = dx == 0 ? xm[m] : (dx == 1 ? xq[m] : xp[m]);
+#pragma unroll
+                for (int p = 0; p < 3; p++) {
+                    const MfEntry e = mf_entry(a, o, p, q);
+                    t[p] = __builtin_fma(e.neg ? -kv[e.idx] : kv[e.idx], d, t[p]);
+                }
+                if constexpr (DYN) mq = __builtin_fma(mh[o], d, mq);
+            }
+#pragma unroll
+            for (int p = 0; p < 3; p++) y[p] = __builtin_fma(Ec[c], t[p], y[p]);
+            if constexpr (DYN) ym += cin[c] ? __builtin_fma(ms, o0, mq) : 0.0;
+            // cells in order: interleaving them costs a wave per SIMD
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (DYN) ym *= C.cM;
+        // the mass couples each component to itself only
+        own[q] = o0;
+        y[q] += ym;
+        // one component at a time: its sums are formed before the next one's
+        // loads (the compiler otherwise sinks them past the loads' branches
+        // and keeps all three components' values)
+        asm volatile("" : "+v"(y[0]), "+v"(y[1]), "+v"(y[2]) :: "memory");
+    }
+    if (!__builtin_amdgcn_readfirstlane(C.mf_free)) {
+        const uint8_t fr = C.block_free[br];
+        y[0] = (fr & 1) ? y[0] : 0.0;
+        y[1] = (fr & 2) ? y[1] : 0.0;
+        y[2] = (fr & 4) ? y[2] : 0.0;
+    }
+}
+
 __global__ __launch_bounds__(256) void k_residual64_mf_box(const ClassDev *__restrict__ cls,
                                                            const int4 *__restrict__ items,
                                                            int nitems)
@@ -3426,16 +3666,24 @@ __global__ __launch_bounds__(256) void k_residual64_mf_box(const ClassDev *__res
         {
             const int cy1 = nx - 1, cz1 = (nx - 1) * (ny - 1);
             const int c0 = (i - 1) + cy1 * (j - 1) + cz1 * (k - 1);
-            const bool ident = __builtin_amdgcn_readfirstlane(C.mf_cell_id) != 0;
+            bool cin[8];
+            int ce[8];
 #pragma unroll
             for (int c = 0; c < 8; c++) {
                 const int cx = c & 1, cy = (c >> 1) & 1, cz = c >> 2;
-                const bool cin = (cx ? hi[0] : lo[0]) && (cy ? hi[1] : lo[1]) && (cz ? hi[2] : lo[2]);
-                int ce = cin ? c0 + cx + cy * cy1 + cz * cz1 : 0;
-                if (!ident) ce = gbl(C.mf_cell)[ce];
-                const double e = buffer_load_f64(eb, (int)(cin ? (unsigned)ce * 8u : eout), 0, 0);
+                cin[c] = (cx ? hi[0] : lo[0]) && (cy ? hi[1] : lo[1]) && (cz ? hi[2] : lo[2]);
+                ce[c] = cin[c] ? c0 + cx + cy * cy1 + cz * cz1 : 0;
+            }
+            // (one branch for all cells, so that the 8 loads issue together)
+            if (!__builtin_amdgcn_readfirstlane(C.mf_cell_id)) {
+#pragma unroll
+                for (int c = 0; c < 8; c++) ce[c] = gbl(C.mf_cell)[ce[c]];
+            }
+#pragma unroll
+            for (int c = 0; c < 8; c++) {
+                const double e = buffer_load_f64(eb, (int)(cin[c] ? (unsigned)ce[c] * 8u : eout), 0, 0);
                 Ec[c] = e * cK;
-                Mc[c] = cin ? cM : 0.0;
+                Mc[c] = cin[c] ? cM : 0.0;
             }
         }
         // x - 1 / x + 1 values count where the neighbour is in the box
@@ -4905,23 +5153,32 @@ hipError_t launch_pcg_a(hipStream_t s, bool mixed, int T, int U, const ClassDev 
     MSA_PCG_LAUNCH(k_pcg_a, d_cls, items, nitems, pbuf, active_count);
 }
 
-hipError_t launch_pcg_a_mf(hipStream_t s, const ClassDev *d_cls, const int4 *items, int nitems,
-                           int pbuf)
+hipError_t launch_pcg_a_mf(hipStream_t s, bool mixed, bool dyn, const ClassDev *d_cls,
+                           const int4 *items, int nitems, int pbuf)
 {
     if (nitems <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_pcg_p, dim3(xcd_grid(nitems)), dim3(256), 0, s, d_cls, items, nitems,
-                       pbuf);
-    hipLaunchKernelGGL(k_pcg_a_mf, dim3(xcd_grid(nitems)), dim3(256), 0, s, d_cls, items, nitems,
-                       pbuf);
+    const dim3 grid(xcd_grid(nitems)), block(256);
+    if (mixed)
+        hipLaunchKernelGGL(k_pcg_p<float>, grid, block, 0, s, d_cls, items, nitems, pbuf);
+    else
+        hipLaunchKernelGGL(k_pcg_p<double>, grid, block, 0, s, d_cls, items, nitems, pbuf);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    if (mixed)
+        hipLaunchKernelGGL(k_pcg_a_mf, grid, block, 0, s, d_cls, items, nitems, pbuf);
+    else if (dyn)
+        hipLaunchKernelGGL(k_pcg_a_mf64<true>, grid, block, 0, s, d_cls, items, nitems, pbuf);
+    else
+        hipLaunchKernelGGL(k_pcg_a_mf64<false>, grid, block, 0, s, d_cls, items, nitems, pbuf);
     return hipGetLastError();
 }
 
-template <typename real, int U>
+template <typename real, int U, int MF>
 static hipError_t pcg_persist_u(hipStream_t s, const ClassDev *d_cls, const int4 *items, int nitems,
                                 const int2 *tiles, int ntiles, const ReduceArgs &ra,
                                 const ReduceArgs &rb, int iters, int *grid_out)
 {
-    const void *fn = (const void *)k_pcg_persist<real, 1, U>;
+    const void *fn = (const void *)k_pcg_persist<real, 1, U, MF>;
     int dev = 0, ncu = 0, coop = 0, per_cu = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev);
@@ -4943,21 +5200,26 @@ static hipError_t pcg_persist_u(hipStream_t s, const ClassDev *d_cls, const int4
 
 hipError_t launch_pcg_persist(hipStream_t s, bool mixed, int U, const ClassDev *d_cls,
                               const int4 *items, int nitems, const int2 *tiles, int ntiles,
-                              const ReduceArgs &ra, const ReduceArgs &rb, int iters, int *grid_out)
+                              const ReduceArgs &ra, const ReduceArgs &rb, int iters, bool any_mf,
+                              bool dyn, int *grid_out)
 {
     if (nitems <= 0) return hipSuccess;
-#define MSA_PERSIST_U(real)                                                                   \
+#define MSA_PERSIST_U(real, MF)                                                               \
     switch (U) {                                                                             \
-    case 1: return pcg_persist_u<real, 1>(s, d_cls, items, nitems, tiles, ntiles, ra, rb, iters, grid_out); \
-    case 2: return pcg_persist_u<real, 2>(s, d_cls, items, nitems, tiles, ntiles, ra, rb, iters, grid_out); \
-    case 3: return pcg_persist_u<real, 3>(s, d_cls, items, nitems, tiles, ntiles, ra, rb, iters, grid_out); \
-    case 4: return pcg_persist_u<real, 4>(s, d_cls, items, nitems, tiles, ntiles, ra, rb, iters, grid_out); \
+    case 1: return pcg_persist_u<real, 1, MF>(s, d_cls, items, nitems, tiles, ntiles, ra, rb, iters, grid_out); \
+    case 2: return pcg_persist_u<real, 2, MF>(s, d_cls, items, nitems, tiles, ntiles, ra, rb, iters, grid_out); \
+    case 3: return pcg_persist_u<real, 3, MF>(s, d_cls, items, nitems, tiles, ntiles, ra, rb, iters, grid_out); \
+    case 4: return pcg_persist_u<real, 4, MF>(s, d_cls, items, nitems, tiles, ntiles, ra, rb, iters, grid_out); \
     default: return hipErrorInvalidValue;                                                    \
     }
     if (mixed) {
-        MSA_PERSIST_U(float)
+        MSA_PERSIST_U(float, 0)
+    } else if (!any_mf) {
+        MSA_PERSIST_U(double, 0)
+    } else if (!dyn) {
+        MSA_PERSIST_U(double, 1)
     } else {
-        MSA_PERSIST_U(double)
+        MSA_PERSIST_U(double, 2)
     }
 #undef MSA_PERSIST_U
 }

@@ -459,6 +459,20 @@ int grid_info(const MeshHost &m, GridInfo &gi_out)
     g.nx = nx;
     g.ny = ny;
     g.nz = nz;
+    // equal cells up to the rounding of the coordinates: every node on its
+    // grid line and every spacing the mean one within 4 units in the last
+    // place of the largest coordinate (a generator's repeated addition
+    // rounds each coordinate once: 1 unit per spacing)
+    g.exact = 1;
+    for (int d = 0; d < 3; d++) {
+        const double big = std::max(std::abs(gx[d].front()), std::abs(gx[d].back()));
+        const double tol = 4.0 * 2.220446049250313e-16 * big;
+        const double h = (gx[d].back() - gx[d].front()) / (double)(gx[d].size() - 1);
+        for (size_t i = 0; i + 1 < gx[d].size(); i++)
+            if (std::abs((gx[d][i + 1] - gx[d][i]) - h) > tol) g.exact = 0;
+        for (int n = 0; n < m.n_nodes && g.exact; n++)
+            if (std::abs(m.xyz[3 * n + d] - gx[d][gi[d][n]]) > tol) g.exact = 0;
+    }
     g.gblock.assign((size_t)nx * ny * nz, -2);
     for (int n = 0; n < m.n_nodes; n++) {
         const size_t p = gi[0][n] + (size_t)nx * (gi[1][n] + (size_t)ny * gi[2][n]);

@@ -130,6 +130,7 @@ struct GridInfo {
     std::vector<int> gblock, cell_elem, bpos;
     int corner_node[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     int cell_identity = 0;  // element number == cell number
+    int exact = 0;          // equal cells up to the rounding of the coordinates
     int box = 0;            // the blocks are exactly the grid points of [box_lo, box_hi],
     int box_lo[3] = {0, 0, 0}, box_hi[3] = {0, 0, 0};  // numbered lexicographically
 };
@@ -137,9 +138,11 @@ int grid_info(const MeshHost &m, GridInfo &g);
 
 // Device view of one class of a batch (copied to device memory).
 // FP64 unit element matrix of matrix-free classes: Khat (576) + Mhat (64),
-// then Khat transposed by input component (576)
+// then Khat transposed by input component (576), then its distinct values by
+// input component (kMfK64S, 16 each; mf64_product)
 constexpr int kMfK64T = 640;
-constexpr int kMfK64 = 640 + 576;
+constexpr int kMfK64S = 640 + 576;
+constexpr int kMfK64 = 640 + 576 + 48;
 
 struct ClassDev {
     int nb, nslices, ntiles, nsamp;
@@ -244,8 +247,13 @@ struct ClassDev {
     int mf_cell_id, mf_box;
     int mf_box_lo[3], mf_box_hi[3];
     // the PCG product q = K p of this box-grid class matrix-free as well
-    // (set per solve: MIXED, one-sample tiles, multigrid set up)
+    // (set per solve: MIXED, one-sample tiles, multigrid set up; or FP64,
+    // mf64)
     int mf_pcg;
+    // FP64 batches, one-sample tiles: a box grid whose cells are equal up to
+    // the rounding of the coordinates (mf stays 0; the mf_ tables and mf_k64
+    // are set).  mf_free: every block fully free.
+    int mf64, mf_free;
     // FP64 copy of the stored values (same layout as a one-sample-tile FP64
     // batch) for the coarsest multigrid level of a MIXED batch: the band
     // factor is computed from these, not from the FP32 values (null: none)
@@ -375,8 +383,9 @@ hipError_t launch_pcg_a(hipStream_t s, bool mixed, int T, int U, const ClassDev 
                         const int4 *items, int nitems, int pbuf, int *active_count);
 hipError_t launch_residual64_mf_box(hipStream_t s, const ClassDev *d_cls, const int4 *items,
                                    int nitems);
-hipError_t launch_pcg_a_mf(hipStream_t s, const ClassDev *d_cls, const int4 *items, int nitems,
-                           int pbuf);
+// mixed: FP32 vectors and product, else FP64; dyn: with the consistent mass
+hipError_t launch_pcg_a_mf(hipStream_t s, bool mixed, bool dyn, const ClassDev *d_cls,
+                           const int4 *items, int nitems, int pbuf);
 hipError_t launch_pcg_b(hipStream_t s, bool mixed, int T, const ClassDev *d_cls, const int4 *items,
                         int nitems, int pbuf, double tol, int max_it, int *active_count);
 hipError_t launch_ir_begin(hipStream_t s, int T, const ClassDev *d_cls, const int4 *items,
@@ -487,9 +496,11 @@ hipError_t launch_extract_sample(hipStream_t s, bool mixed, int T, const void *s
                                  int lane, double *dst);
 // The whole Jacobi-PCG (one-sample tiles) in one cooperative launch of at
 // most `iters` iterations; *grid_out = workgroups launched.
+// any_mf: some class takes the (FP64) matrix-free product.
 hipError_t launch_pcg_persist(hipStream_t s, bool mixed, int U, const ClassDev *d_cls,
                               const int4 *items, int nitems, const int2 *tiles, int ntiles,
-                              const ReduceArgs &ra, const ReduceArgs &rb, int iters, int *grid_out);
+                              const ReduceArgs &ra, const ReduceArgs &rb, int iters, bool any_mf,
+                              bool dyn, int *grid_out);
 // Lanczos estimate of the top of the spectrum of D^-1 K per sample and
 // level (the upper end of the Chebyshev smoothing interval).  op: 0 start
 // vector, 2 alpha partials, 3 next vector and its D-norm partials; sum

@@ -1,0 +1,129 @@
+"""The FP64 matrix-free PCG product (box grids of equal cells, one-sample
+tiles): against the stored upper-triangle product and the full image on the
+same batch over the grids it accepts (rows shorter and longer than a
+wavefront, one or two nodes across, partly constrained blocks, unequal cell
+lengths), static and dynamic; what it does not accept keeps the stored
+product; the persistent launch gives the same bits.
+
+Both products are FP64 sums of the same terms, so each row agrees to a few
+rounding errors of |K||p| and two solves to a residual of 1e-12 agree to
+about 1e-12 times the condition number of these small blocks (below 1e4)."""
+import numpy as np
+import pytest
+
+import msolve_amd as msa
+from msolve_amd import _lib as L
+from msolve_amd.model import box_mesh
+
+pytestmark = pytest.mark.gpu
+
+NS = 130  # samples of one chunk each: past the 128 chunks the product starts at
+
+
+def rel(a, b):
+    return float(np.linalg.norm(a - b) / np.linalg.norm(b))
+
+
+def block(shape, lengths=None, roller=False):
+    """Block clamped at x = 0 (roller: the x = end face also held in z)."""
+    lengths = lengths or [float(v) for v in shape]
+    xyz, conn = box_mesh(*shape, *lengths)
+    cons = np.zeros((xyz.shape[0], 3), bool)
+    cons[xyz[:, 0] < 1e-12] = True
+    if roller:
+        cons[xyz[:, 0] > lengths[0] * (1 - 1e-12), 2] = True
+    dof, nf = msa.enumerate_dofs(cons)
+    f = np.random.default_rng(1).standard_normal(nf)
+    return xyz, conn, dof, nf, f
+
+
+def solve(ctx, blk, ns, E, form, persistent=False, dyn=False):
+    xyz, conn, dof, nf, f = blk
+    mesh = msa.Mesh(ctx, xyz, conn, dof, nf)
+    b = msa.Batch(ctx, [mesh], [ns], L.MSA_FP64, 1)
+    b.set_matrix_free_product(form == "matrix_free")
+    b.set_symmetric_product(form != "stored")
+    b.set_persistent(persistent)
+    b.set_modulus(0, E)
+    b.set_rhs(0, f)
+    if dyn:
+        b.set_dynamics(1e-2, 0.5, 1e-3, 0.25, 0.5, 1e-2)
+    b.assemble(0.3)
+    b.solve(tol=1e-12, max_it=20000, graph_iters=8)
+    st = b.stats(0)
+    assert (st["status"] == msa.MSA_OK).all()
+    got = b.product_form(0)
+    u = [b.solution(0, s) for s in range(0, ns, max(1, ns // 4))]
+    b.close()
+    mesh.close()
+    return u, st["iters"], got
+
+
+GRIDS = [dict(shape=(4, 3, 2)), dict(shape=(3, 1, 1)), dict(shape=(2, 2, 1)),
+         dict(shape=(1, 4, 3)), dict(shape=(70, 1, 2), lengths=[4.0, 1.0, 1.0]),
+         dict(shape=(5, 4, 3), roller=True),
+         dict(shape=(6, 4, 5), lengths=[1.0, 0.3, 2.0])]
+
+
+@pytest.mark.parametrize("dyn", [False, True])
+@pytest.mark.parametrize("grid", GRIDS)
+def test_matrix_free_fp64_product(ctx, grid, dyn):
+    blk = block(**grid)
+    ns = NS
+    E = 2.1e5 * np.exp(0.3 * np.random.default_rng(2).standard_normal((ns, blk[1].shape[0])))
+    out = {f: solve(ctx, blk, ns, E, f, dyn=dyn)
+           for f in ("matrix_free", "upper_triangle", "stored")}
+    thin = grid["shape"][0] < 3 or grid["shape"][1] < 2
+    assert out["matrix_free"][2] == "matrix_free"
+    assert out["upper_triangle"][2] == ("stored" if thin else "upper_triangle")
+    assert out["stored"][2] == "stored"
+    for f in ("upper_triangle", "stored"):
+        d = max(rel(a, b) for a, b in zip(out["matrix_free"][0], out[f][0]))
+        print(f"\n[case] {grid} dyn={dyn} vs {f}: {d:.2e}", flush=True)
+        assert d < 1e-8
+        assert np.abs(out["matrix_free"][1] - out[f][1]).max() <= 3
+
+
+def test_large_grid_and_persistent(ctx):
+    blk = block((33, 31, 34))
+    E = 2.1e5 * np.exp(0.3 * np.random.default_rng(3).standard_normal((1, blk[1].shape[0])))
+    um, im, fm = solve(ctx, blk, 1, E, "matrix_free")
+    us, is_, fs = solve(ctx, blk, 1, E, "upper_triangle")
+    up, ip, fp = solve(ctx, blk, 1, E, "matrix_free", persistent=True)
+    assert (fm, fs, fp) == ("matrix_free", "upper_triangle", "matrix_free")
+    assert rel(um[0], us[0]) < 1e-9 and abs(int(im[0]) - int(is_[0])) <= 3
+    assert np.array_equal(um[0], up[0]) and np.array_equal(im, ip)
+
+
+def test_what_keeps_the_stored_product(ctx):
+    # a grid off by more than rounding, a small batch, a loaded matrix, lane tiles
+    xyz, conn, dof, nf, f = block((4, 3, 2))
+    E = np.full((NS, conn.shape[0]), 2.1e5)
+    bent = xyz.copy()
+    bent[np.isclose(xyz[:, 0], 2.0), 0] += 1e-12
+    assert solve(ctx, (bent, conn, dof, nf, f), NS, E, "matrix_free")[2] != "matrix_free"
+    assert solve(ctx, (xyz, conn, dof, nf, f), 4, E[:4], "matrix_free")[2] != "matrix_free"
+    mesh = msa.Mesh(ctx, xyz, conn, dof, nf)
+    b = msa.Batch(ctx, [mesh], [NS], L.MSA_FP64, 1)
+    b.set_modulus(0, E)
+    b.set_rhs(0, f)
+    b.assemble(0.3)
+    rp, col, val = b.matrix_csr(0, 0)
+    for s in range(NS):
+        b.set_matrix_csr(0, s, rp, col, 2.0 * val)
+    b.solve(tol=1e-11, max_it=5000, graph_iters=8)
+    assert b.product_form(0) == "upper_triangle"
+    u2 = b.solution(0, 5)
+    b.assemble(0.3)
+    b.solve(tol=1e-11, max_it=5000, graph_iters=8)
+    assert b.product_form(0) == "matrix_free"
+    assert rel(2.0 * u2, b.solution(0, 5)) < 1e-8
+    b.close()
+    bt = msa.Batch(ctx, [mesh], [NS], L.MSA_FP64, 2)
+    bt.set_modulus(0, E)
+    bt.set_rhs(0, f)
+    bt.assemble(0.3)
+    bt.solve(tol=1e-11, max_it=5000, graph_iters=8)
+    assert bt.product_form(0) == "stored"
+    bt.close()
+    mesh.close()
