@@ -527,7 +527,13 @@ int launch_iteration_pair(msa_batch *b, int pbuf, double tol, int max_it, double
     return MSA_OK;
 }
 
-ColourLaunch colour_launch(const msa_batch *b, int colour, int *nblocks, bool skip_mf = false);
+// Classes an element-by-element (coloured) launch leaves to a matrix-free
+// kernel: none; those whose replacement residual is matrix-free; of these
+// the ones whose cells are equal up to coordinate rounding (residual at the
+// start of a Newmark step); the box grids among the latter (its right-hand
+// side).
+enum ColourSkip { SKIP_NONE = 0, SKIP_MF, SKIP_MF_EXACT, SKIP_MF_RHS };
+ColourLaunch colour_launch(const msa_batch *b, int colour, int *nblocks, ColourSkip skip = SKIP_NONE);
 int max_colours(const msa_batch *b);
 
 int max_tiles(const msa_batch *b)
@@ -535,6 +541,24 @@ int max_tiles(const msa_batch *b)
     int m = 1;
     for (auto &c : b->cls) m = std::max(m, c.ntiles);
     return m;
+}
+
+// Whether uniform-grid classes of a MIXED batch have their FP64 residual
+// formed matrix-free (multigrid set up), and those launches.
+bool mf_residual(const msa_batch *b)
+{
+    return is_mixed(b) && b->precond == MSA_PRECOND_MULTIGRID && b->mg_ready &&
+           b->n_mf_items + b->n_mf_box_items > 0;
+}
+int launch_residual_mf(msa_batch *b, int need_due)
+{
+    hipStream_t s = b->ctx->stream;
+    return timed(b, KK_RES64, [&] {
+        const hipError_t e = launch_residual64_mf(s, b->d_cls, b->mf_items, b->n_mf_items, need_due);
+        return e != hipSuccess ? e
+                               : launch_residual64_mf_box(s, b->dyn, b->d_cls, b->mf_box_items,
+                                                          b->n_mf_box_items, need_due);
+    });
 }
 
 // Fold the FP32 correction into u64, form the FP64 residual, test it and
@@ -546,19 +570,12 @@ int launch_replacement(msa_batch *b, double tol, int max_it)
     MSA_TRY(timed(b, KK_OTHER, [&] { return launch_ru_fold(s, T, b->d_cls, b->d_items, ni); }));
     // matrix-free residual of the uniform-grid classes (multigrid set up),
     // the coloured element scatter for the others
-    const bool mfres = b->precond == MSA_PRECOND_MULTIGRID && b->mg_ready &&
-                       b->n_mf_items + b->n_mf_box_items > 0;
-    if (mfres)
-        MSA_TRY(timed(b, KK_RES64, [&] {
-            const hipError_t e = launch_residual64_mf(s, b->d_cls, b->mf_items, b->n_mf_items);
-            return e != hipSuccess
-                       ? e
-                       : launch_residual64_mf_box(s, b->d_cls, b->mf_box_items, b->n_mf_box_items);
-        }));
+    const bool mfres = mf_residual(b);
+    if (mfres) MSA_TRY(launch_residual_mf(b, 1));
     const int ncol = max_colours(b);
     for (int k = 0; k < ncol; k++) {
         int nblk = 0;
-        ColourLaunch cl = colour_launch(b, k, &nblk, mfres);
+        ColourLaunch cl = colour_launch(b, k, &nblk, mfres ? SKIP_MF : SKIP_NONE);
         if (nblk == 0) continue;
         MSA_TRY(timed(b, KK_RES64, [&] { return launch_residual64(s, T, b->d_cls, cl, nblk, b->nu, 1, max_tiles(b)); }));
     }
@@ -734,8 +751,7 @@ int pcg_loop(msa_batch *b, int kind, double tol, int max_it, int graph_iters)
     return MSA_OK;
 }
 
-// skip_mf: leave out the classes whose replacement residual is matrix-free
-ColourLaunch colour_launch(const msa_batch *b, int colour, int *nblocks, bool skip_mf)
+ColourLaunch colour_launch(const msa_batch *b, int colour, int *nblocks, ColourSkip skip)
 {
     ColourLaunch cl{};
     cl.ncls = (int)b->cls.size();
@@ -744,7 +760,11 @@ ColourLaunch colour_launch(const msa_batch *b, int colour, int *nblocks, bool sk
     for (size_t c = 0; c < b->cls.size(); c++) {
         const MeshHost &m = b->cls[c].mesh->h;
         int cnt = colour < m.ncolours ? m.colour_ptr[colour + 1] - m.colour_ptr[colour] : 0;
-        if (skip_mf && b->cls[c].dev.mf) cnt = 0;
+        const ClassDev &D = b->cls[c].dev;
+        const bool box = is_mixed(b) ? D.mf && D.mf_box : D.mf_pcg != 0;
+        if ((skip == SKIP_MF && D.mf) || (skip == SKIP_MF_EXACT && D.mf && D.mf_exact) ||
+            (skip == SKIP_MF_RHS && box && D.mf_exact))
+            cnt = 0;
         cl.prefix[c + 1] = cl.prefix[c] + cnt;
     }
     *nblocks = cl.prefix[cl.ncls];
@@ -1166,6 +1186,7 @@ int mf_setup(msa_batch *b, ClassHost &C)
         D.mf_box_hi[d] = g.box_hi[d];
     }
     const MeshHost &m = C.mesh->h;
+    D.mf_exact = g.exact;
     D.mf_free = 1;
     for (int bb = 0; bb < m.nb; bb++)
         if (m.node_free[m.block_node[bb]] != 7) D.mf_free = 0;
@@ -2502,9 +2523,19 @@ int newmark_head(msa_batch *b, const DynCoef &dc, double tol, int max_it)
     const bool mx = is_mixed(b);
     const int T = b->T, ni = (int)b->items.size(), ncol = max_colours(b);
     MSA_TRY(timed(b, KK_OTHER, [&] { return launch_dyn_prep(s, mx, T, b->d_cls, b->d_items, ni, dc); }));
+    // box grids of equal cells matrix-free (64 samples of 48x48x24: 2.4 ms
+    // per step for the 8 colours), the element scatter for the others
+    const bool mfres = mf_residual(b);
+    const bool mfrhs = mx ? mfres : b->n_items_mf > 0;
+    if (mfrhs)
+        MSA_TRY(timed(b, KK_RES64, [&] {
+            return launch_dyn_rhs_mf(s, dc.betaR != 0.0, b->d_cls, mx ? b->mf_box_items : b->d_items_mf,
+                                     mx ? b->n_mf_box_items : b->n_items_mf);
+        }));
     for (int k = 0; k < ncol; k++) {
         int nblk = 0;
-        ColourLaunch cl = colour_launch(b, k, &nblk);
+        ColourLaunch cl = colour_launch(b, k, &nblk, mfrhs ? SKIP_MF_RHS : SKIP_NONE);
+        if (nblk == 0) continue;
         MSA_TRY(timed(b, KK_RES64, [&] { return launch_dyn_rhs(s, T, b->d_cls, cl, nblk, b->nu, dc.betaR, max_tiles(b)); }));
     }
     MSA_TRY(timed(b, KK_OTHER, [&] { return launch_fs_norm(s, T, b->d_cls, b->d_items, ni); }));
@@ -2527,9 +2558,11 @@ int newmark_head(msa_batch *b, const DynCoef &dc, double tol, int max_it)
     MSA_TRY(timed(b, KK_OTHER, [&] { return launch_set_int(s, b->d_counts, 2, 0); }));
     const int warm = dc.start ? 1 : 0;
     MSA_TRY(timed(b, KK_OTHER, [&] { return launch_ir_begin(s, T, b->d_cls, b->d_items, ni, b->d_counts + 1, warm); }));
+    if (mfres) MSA_TRY(launch_residual_mf(b, 0));
     for (int k = 0; k < ncol; k++) {
         int nblk = 0;
-        ColourLaunch cl = colour_launch(b, k, &nblk);
+        ColourLaunch cl = colour_launch(b, k, &nblk, mfres ? SKIP_MF_EXACT : SKIP_NONE);
+        if (nblk == 0) continue;
         MSA_TRY(timed(b, KK_RES64, [&] { return launch_residual64(s, T, b->d_cls, cl, nblk, b->nu, 0, max_tiles(b)); }));
     }
     MSA_TRY(timed(b, KK_OTHER, [&] {

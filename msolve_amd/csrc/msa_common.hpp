@@ -138,11 +138,10 @@ int grid_info(const MeshHost &m, GridInfo &g);
 
 // Device view of one class of a batch (copied to device memory).
 // FP64 unit element matrix of matrix-free classes: Khat (576) + Mhat (64),
-// then Khat transposed by input component (576), then its distinct values by
-// input component (kMfK64S, 16 each; mf64_product)
-constexpr int kMfK64T = 640;
-constexpr int kMfK64S = 640 + 576;
-constexpr int kMfK64 = 640 + 576 + 48;
+// then Khat's distinct values by input component (kMfK64S, 16 each;
+// mf64_product)
+constexpr int kMfK64S = 640;
+constexpr int kMfK64 = 640 + 48;
 
 struct ClassDev {
     int nb, nslices, ntiles, nsamp;
@@ -237,9 +236,7 @@ struct ClassDev {
     // matrix-free smoothing products (mixed precision, one-sample tiles) on
     // a uniform structured grid: K v from the cell moduli and the shared
     // unit element matrix mf_k[576] (+ unit mass mf_k[576 + 64])
-    // (mf_k64: the same in FP64, then Khat again at kMfK64T with the 3x3
-    // blocks transposed and grouped by (a, input component q, b):
-    // [((a * 3 + q) * 8 + b) * 3 + p] = Khat[a][b][p][q])
+    // (mf_k64: the same in FP64, then the distinct values at kMfK64S)
     int mf, mf_nx, mf_ny, mf_nz;
     int mf_corner[8];
     // index shortcuts: element = cell (mf_cell_id); blocks = a lexicographic
@@ -254,6 +251,7 @@ struct ClassDev {
     // the rounding of the coordinates (mf stays 0; the mf_ tables and mf_k64
     // are set).  mf_free: every block fully free.
     int mf64, mf_free;
+    int mf_exact;  // mf / mf64 class whose cells are equal up to coordinate rounding
     // FP64 copy of the stored values (same layout as a one-sample-tile FP64
     // batch) for the coarsest multigrid level of a MIXED batch: the band
     // factor is computed from these, not from the FP32 values (null: none)
@@ -264,7 +262,7 @@ struct ClassDev {
     int mf_allfree;
     const int *mf_gblock, *mf_cell, *mf_bpos;
     float *mf_k;
-    double *mf_k64;       // [640] the same in FP64 (replacement residuals)
+    double *mf_k64;       // [kMfK64] the same in FP64 (replacement residuals, FP64 products)
 };
 
 // Samples a multigrid cycle serves: 0 every sample, 1 active, 2 due for a
@@ -381,8 +379,11 @@ hipError_t launch_pcg_init(hipStream_t s, bool mixed, int T, const ClassDev *d_c
 // U: slots per group of a row (1..4 at T = 1, 3 for T > 1)
 hipError_t launch_pcg_a(hipStream_t s, bool mixed, int T, int U, const ClassDev *d_cls,
                         const int4 *items, int nitems, int pbuf, int *active_count);
-hipError_t launch_residual64_mf_box(hipStream_t s, const ClassDev *d_cls, const int4 *items,
-                                   int nitems);
+// need_due 1: the samples due for a replacement, 0: every refining one
+hipError_t launch_residual64_mf_box(hipStream_t s, bool dyn, const ClassDev *d_cls,
+                                   const int4 *items, int nitems, int need_due);
+hipError_t launch_dyn_rhs_mf(hipStream_t s, bool stiff, const ClassDev *d_cls, const int4 *items,
+                             int nitems);
 // mixed: FP32 vectors and product, else FP64; dyn: with the consistent mass
 hipError_t launch_pcg_a_mf(hipStream_t s, bool mixed, bool dyn, const ClassDev *d_cls,
                            const int4 *items, int nitems, int pbuf);
@@ -459,7 +460,8 @@ hipError_t launch_mg_band_out(hipStream_t s, bool mixed, int T, const ClassDev *
                               int nrows, int mode);
 hipError_t launch_mf_khat(hipStream_t s, const ClassDev *cp);
 // replacement residual of the due samples of matrix-free classes (T = 1)
-hipError_t launch_residual64_mf(hipStream_t s, const ClassDev *d_cls, const int4 *items, int nitems);
+hipError_t launch_residual64_mf(hipStream_t s, const ClassDev *d_cls, const int4 *items, int nitems,
+                                int need_due);
 // coarsest multigrid level: dense inverse from the band factor, and its use
 hipError_t launch_band_inverse(hipStream_t s, const ClassDev *cp, int nsamp, int bn);
 hipError_t launch_mg_dense_solve(hipStream_t s, bool mixed, int T, const ClassDev *cp, int nsamp,

@@ -127,3 +127,40 @@ def test_what_keeps_the_stored_product(ctx):
     assert bt.product_form(0) == "stored"
     bt.close()
     mesh.close()
+
+
+@pytest.mark.parametrize("precision", [L.MSA_FP64, L.MSA_MIXED])
+@pytest.mark.parametrize("beta", [0.0, 1e-3])
+@pytest.mark.parametrize("grid", [dict(shape=(8, 6, 4)), dict(shape=(68, 4, 4), lengths=[8.0, 2.0, 2.0]),
+                                  dict(shape=(8, 4, 6), roller=True)])
+def test_newmark_step_forms(ctx, grid, beta, precision):
+    """A Newmark run on a grid of equal cells (right-hand side and first
+    residual matrix-free) against the same grid with one plane moved by
+    1e-12, which keeps the element-by-element kernels: steps solved to 1e-11
+    agree to that, amplified over the steps."""
+    xyz, conn, dof, nf, f = block(**grid)
+    bent = xyz.copy()
+    bent[np.isclose(xyz[:, 1], grid.get("lengths", grid["shape"])[1] / 2), 1] += 1e-12
+    ns = NS if precision == L.MSA_FP64 else 3
+    E = 2.1e5 * np.exp(0.3 * np.random.default_rng(5).standard_normal((ns, conn.shape[0])))
+    acc = 1e3 * np.sin(np.arange(1, 6))
+    out = []
+    for x in (xyz, bent):
+        mesh = msa.Mesh(ctx, x, conn, dof, nf)
+        b = msa.Batch(ctx, [mesh], [ns], precision, 1)
+        if precision == L.MSA_MIXED:
+            b.set_preconditioner(msa.MSA_PRECOND_MULTIGRID)
+            assert b.mg_info(0)["levels"] >= 1
+        b.set_modulus(0, E)
+        b.set_rhs(0, f)
+        b.set_dynamics(1e-2, 0.5, beta, 0.25, 0.5, 1e-2)
+        b.set_probe(0, nf - 2)
+        b.assemble(0.3)
+        b.newmark(acc, 1, 1e-11, 20000, 8)
+        out.append([(b.history(0, s), *b.dynamic_state(0, s)[:3]) for s in (0, ns - 1)])
+        b.close()
+        mesh.close()
+    for a, c in zip(*out):
+        d = [rel(x, y) for x, y in zip(a, c)]
+        print(f"\n[case] newmark {grid} beta={beta} precision={precision}: {d}", flush=True)
+        assert d[0] < 1e-8 and d[1] < 1e-8 and d[2] < 1e-6 and d[3] < 1e-6
