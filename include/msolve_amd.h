@@ -455,10 +455,12 @@ int msa_batch_set_matrix_cores(msa_batch *b, int enable);
  * coarsest level, [2] free DOFs summed over the coarse levels, [3] half
  * bandwidth of the coarsest level, [4] 1 if the finest level's smoothing
  * products are matrix-free, [5] the number of coarse levels that are.
- * Matrix-free products are used by MIXED batches with one-sample tiles on
- * grids of equal, equally oriented cells (all elements share one element
- * matrix): K v from the cell moduli and that matrix in FP32, without
- * reading the stored values. */
+ * These count the FP32 form: MIXED batches with one-sample tiles on grids of
+ * equal, equally oriented cells (all elements share one element matrix): K v
+ * from the cell moduli and that matrix, without reading the stored values.
+ * FP64 batches report 0; on box grids of cells equal up to coordinate
+ * rounding (one-sample tiles, upper-triangle storage) their smoothing
+ * products have the same form in FP64. */
 int msa_batch_mg_info(msa_batch *b, int cls, long long *info);
 /* Upper end lam of each level's Chebyshev smoothing interval [lam/ratio,
  * lam] (no counterpart in the reference, whose PCG preconditioner is Jacobi

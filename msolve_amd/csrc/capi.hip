@@ -145,6 +145,10 @@ struct msa_batch {
     std::vector<int4 *> mg_sm_a, mg_sm_f, mg_sm_b;  // the same split: stored-value / matrix-free
                                                    // products on general / box grids
     std::vector<int> mg_nsm_a, mg_nsm_f, mg_nsm_b;
+    // FP64 box grids of equal cells: runs of chunks for the matrix-free
+    // kernel, and chunks for the stored values (full image selected)
+    std::vector<int4 *> mg_sm_d, mg_sm_ds;
+    std::vector<int> mg_nsm_d, mg_nsm_ds;
     // box grids whose products can run on the matrix cores: their items for
     // the MFMA kernel (class, sample, y block) and for the VALU box kernel
     std::vector<int4 *> mg_sm_m, mg_sm_e;
@@ -1320,7 +1324,7 @@ int mg_build(msa_batch *b, int max_levels)
     }
     for (auto &L : b->lv) {
         ClassHost &P = tab(b, L.dev.mg_fine);
-        if (L.dev.mf && P.dev.mf && L.dev.mf_box && P.dev.mf_box && all_free(L.mesh->h) &&
+        if ((L.dev.mf || L.dev.mf64) && (P.dev.mf || P.dev.mf64) && L.dev.mf_box && P.dev.mf_box && all_free(L.mesh->h) &&
             all_free(P.mesh->h)) {
             L.dev.mg_rstruct = 1;
             P.dev.mg_pstruct = 1;
@@ -1339,11 +1343,15 @@ int mg_build(msa_batch *b, int max_levels)
     b->mg_sm_e.assign(b->mg_depth, nullptr);
     b->mg_nsm_e.assign(b->mg_depth, 0);
     b->mg_nsm_f.assign(b->mg_depth, 0);
+    b->mg_sm_d.assign(b->mg_depth, nullptr);
+    b->mg_nsm_d.assign(b->mg_depth, 0);
+    b->mg_sm_ds.assign(b->mg_depth, nullptr);
+    b->mg_nsm_ds.assign(b->mg_depth, 0);
     b->mg_restr.assign(b->mg_depth + 1, nullptr);
     b->mg_nrestr.assign(b->mg_depth + 1, 0);
     std::vector<int4> all, co;
     for (int d = 0; d <= b->mg_depth; d++) {
-        std::vector<int4> sm, sma, smf, smb, smm, sme, re;
+        std::vector<int4> sm, sma, smf, smb, smm, sme, smd, smds, re;
         for (int ci : depth_classes[d]) {
             ClassHost &C = tab(b, ci);
             if (d > 0) {
@@ -1352,7 +1360,10 @@ int mg_build(msa_batch *b, int max_levels)
             }
             if (C.dev.mg_coarse >= 0) {
                 class_items(C, ci, sm);
-                if (mfma_ok(b, C)) {
+                if (C.dev.mf64) {
+                    class_run_items(C, ci, smd);
+                    class_items(C, ci, smds);
+                } else if (mfma_ok(b, C)) {
                     mfma_items(C, ci, smm);
                     class_run_items(C, ci, sme);
                 } else if (C.dev.mf && C.dev.mf_box && b->T == 1) {
@@ -1371,6 +1382,8 @@ int mg_build(msa_batch *b, int max_levels)
             MSA_TRY(items_to_device(b, smb, &b->mg_sm_b[d], &b->mg_nsm_b[d]));
             MSA_TRY(items_to_device(b, smm, &b->mg_sm_m[d], &b->mg_nsm_m[d]));
             MSA_TRY(items_to_device(b, sme, &b->mg_sm_e[d], &b->mg_nsm_e[d]));
+            MSA_TRY(items_to_device(b, smd, &b->mg_sm_d[d], &b->mg_nsm_d[d]));
+            MSA_TRY(items_to_device(b, smds, &b->mg_sm_ds[d], &b->mg_nsm_ds[d]));
         }
         if (d > 0) MSA_TRY(items_to_device(b, re, &b->mg_restr[d], &b->mg_nrestr[d]));
     }
@@ -1448,7 +1461,7 @@ int mg_values(msa_batch *b)
     }
     MSA_TRY(assemble_items(b, b->mg_lv_items, b->mg_nlv_items, b->mg_lv_gitems, b->mg_nlv_gitems));
     for (int ci = 0; ci < nc + (int)b->lv.size(); ci++)
-        if (tab(b, ci).dev.mf)
+        if (tab(b, ci).dev.mf || tab(b, ci).dev.mf64)
             MSA_TRY(timed(b, KK_OTHER, [&] { return launch_mf_khat(s, b->d_cls + ci); }));
     MSA_TRY(timed(b, KK_OTHER, [&] {
         return launch_dinv(s, mx, T, b->d_cls, b->mg_lv_items, b->mg_nlv_items);
@@ -1614,6 +1627,14 @@ int mg_smooth_level(msa_batch *b, int d, int step, int pbuf, int mode)
         MSA_TRY(timed(b, d == 0 ? KK_MG : KK_OTHER, [&] {
             return launch_mg_smooth(s, mx, T, b->d_cls, b->mg_sm_a[d], b->mg_nsm_a[d], step, pbuf,
                                     mode, ratio, 0);
+        }));
+    if (b->mg_nsm_d[d] > 0)
+        MSA_TRY(timed(b, d == 0 ? KK_MG : KK_OTHER, [&] {
+            return b->full_storage
+                       ? launch_mg_smooth(s, mx, T, b->d_cls, b->mg_sm_ds[d], b->mg_nsm_ds[d], step,
+                                          pbuf, mode, ratio, 0)
+                       : launch_mg_smooth(s, mx, T, b->d_cls, b->mg_sm_d[d], b->mg_nsm_d[d], step,
+                                          pbuf, mode, ratio, b->dyn ? 4 : 3);
         }));
     if (b->mg_nsm_f[d] > 0)
         MSA_TRY(timed(b, d == 0 ? KK_MG : KK_OTHER, [&] {
@@ -3329,6 +3350,7 @@ int msa_batch_set_symmetric_product(msa_batch *b, int enable)
         // leftovers are never read)
         b->assembled = false;
         b->mg_ready = false;
+        drop_graph(b);  // captured blocks hold the smoothing product's form
         MSA_TRY(upload_class_table(b));
     }
     return MSA_OK;

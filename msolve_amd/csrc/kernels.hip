@@ -3838,7 +3838,16 @@ __global__ __launch_bounds__(256) void k_mg_smooth(const ClassDev *__restrict__ 
                 const int W = sptr[slice + 1] - base;
                 if (!act || br >= C.nb) continue;
                 real y[3];
-                if constexpr (T == 1) {
+                if constexpr (MF >= 3) {
+                    // FP64: the row's operands after the product, whose
+                    // registers they would take
+                    double own[3];
+                    mf64_product<MF == 4>(C, (const MSA_GLOBAL double *)src,
+                                          C.E + (size_t)tile * C.n_elem, br, y, own);
+                    const MgRow<real> w = mg_load1<real, STEP>(b, dinv, z, A, B, br);
+                    mg_finish1<real, STEP>(w, dst, br, y, ith, c1, c2, rz);
+                    continue;
+                } else if constexpr (T == 1) {
                     const MgRow<real> w = mg_load1<real, STEP>(b, dinv, z, A, B, br);
                     if constexpr (MF != 0)
                         mf_product<MF == 2, MF == 2>(C, (const MSA_GLOBAL float *)src,
@@ -5458,8 +5467,14 @@ static hipError_t mg_smooth_step(hipStream_t s, bool mixed, int T, const ClassDe
     if (nitems <= 0) return hipSuccess;
     const dim3 grid(xcd_grid(nitems)), block(256);
     if (mf != 0) {
-        if (!mixed || T != 1) return hipErrorInvalidValue;
-        if (mf == 2)
+        if (mixed != (mf < 3) || T != 1) return hipErrorInvalidValue;
+        if (mf == 3)
+            hipLaunchKernelGGL((k_mg_smooth<double, 1, STEP, 3>), grid, block, 0, s, d_cls, items,
+                               nitems, pbuf, mode, ratio);
+        else if (mf == 4)
+            hipLaunchKernelGGL((k_mg_smooth<double, 1, STEP, 4>), grid, block, 0, s, d_cls, items,
+                               nitems, pbuf, mode, ratio);
+        else if (mf == 2)
             hipLaunchKernelGGL((k_mg_smooth<float, 1, STEP, 2>), grid, block, 0, s, d_cls, items,
                                nitems, pbuf, mode, ratio);
         else

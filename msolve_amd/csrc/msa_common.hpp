@@ -428,7 +428,8 @@ enum MgStep { MG_PRE = 0, MG_RESID = 1, MG_POST1 = 2, MG_POST2 = 3 };
 // which samples a cycle serves: 0 every sample, 1 active, 2 due for a
 // residual replacement (ir_active && ru_due), 3 refining (ir_active)
 // mf: 0 stored values; the items' classes use the matrix-free product
-// (mixed, T = 1) on general uniform grids (1) or on box grids (2)
+// (T = 1): mixed on general uniform grids (1) or on box grids (2), FP64 on
+// box grids, static (3) or dynamic (4)
 hipError_t launch_mg_smooth(hipStream_t s, bool mixed, int T, const ClassDev *d_cls,
                             const int4 *items, int nitems, int step, int pbuf, int mode,
                             double ratio, int mf);

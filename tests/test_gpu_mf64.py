@@ -164,3 +164,36 @@ def test_newmark_step_forms(ctx, grid, beta, precision):
         d = [rel(x, y) for x, y in zip(a, c)]
         print(f"\n[case] newmark {grid} beta={beta} precision={precision}: {d}", flush=True)
         assert d[0] < 1e-8 and d[1] < 1e-8 and d[2] < 1e-6 and d[3] < 1e-6
+
+
+@pytest.mark.parametrize("dyn", [False, True])
+@pytest.mark.parametrize("grid", [dict(shape=(8, 6, 4)), dict(shape=(72, 4, 4), lengths=[8.0, 2.0, 2.0]),
+                                  dict(shape=(8, 4, 12), roller=True)])
+def test_fp64_cycle_forms(ctx, grid, dyn):
+    """One FP64 V-cycle with matrix-free smoothing products against the
+    stored values (full image selected): the same sums in another order, a
+    few hundred rounding errors through the levels."""
+    xyz, conn, dof, nf, f = block(**grid)
+    E = 2.1e5 * np.exp(0.3 * np.random.default_rng(6).standard_normal((2, conn.shape[0])))
+    mesh = msa.Mesh(ctx, xyz, conn, dof, nf)
+    b = msa.Batch(ctx, [mesh], [2], L.MSA_FP64, 1)
+    b.set_preconditioner(msa.MSA_PRECOND_MULTIGRID)
+    assert b.mg_info(0)["levels"] >= 1
+    b.set_modulus(0, E)
+    b.set_rhs(0, f)
+    if dyn:
+        b.set_dynamics(1e-2, 0.5, 1e-3, 0.25, 0.5, 1e-2)
+    r = np.random.default_rng(7).standard_normal(nf)
+    z = []
+    for sym in (True, False, True):
+        b.set_symmetric_product(sym)
+        b.assemble(0.3)
+        b.solve(tol=1e-8, max_it=200, graph_iters=4)
+        assert (b.stats(0)["status"] == msa.MSA_OK).all()
+        z.append([b.mg_apply(0, s, r) for s in range(2)])
+    for s in range(2):
+        assert np.array_equal(z[0][s], z[2][s])
+        print(f"\n[case] cycle {grid} dyn={dyn}: {rel(z[0][s], z[1][s]):.2e}", flush=True)
+        assert rel(z[0][s], z[1][s]) < 1e-11
+    b.close()
+    mesh.close()
