@@ -1175,7 +1175,7 @@ int mf_setup(msa_batch *b, ClassHost &C)
     MSA_TRY(upload_vec(b, g.cell_elem, &D.mf_cell));
     MSA_TRY(upload_vec(b, g.bpos, &D.mf_bpos));
     void *p = nullptr;
-    MSA_TRY(dalloc(b, &p, 640 * sizeof(float)));
+    MSA_TRY(dalloc(b, &p, kMfK * sizeof(float)));
     D.mf_k = (float *)p;
     MSA_TRY(dalloc(b, &p, kMfK64 * sizeof(double)));
     D.mf_k64 = (double *)p;

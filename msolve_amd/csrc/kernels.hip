@@ -1154,7 +1154,7 @@ __device__ __forceinline__ real pcg_a_sym_rows(const ClassDev &C, int s0, int s1
 
 // The matrix-free product of a uniform-grid class (defined with the
 // smoothing kernels below).
-template <bool BOX, bool PG = false>
+template <bool BOX>
 __device__ __forceinline__ void mf_product(const ClassDev &C, const MSA_GLOBAL float *v,
                                            const double *Es, int br, float &y0, float &y1,
                                            float &y2, float *pown = nullptr);
@@ -1350,7 +1350,7 @@ __global__ __launch_bounds__(256) void k_pcg_a_mf(const ClassDev *__restrict__ c
                 const int br = slice * 64 + lane;
                 if (br >= C.nb) continue;
                 float y[3], own[3];
-                mf_product<true, true>(C, p, Es, br, y[0], y[1], y[2], own);
+                mf_product<true>(C, p, Es, br, y[0], y[1], y[2], own);
                 // a constrained component's row is zero in K (as in the
                 // stored product); classes of fully free blocks have none
                 if (!__builtin_amdgcn_readfirstlane(C.mf_allfree)) {
@@ -3081,6 +3081,28 @@ __device__ __forceinline__ void mf_mass(cfloat *mh, const float (&xv)[27][3], co
     }
 }
 
+// Entry (p, q) of the unit element matrix of an axis-aligned cell between its
+// corners a (row) and o, from the 16 distinct values of input component q:
+// with d = a xor o and s = the corner's sign per axis, Khat_qq depends on d
+// only (values 0..7), and Khat_pq = s_p(a) s_q(a) c m(d_r) (lambda sigma(d_q)
+// + mu sigma(d_p)), r the third axis, sigma(0) = 1, sigma(1) = -1: up to the
+// sign one of the values 8 + (p = q + 1 ? 0 : 4) + 2 [d_p != d_q] + d_r (the
+// quadrature is a product rule, so the factors separate for any cell
+// lengths).  All indices are compile-time constants: 16 scalar values per
+// component serve its 168 products, where the full matrix took 24 scalar
+// loads of 48 registers per row.
+struct MfEntry {
+    int idx, neg;
+};
+__device__ __forceinline__ constexpr MfEntry mf_entry(int a, int o, int p, int q)
+{
+    const int d = a ^ o;
+    if (p == q) return {d, 0};
+    const int r = 3 - p - q, dp = (d >> p) & 1, dq = (d >> q) & 1;
+    const int minus = (((a >> p) & 1) ^ ((a >> q) & 1)) ^ dq;
+    return {8 + (p == (q + 1) % 3 ? 0 : 4) + 2 * (dp ^ dq) + ((d >> r) & 1), minus};
+}
+
 // y = K v for block row br of a uniform structured grid class, from the
 // moduli of the (up to) 8 cells around the node and the shared unit element
 // matrix (FP32, stored in corner order): y = sum_cells cK E_c Khat[a][b] v_b
@@ -3101,15 +3123,13 @@ __device__ __forceinline__ void mf_mass(cfloat *mh, const float (&xv)[27][3], co
 // forms would share one scalar-register budget for their element-matrix
 // loads.
 //
-// PG (box grids): the PCG product K p, summed over the corners'
-// differences from the node's value (below); pown receives the node's own
-// value of v.
-template <bool BOX, bool PG>
+// Box grids sum over the corners' differences from the node's value
+// (below); pown receives the node's own value of v.
+template <bool BOX>
 __device__ __forceinline__ void mf_product(const ClassDev &C, const MSA_GLOBAL float *v,
                                            const double *Es, int br, float &y0, float &y1,
                                            float &y2, float *pown)
 {
-    static_assert(BOX || !PG, "the difference form is a box-grid form");
     const int g = gbl(C.mf_bpos)[br];
     const int i = g & 1023, j = (g >> 10) & 1023, k = g >> 20;
     const int nx = __builtin_amdgcn_readfirstlane(C.mf_nx);
@@ -3153,12 +3173,10 @@ __device__ __forceinline__ void mf_product(const ClassDev &C, const MSA_GLOBAL f
             x0[m][1] = w.y;
             x0[m][2] = w.z;
         }
-        if constexpr (PG) {
-            if (pown) {
-                pown[0] = x0[4][0];
-                pown[1] = x0[4][1];
-                pown[2] = x0[4][2];
-            }
+        if (pown) {
+            pown[0] = x0[4][0];
+            pown[1] = x0[4][1];
+            pown[2] = x0[4][2];
         }
         // lane 0: the column at x - 1, lane 63: at x + 1 (zeros past the
         // box ends; other lanes take them from their neighbours)
@@ -3179,72 +3197,69 @@ __device__ __forceinline__ void mf_product(const ClassDev &C, const MSA_GLOBAL f
         mf_moduli(C, Es, i, j, k, nx, ny, lo, hi, cK, Ec, cw);
         // x - 1 and x + 1 parts count where the neighbour is in the box
         const float fm = blo[0] ? 1.f : 0.f, fp = bhi[0] ? 1.f : 0.f;
-        // column values: dx = 0 own, dx = -1 / +1 from lane l - 1 / l + 1
-        // (lanes 0 / 63: their own loads), times fm / fp
-        auto col = [&](int m, int dx, int p) -> float {
-            if (dx == 1) return x0[m][p];
-            const int o = __builtin_bit_cast(int, xf[m][p]), s = __builtin_bit_cast(int, x0[m][p]);
-            const int v = dx == 0 ? __builtin_amdgcn_update_dpp(o, s, 0x138, 0xf, 0xf, false)
-                                  : __builtin_amdgcn_update_dpp(o, s, 0x130, 0xf, 0xf, false);
-            return __builtin_bit_cast(float, v);
-        };
-        // PG: each cell's block row times the corners' differences from the
+        // Each cell's block row times the corners' differences from the
         // node's own value, Khat[a][.] (x_o - x_a), which equals Khat[a][.] x
         // since the blocks of a row sum to zero (a translation stores no
         // energy).  Smooth search directions make K p a small difference of
         // large terms; the differences are small, so the FP32 product keeps
         // the accuracy the PCG needs.  A corner outside the box counts as
-        // x_o = 0 (its difference -x_a).
-        float xn[3] = {0.f, 0.f, 0.f};
-        if constexpr (PG) {
-            xn[0] = x0[4][0];
-            xn[1] = x0[4][1];
-            xn[2] = x0[4][2];
-        }
+        // x_o = 0 (its difference -x_a).  One input component at a time:
+        // its 26 differences are formed once (the columns at x - 1 / x + 1
+        // by whole-wave DPP shifts) and its 16 matrix values sit in scalar
+        // registers (mf_entry).
 #pragma unroll
-        for (int c = 0; c < 8; c++) {
-            const int cx = c & 1, cy = (c >> 1) & 1, cz = c >> 2;
-            const int a = (1 - cx) + 2 * (1 - cy) + 4 * (1 - cz);  // the node's corner
-            const float f = cx ? fp : fm;
-            float t0[3] = {0.f, 0.f, 0.f}, ts[3] = {0.f, 0.f, 0.f};
+        for (int q = 0; q < 3; q++) {
+            cfloat *ks = kh + kMfKS + 16 * q;
+            float kv[16];
 #pragma unroll
-            for (int o = 0; o < 8; o++) {
-                if (PG && o == a) continue;  // the node itself: difference 0
-                const int ox = o & 1, oy = (o >> 1) & 1, oz = o >> 2;
-                const int m = (cy + oy) + 3 * (cz + oz);
-                cfloat *kab = kh + (a * 8 + o) * 9;
-                const int dx = cx + ox;  // 0: x - 1, 1: own column, 2: x + 1
-                float xb[3];
+            for (int e = 0; e < 16; e++) kv[e] = ks[e];
+            const float xn = x0[4][q];
+            float xc[9], xm[9], xp[9];
 #pragma unroll
-                for (int q = 0; q < 3; q++) {
-                    const float v = col(m, dx, q);
-                    xb[q] = !PG ? v : (dx == 1 ? v - xn[q] : __builtin_fmaf(f, v, -xn[q]));
-                }
-                float(&tt)[3] = (PG || dx == 1) ? t0 : ts;
-#pragma unroll
-                for (int p = 0; p < 3; p++) {
-                    tt[p] = __builtin_fmaf(kab[3 * p], xb[0], tt[p]);
-                    tt[p] = __builtin_fmaf(kab[3 * p + 1], xb[1], tt[p]);
-                    tt[p] = __builtin_fmaf(kab[3 * p + 2], xb[2], tt[p]);
-                }
+            for (int m = 0; m < 9; m++) {
+                xp[m] = __builtin_fmaf(fp, dpp_wave<kDppWaveShl1>(xf[m][q], x0[m][q]), -xn);
+                xm[m] = __builtin_fmaf(fm, dpp_wave<kDppWaveShr1>(xf[m][q], x0[m][q]), -xn);
+                xc[m] = x0[m][q] - xn;
             }
 #pragma unroll
-            for (int p = 0; p < 3; p++)
-                acc[p] = PG ? __builtin_fmaf(Ec[c], t0[p], acc[p])
-                            : __builtin_fmaf(Ec[c], __builtin_fmaf(f, ts[p], t0[p]), acc[p]);
-            // keep each cell's 72 scalar loads next to their use
+            for (int c = 0; c < 8; c++) {
+                const int cx = c & 1, cy = (c >> 1) & 1, cz = c >> 2;
+                const int a = (1 - cx) + 2 * (1 - cy) + 4 * (1 - cz);  // the node's corner
+                float t[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+                for (int o = 0; o < 8; o++) {
+                    if (o == a) continue;  // the node itself: difference 0
+                    const int ox = o & 1, oy = (o >> 1) & 1, oz = o >> 2;
+                    const int m = (cy + oy) + 3 * (cz + oz), dx = cx + ox;
+                    const float d = dx == 0 ? xm[m] : (dx == 1 ? xc[m] : xp[m]);
+#pragma unroll
+                    for (int p = 0; p < 3; p++) {
+                        const MfEntry e = mf_entry(a, o, p, q);
+                        t[p] = __builtin_fmaf(e.neg ? -kv[e.idx] : kv[e.idx], d, t[p]);
+                    }
+                }
+#pragma unroll
+                for (int p = 0; p < 3; p++) acc[p] = __builtin_fmaf(Ec[c], t[p], acc[p]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (cM != 0.f) {
+                // consistent mass as a product of 1-D masses (k_dyn_rhs_mf):
+                // m0, then the axis ratios
+                cfloat *mr = kh + kMfKS + 48;
+                const float wx = (lo[0] ? 1.f : 0.f) + (hi[0] ? 1.f : 0.f);
+                const float wy = (lo[1] ? 1.f : 0.f) + (hi[1] ? 1.f : 0.f);
+                const float wz = (lo[2] ? 1.f : 0.f) + (hi[2] ? 1.f : 0.f);
+                float g[9], pl[3];
+#pragma unroll
+                for (int m = 0; m < 9; m++)
+                    g[m] = __builtin_fmaf(mr[1], (xm[m] + xn) + (xp[m] + xn), wx * (xc[m] + xn));
+#pragma unroll
+                for (int z = 0; z < 3; z++)
+                    pl[z] = __builtin_fmaf(mr[2], g[3 * z] + g[3 * z + 2], wy * g[3 * z + 1]);
+                const float ms = __builtin_fmaf(mr[3], pl[0] + pl[2], wz * pl[1]);
+                acc[q] = __builtin_fmaf(cM * mr[0], ms, acc[q]);
+            }
             __builtin_amdgcn_sched_barrier(0);
-        }
-        if (cM != 0.f) {
-            float xs[27][3];  // (dx, dy, dz), x fastest
-#pragma unroll
-            for (int m = 0; m < 9; m++)
-#pragma unroll
-                for (int dx = 0; dx < 3; dx++)
-#pragma unroll
-                    for (int p = 0; p < 3; p++)
-                        xs[m * 3 + dx][p] = col(m, dx, p) * (dx == 0 ? fm : (dx == 2 ? fp : 1.f));
-            mf_mass(kh + 576, xs, cw, cM, acc);
         }
         y0 = acc[0];
         y1 = acc[1];
@@ -3331,7 +3346,14 @@ __global__ void k_mf_khat(const ClassDev *__restrict__ cp)
         int o = e;  // corner of the entry
         if (e >= 8) o = (e & 2 ? 1 << p : 0) | (e & 1 ? 1 << (3 - p - q) : 0);
         const int a = C.mf_corner[0], b = C.mf_corner[o];
-        C.mf_k64[kMfK64S + i] = C.kc[(a * 8 + b) * 9 + 3 * p + q];
+        const double k = C.kc[(a * 8 + b) * 9 + 3 * p + q];
+        C.mf_k64[kMfK64S + i] = k;
+        C.mf_k[kMfKS + i] = (float)k;
+    } else if (i < 52) {
+        // the consistent mass: M[0][0] and its ratios along the axes
+        const int e = i - 48, a = C.mf_corner[0], b = e ? C.mf_corner[1 << (e - 1)] : a;
+        const double m0 = C.mc ? C.mc[a * 8 + a] : 0.0;
+        C.mf_k[kMfKS + i] = (float)(e == 0 ? m0 : (m0 != 0.0 ? C.mc[a * 8 + b] / m0 : 0.0));
     }
 }
 
@@ -3438,28 +3460,6 @@ __device__ __forceinline__ cdouble *mf_khat64(const ClassDev &C)
     unsigned long long kp = (unsigned long long)C.mf_k64;
     asm volatile("" : "+s"(kp));
     return (cdouble *)kp;
-}
-
-// Entry (p, q) of the unit element matrix of an axis-aligned cell between its
-// corners a (row) and o, from the 16 distinct values of input component q:
-// with d = a xor o and s = the corner's sign per axis, Khat_qq depends on d
-// only (values 0..7), and Khat_pq = s_p(a) s_q(a) c m(d_r) (lambda sigma(d_q)
-// + mu sigma(d_p)), r the third axis, sigma(0) = 1, sigma(1) = -1: up to the
-// sign one of the values 8 + (p = q + 1 ? 0 : 4) + 2 [d_p != d_q] + d_r (the
-// quadrature is a product rule, so the factors separate for any cell
-// lengths).  All indices are compile-time constants: 16 scalar values per
-// component serve its 168 products, where the full matrix took 24 scalar
-// loads of 48 registers per row.
-struct MfEntry {
-    int idx, neg;
-};
-__device__ __forceinline__ constexpr MfEntry mf_entry(int a, int o, int p, int q)
-{
-    const int d = a ^ o;
-    if (p == q) return {d, 0};
-    const int r = 3 - p - q, dp = (d >> p) & 1, dq = (d >> q) & 1;
-    const int minus = (((a >> p) & 1) ^ ((a >> q) & 1)) ^ dq;
-    return {8 + (p == (q + 1) % 3 ? 0 : 4) + 2 * (dp ^ dq) + ((d >> r) & 1), minus};
 }
 
 // y = K v for block row br of a box-grid class (one-sample tiles) in FP64,
@@ -3850,7 +3850,7 @@ __global__ __launch_bounds__(256) void k_mg_smooth(const ClassDev *__restrict__ 
                 } else if constexpr (T == 1) {
                     const MgRow<real> w = mg_load1<real, STEP>(b, dinv, z, A, B, br);
                     if constexpr (MF != 0)
-                        mf_product<MF == 2, MF == 2>(C, (const MSA_GLOBAL float *)src,
+                        mf_product<MF == 2>(C, (const MSA_GLOBAL float *)src,
                                                      C.E + (size_t)tile * C.n_elem, br, y[0],
                                                      y[1], y[2]);
                     else

@@ -141,6 +141,10 @@ int grid_info(const MeshHost &m, GridInfo &g);
 // then Khat's distinct values by input component (kMfK64S, 16 each;
 // mf64_product)
 constexpr int kMfK64S = 640;
+// FP32: Khat (576) + Mhat (64), the distinct values (kMfKS, 48), the mass
+// M[0][0] and its ratios along the axes (4)
+constexpr int kMfKS = 640;
+constexpr int kMfK = 640 + 52;
 constexpr int kMfK64 = 640 + 48;
 
 struct ClassDev {
