@@ -99,8 +99,8 @@ def ke_packed(ctx: Context, xyz8, E, nu: float):
     x = f64(xyz8).reshape(-1, 24)
     E = f64(E).ravel()
     n = x.shape[0]
-    ke = np.zeros((n, 300))
-    st = np.zeros(n, np.int32)
+    ke = np.empty((n, 300))  # the call writes every entry
+    st = np.empty(n, np.int32)
     check(lib().msa_ke_packed(ctx.h, n, ptr(x, C.c_double), ptr(E, C.c_double), nu,
                               ptr(ke, C.c_double), ptr(st, C.c_int)))
     return ke, st
@@ -168,7 +168,7 @@ class Batch:
         check(lib().msa_batch_run(self.h, nu, tol, max_it, inner_tol, max_outer, graph_iters))
 
     def solution(self, cls: int, sample: int):
-        u = np.zeros(self.meshes[cls].n_free)
+        u = np.empty(self.meshes[cls].n_free)
         check(lib().msa_batch_get_solution(self.h, cls, sample, ptr(u, C.c_double)))
         return u
 
@@ -187,13 +187,13 @@ class Batch:
         [n_elem, 24] of one solved sample (Hexa8.CalculateStresses /
         CalculateForces)."""
         ne = self.meshes[cls].n_elem
-        eps, sig, f = np.zeros((ne, 8, 6)), np.zeros((ne, 8, 6)), np.zeros((ne, 24))
+        eps, sig, f = np.empty((ne, 8, 6)), np.empty((ne, 8, 6)), np.empty((ne, 24))
         check(lib().msa_batch_element_results(self.h, cls, sample, ptr(eps, C.c_double),
                                               ptr(sig, C.c_double), ptr(f, C.c_double)))
         return eps, sig, f
 
     def modulus(self, cls: int, sample: int):
-        E = np.zeros(self.meshes[cls].n_elem)
+        E = np.empty(self.meshes[cls].n_elem)
         check(lib().msa_batch_get_modulus(self.h, cls, sample, ptr(E, C.c_double)))
         return E
 
@@ -348,7 +348,7 @@ class Batch:
 
     def dynamic_state(self, cls: int, sample: int):
         n = self.meshes[cls].n_free
-        u, v, a = np.zeros(n), np.zeros(n), np.zeros(n)
+        u, v, a = np.empty(n), np.empty(n), np.empty(n)
         it = C.c_longlong()
         check(lib().msa_batch_get_dynamic_state(self.h, cls, sample, ptr(u, C.c_double),
                                                 ptr(v, C.c_double), ptr(a, C.c_double),

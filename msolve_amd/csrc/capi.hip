@@ -1756,6 +1756,45 @@ int mg_vcycle(msa_batch *b, int pbuf, int mode)
 
 }  // namespace
 
+// Device scratch of one call: the context's, or memory of its own when the call
+// needs more than kCtxScratchMax or another thread holds the context's.  Every
+// user waits for its stream before it lets go; an error return leaves at most
+// work of the same stream behind, which orders the next user after it.
+struct CtxScratch {
+    msa_ctx *c;
+    void *p = nullptr;
+    bool held = false, own = false;
+    explicit CtxScratch(msa_ctx *ctx) : c(ctx) {}
+    CtxScratch(const CtxScratch &) = delete;
+    CtxScratch &operator=(const CtxScratch &) = delete;
+    hipError_t get(size_t bytes)
+    {
+        bytes = std::max<size_t>(bytes, 256);
+        held = bytes <= kCtxScratchMax && c->scratch_mutex.try_lock();
+        if (!held) {
+            hipError_t e = hipMalloc(&p, bytes);
+            own = e == hipSuccess;
+            return e;
+        }
+        if (c->scratch_cap < bytes) {
+            if (c->scratch) (void)hipFree(c->scratch);
+            c->scratch = nullptr;
+            c->scratch_cap = 0;
+            const size_t cap = (bytes + ((size_t)1 << 20) - 1) >> 20 << 20;
+            hipError_t e = hipMalloc(&c->scratch, cap);
+            if (e != hipSuccess) return e;
+            c->scratch_cap = cap;
+        }
+        p = c->scratch;
+        return hipSuccess;
+    }
+    ~CtxScratch()
+    {
+        if (own) (void)hipFree(p);
+        if (held) c->scratch_mutex.unlock();
+    }
+};
+
 extern "C" {
 
 const char *msa_last_error(void) { return g_last_error.c_str(); }
@@ -1797,6 +1836,7 @@ int msa_ctx_destroy(msa_ctx *ctx)
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
     if (ctx->h_pinned) (void)hipHostFree(ctx->h_pinned);
+    if (ctx->scratch) (void)hipFree(ctx->scratch);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return MSA_OK;
@@ -1880,13 +1920,12 @@ int msa_ke_packed(msa_ctx *ctx, int n_elem, const double *xyz8, const double *E,
     MSA_CHECK(ctx && xyz8 && E && ke300 && n_elem >= 0, MSA_ERR_ARG, "msa_ke_packed: bad args");
     if (n_elem == 0) return MSA_OK;
     MSA_HIP(hipSetDevice(ctx->device));
-    double *dx = nullptr, *dE = nullptr, *dk = nullptr;
-    int *ds = nullptr;
     hipStream_t s = ctx->stream;
-    hipError_t e = hipMalloc(&dx, sizeof(double) * 24 * (size_t)n_elem);
-    if (e == hipSuccess) e = hipMalloc(&dE, sizeof(double) * (size_t)n_elem);
-    if (e == hipSuccess) e = hipMalloc(&dk, sizeof(double) * 300 * (size_t)n_elem);
-    if (e == hipSuccess) e = hipMalloc(&ds, sizeof(int) * (size_t)n_elem);
+    const size_t ne = (size_t)n_elem;
+    CtxScratch w(ctx);
+    hipError_t e = w.get(ne * (325 * sizeof(double) + sizeof(int)));
+    double *dk = (double *)w.p, *dx = dk + 300 * ne, *dE = dx + 24 * ne;
+    int *ds = (int *)(dE + ne);
     if (e == hipSuccess)
         e = hipMemcpyAsync(dx, xyz8, sizeof(double) * 24 * (size_t)n_elem, hipMemcpyHostToDevice, s);
     if (e == hipSuccess)
@@ -1897,8 +1936,6 @@ int msa_ke_packed(msa_ctx *ctx, int n_elem, const double *xyz8, const double *E,
     if (e == hipSuccess && elem_status)
         e = hipMemcpyAsync(elem_status, ds, sizeof(int) * (size_t)n_elem, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
-    for (void *p : {(void *)dx, (void *)dE, (void *)dk, (void *)ds})
-        if (p) (void)hipFree(p);
     if (e != hipSuccess) {
         set_error("msa_ke_packed: %s", hipGetErrorString(e));
         return MSA_ERR_HIP;
@@ -2420,18 +2457,39 @@ int msa_batch_run(msa_batch *b, double nu, double tol, int max_it, double inner_
     return msa_batch_solve(b, tol, max_it, inner_tol, max_outer, graph_iters);
 }
 
+// One sample's n values of a lane-tiled array, into host memory.  One-sample
+// tiles hold them contiguously: the copy reads the array itself; wider tiles
+// (and FP32 values, which are widened) go through an extraction kernel.
 static int extract_lane(msa_batch *b, bool real_is_float, const void *tile_base, size_t n, int lane,
-                        std::vector<double> &host)
+                        double *host)
 {
-    double *d = nullptr;
-    MSA_HIP(hipMalloc(&d, std::max<size_t>(n, 1) * sizeof(double)));
-    host.resize(n);
-    hipError_t e = launch_extract_sample(b->ctx->stream, real_is_float, b->T, tile_base, n, lane, d);
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(host.data(), d, n * sizeof(double), hipMemcpyDeviceToHost, b->ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(b->ctx->stream);
-    (void)hipFree(d);
-    MSA_HIP(e);
+    if (!n) return MSA_OK;
+    hipStream_t s = b->ctx->stream;
+    CtxScratch w(b->ctx);
+    const void *src = tile_base;
+    if (b->T != 1 || real_is_float) {
+        MSA_HIP(w.get(n * sizeof(double)));
+        MSA_HIP(launch_extract_sample(s, real_is_float, b->T, tile_base, n, lane, (double *)w.p));
+        src = w.p;
+    }
+    MSA_HIP(hipMemcpyAsync(host, src, n * sizeof(double), hipMemcpyDeviceToHost, s));
+    MSA_HIP(hipStreamSynchronize(s));
+    return MSA_OK;
+}
+
+// One sample's DOF vector, in the caller's numbering.  Meshes whose nodes are
+// either entirely free or entirely fixed and numbered in node order (every
+// enumerate_dofs numbering of such supports) share the internal order, and the
+// copy lands in the caller's array.  1024 vectors of 16^3 to 48^3 meshes
+// (1.16 GB) took about 150 ms with a device buffer, a host vector and the
+// permutation per call and take 75 ms so, the pageable copy's own rate.
+static int extract_dofs(msa_batch *b, const MeshHost &m, const double *tile_base, int lane, double *u)
+{
+    const size_t n = (size_t)m.nb * 3;
+    if (m.ref_identity) return extract_lane(b, false, tile_base, n, lane, u);
+    std::vector<double> h(n);
+    MSA_TRY(extract_lane(b, false, tile_base, n, lane, h.data()));
+    for (int g = 0; g < m.n_free; g++) u[g] = h[m.ref2int[g]];
     return MSA_OK;
 }
 
@@ -2442,15 +2500,8 @@ int msa_batch_get_solution(msa_batch *b, int cls, int sample, double *u)
     MSA_CHECK(sample >= 0 && sample < C.nsamp, MSA_ERR_ARG, "sample %d out of range", sample);
     MSA_HIP(hipSetDevice(b->ctx->device));
     const int tile = sample / b->T, lane = sample % b->T;
-    std::vector<double> h;
-    const size_t n = (size_t)C.mesh->h.nb * 3;
-    if (is_mixed(b))
-        MSA_TRY(extract_lane(b, false, C.dev.u64 + (size_t)tile * C.tile_vec, n, lane, h));
-    else
-        MSA_TRY(extract_lane(b, false, (double *)C.dev.x + (size_t)tile * C.tile_vec, n, lane, h));
-    const MeshHost &m = C.mesh->h;
-    for (int g = 0; g < m.n_free; g++) u[g] = h[m.ref2int[g]];
-    return MSA_OK;
+    const double *x = is_mixed(b) ? C.dev.u64 : (const double *)C.dev.x;
+    return extract_dofs(b, C.mesh->h, x + (size_t)tile * C.tile_vec, lane, u);
 }
 
 // ---------------------------------------------------------------- dynamics
@@ -3020,16 +3071,13 @@ int msa_batch_get_dynamic_state(msa_batch *b, int cls, int sample, double *u, do
     MSA_CHECK(sample >= 0 && sample < C.nsamp, MSA_ERR_ARG, "sample %d out of range", sample);
     MSA_HIP(hipSetDevice(b->ctx->device));
     const int tile = sample / b->T, lane = sample % b->T;
-    const size_t n = (size_t)C.mesh->h.nb * 3, off = (size_t)tile * C.tile_vec;
-    const MeshHost &m = C.mesh->h;
-    std::vector<double> h;
+    const size_t off = (size_t)tile * C.tile_vec;
     const double *src[3] = {is_mixed(b) ? C.dev.u64 + off : (const double *)C.dev.x + off,
                             C.dev.vel + off, C.dev.acc + off};
     double *dst[3] = {u, v, a};
     for (int k = 0; k < 3; k++) {
         if (!dst[k]) continue;
-        MSA_TRY(extract_lane(b, false, src[k], n, lane, h));
-        for (int g = 0; g < m.n_free; g++) dst[k][g] = h[m.ref2int[g]];
+        MSA_TRY(extract_dofs(b, C.mesh->h, src[k], lane, dst[k]));
     }
     if (iters) {
         SampleState st;
@@ -3052,9 +3100,9 @@ int msa_batch_element_results(msa_batch *b, int cls, int sample, double *strains
     hipStream_t s = b->ctx->stream;
     const int ne = C.mesh->h.n_elem, tile = sample / b->T, lane = sample % b->T;
     const double *u = (is_mixed(b) ? C.dev.u64 : (const double *)C.dev.x) + (size_t)tile * C.tile_vec;
-    double *d = nullptr;
-    const size_t n = (size_t)ne * 120;
-    MSA_HIP(hipMalloc(&d, n * sizeof(double)));
+    CtxScratch w(b->ctx);
+    MSA_HIP(w.get((size_t)ne * 120 * sizeof(double)));
+    double *d = (double *)w.p;
     hipError_t e = launch_element_results(s, b->T, b->d_cls + cls, ne, u, lane, tile, b->nu,
                                           strains ? d : nullptr, stresses ? d + (size_t)ne * 48 : nullptr,
                                           forces ? d + (size_t)ne * 96 : nullptr);
@@ -3067,7 +3115,6 @@ int msa_batch_element_results(msa_batch *b, int cls, int sample, double *strains
         e = hipMemcpyAsync(forces, d + (size_t)ne * 96, (size_t)ne * 24 * sizeof(double),
                            hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
-    (void)hipFree(d);
     MSA_HIP(e);
     return MSA_OK;
 }
@@ -3101,10 +3148,7 @@ int msa_batch_get_modulus(msa_batch *b, int cls, int sample, double *E)
     MSA_CHECK(sample >= 0 && sample < C.nsamp, MSA_ERR_ARG, "sample %d out of range", sample);
     MSA_HIP(hipSetDevice(b->ctx->device));
     const int tile = sample / b->T, lane = sample % b->T, ne = C.mesh->h.n_elem;
-    std::vector<double> h;
-    MSA_TRY(extract_lane(b, false, C.dev.E + (size_t)tile * ne * b->T, ne, lane, h));
-    memcpy(E, h.data(), ne * sizeof(double));
-    return MSA_OK;
+    return extract_lane(b, false, C.dev.E + (size_t)tile * ne * b->T, ne, lane, E);
 }
 
 int msa_batch_get_matrix_csr(msa_batch *b, int cls, int sample, long long *rowptr, int *col,
@@ -3118,10 +3162,10 @@ int msa_batch_get_matrix_csr(msa_batch *b, int cls, int sample, long long *rowpt
     MSA_HIP(hipSetDevice(b->ctx->device));
     const int tile = sample / b->T, lane = sample % b->T, R = b->R;
     const size_t rs = real_size(b);
-    std::vector<double> hv;
     const size_t n = (size_t)C.slice_ptr[C.nslices] * 9 * R;
+    std::vector<double> hv(n);
     MSA_TRY(extract_lane(b, is_mixed(b), (const char *)C.dev.val + (size_t)tile * C.tile_vals * rs, n,
-                         lane, hv));
+                         lane, hv.data()));
     const MeshHost &m = C.mesh->h;
     long long k = 0;
     rowptr[0] = 0;

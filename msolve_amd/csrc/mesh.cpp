@@ -65,6 +65,8 @@ int build_mesh_host(MeshHost &m, int n_nodes, const double *xyz, int n_elem,
         }
     for (int g = 0; g < n_free; g++)
         MSA_CHECK(m.ref2int[g] >= 0, MSA_ERR_ARG, "mesh: free DOF %d not assigned", g);
+    m.ref_identity = n_free == 3 * m.nb;
+    for (int g = 0; g < n_free && m.ref_identity; g++) m.ref_identity = m.ref2int[g] == g;
 
     // node -> incident elements
     std::vector<int> inc_ptr(n_nodes + 1, 0), inc;

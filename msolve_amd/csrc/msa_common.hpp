@@ -19,6 +19,7 @@
 #include <cstdint>
 #include <cstdio>
 #include <string>
+#include <mutex>
 #include <vector>
 
 #include "../../include/msolve_amd.h"
@@ -89,6 +90,7 @@ struct MeshHost {
     std::vector<uint8_t> node_free;      // [n_nodes] bit d = DOF d free
     std::vector<int> block_node;         // [nb]
     std::vector<int> ref2int;            // [n_free] -> 3*block + d
+    bool ref_identity = false;           // ref2int is the identity onto [0, 3 nb)
     std::vector<int> brow_ptr, bcol;     // block adjacency, sorted
     std::vector<int> diag_pos;           // [nb] position of the diagonal
     std::vector<uint8_t> emap;           // [n_elem*64] slot of (a,b) or 255
@@ -530,7 +532,16 @@ struct msa_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
     int *h_pinned = nullptr;  // small pinned host scratch for polling
+    // device scratch of the calls that stage through one (element matrices,
+    // element results, lane-tile read-back), handed out by CtxScratch: grown on
+    // demand up to kCtxScratchMax bytes, freed with the context
+    std::mutex scratch_mutex;
+    void *scratch = nullptr;
+    size_t scratch_cap = 0;
 };
+// a 32^3 mesh's element results are 31 MB, 24 k element matrices 60 MB; beyond
+// this the transfer is milliseconds and an allocation of its own does not show
+constexpr size_t kCtxScratchMax = (size_t)64 << 20;
 
 struct msa_mesh {
     msa_ctx *ctx = nullptr;
