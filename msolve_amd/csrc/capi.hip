@@ -90,7 +90,9 @@ struct msa_batch {
     int n_gitems = 0;
     std::vector<int2> tiles;  // (class, tile) pairs, one reduction workgroup each
     int2 *d_tiles = nullptr;
-    int *d_counts = nullptr;  // [0] PCG active samples, [1] refinement active samples
+    // [0] PCG active samples, [1] refinement active samples, [2] those of the
+    // classes with a hierarchy after the last block (launch_block)
+    int *d_counts = nullptr;
     std::vector<void *> allocs;
     long long bytes = 0;
     bool assembled = false;
@@ -122,6 +124,7 @@ struct msa_batch {
     // the caller's block and the short tail block replayed once a sample
     // has converged
     hipGraphExec_t graph = nullptr, graph_tail = nullptr;
+    hipGraphExec_t graph_flat[2] = {nullptr, nullptr};  // block, tail block without the cycle
     int graph_iters = 0, graph_tail_iters = 0, graph_kind = -1;
     double graph_tol = -1;
     int graph_maxit = -1;
@@ -455,7 +458,7 @@ int reduce(msa_batch *b, int op, double tol = 0.0, int max_it = 0, int max_outer
 
 void drop_graph(msa_batch *b)
 {
-    for (hipGraphExec_t *g : {&b->graph, &b->graph_tail})
+    for (hipGraphExec_t *g : {&b->graph, &b->graph_tail, &b->graph_flat[0], &b->graph_flat[1]})
         if (*g) {
             (void)hipGraphExecDestroy(*g);
             *g = nullptr;
@@ -484,12 +487,13 @@ int upload_class_table(msa_batch *b)
     return MSA_OK;
 }
 
-int read_count(msa_batch *b, int which, int *out)
+// `n` consecutive counters, one copy and one wait.
+int read_count(msa_batch *b, int which, int *out, int n = 1)
 {
-    MSA_HIP(hipMemcpyAsync(b->ctx->h_pinned, b->d_counts + which, sizeof(int),
+    MSA_HIP(hipMemcpyAsync(b->ctx->h_pinned, b->d_counts + which, n * sizeof(int),
                            hipMemcpyDeviceToHost, b->ctx->stream));
     MSA_HIP(hipStreamSynchronize(b->ctx->stream));
-    *out = *b->ctx->h_pinned;
+    std::copy(b->ctx->h_pinned, b->ctx->h_pinned + n, out);
     return MSA_OK;
 }
 
@@ -513,7 +517,8 @@ hipError_t launch_product(msa_batch *b, int pbuf)
 }
 
 // ru_tol > 0: reliable-update mode (inner test off, replacement triggers on).
-int launch_iteration_pair(msa_batch *b, int pbuf, double tol, int max_it, double ru_tol = 0.0)
+// cycle: with the preconditioner's own launches.
+int launch_iteration_pair(msa_batch *b, int pbuf, double tol, int max_it, double ru_tol, bool cycle)
 {
     const bool mx = is_mixed(b);
     hipStream_t s = b->ctx->stream;
@@ -523,7 +528,7 @@ int launch_iteration_pair(msa_batch *b, int pbuf, double tol, int max_it, double
         return launch_pcg_b(s, mx, b->T, b->d_cls, b->d_items, (int)b->items.size(), pbuf, tol,
                             max_it, b->d_counts);
     }));
-    MSA_TRY(mg_vcycle(b, pbuf, 1));
+    if (cycle) MSA_TRY(mg_vcycle(b, pbuf, 1));
     if (ru_tol > 0)
         MSA_TRY(reduce(b, OP_B, 0.0, max_it, 0, b->drop, ru_tol));
     else
@@ -567,7 +572,7 @@ int launch_residual_mf(msa_batch *b, int need_due)
 
 // Fold the FP32 correction into u64, form the FP64 residual, test it and
 // restart the FP32 recurrence from it (reliable-update refinement).
-int launch_replacement(msa_batch *b, double tol, int max_it)
+int launch_replacement(msa_batch *b, double tol, int max_it, bool cycle)
 {
     hipStream_t s = b->ctx->stream;
     const int T = b->T, ni = (int)b->items.size();
@@ -589,19 +594,36 @@ int launch_replacement(msa_batch *b, double tol, int max_it)
     }));
     MSA_TRY(reduce(b, OP_RUNORM, tol, max_it));
     MSA_TRY(timed(b, KK_OTHER, [&] { return launch_ru_restart(s, T, b->d_cls, b->d_items, ni); }));
-    MSA_TRY(mg_vcycle(b, 1, 2));  // the restart keeps the search direction in p0
+    if (cycle) MSA_TRY(mg_vcycle(b, 1, 2));  // the restart keeps the search direction in p0
     MSA_TRY(reduce(b, OP_RURESTART));
     return MSA_OK;
 }
 
+// Whether some classes of a multigrid batch have a hierarchy and others are
+// solved with Jacobi beside them (odd cell counts do not coarsen).
+bool part_hierarchy(const msa_batch *b)
+{
+    if (b->precond != MSA_PRECOND_MULTIGRID || b->mg_depth == 0) return false;
+    for (auto &C : b->cls)
+        if (C.dev.mg_coarse < 0) return true;
+    return false;
+}
+
 // One block of `iters` PCG iterations; kind 1 adds a residual replacement
-// after every b->period iterations (inner stopping test disabled).
-int launch_block(msa_batch *b, int kind, int iters, double tol, int max_it)
+// after every b->period iterations (inner stopping test disabled).  In a
+// batch with a partial hierarchy it ends with the count of samples that still
+// need the cycle; at zero the following blocks go without it (cycle false).
+int launch_block(msa_batch *b, int kind, int iters, double tol, int max_it, bool cycle = true)
 {
     for (int k = 0; k < iters; k++) {
-        MSA_TRY(launch_iteration_pair(b, k & 1, kind == 1 ? 0.0 : tol, max_it, kind == 1 ? tol : 0.0));
-        if (kind == 1 && (k + 1) % b->period == 0) MSA_TRY(launch_replacement(b, tol, max_it));
+        MSA_TRY(launch_iteration_pair(b, k & 1, kind == 1 ? 0.0 : tol, max_it, kind == 1 ? tol : 0.0,
+                                      cycle));
+        if (kind == 1 && (k + 1) % b->period == 0) MSA_TRY(launch_replacement(b, tol, max_it, cycle));
     }
+    if (cycle && part_hierarchy(b))
+        MSA_TRY(timed(b, KK_OTHER, [&] {
+            return launch_mg_count(b->ctx->stream, b->d_cls, (int)b->cls.size(), kind, b->d_counts + 2);
+        }));
     return MSA_OK;
 }
 
@@ -731,24 +753,41 @@ int pcg_loop(msa_batch *b, int kind, double tol, int max_it, int graph_iters)
     // in a Monte Carlo batch, and every launch of a block still dispatches
     // the tiles of the converged samples: the loop then replays the tail
     // block, which stops at most tail - 1 iterations after the last sample.
+    //
+    // In a batch with a partial hierarchy the multigrid classes are done after
+    // some tens of iterations and the Jacobi classes go on for hundreds, each
+    // with the launches of a cycle that no sample takes part in.  Once none
+    // does, the loop goes on without them, in full blocks again until one of
+    // the remaining samples has converged (17 samples over 4 meshes, 446
+    // iterations: 65 -> 37 ms).
     const int tail = tail_iters(b, kind);
+    const bool part = part_hierarchy(b);
+    bool cycle = true;
     int total = 0;
     for (auto &C : b->cls) total += C.nsamp;
     long long done = 0;
     for (;;) {
-        int active = 0;
-        MSA_TRY(read_count(b, which, &active));
+        int c[3];
+        MSA_TRY(read_count(b, 0, c, 3));
+        const int active = c[which];
         if (active <= 0) break;
         if (done > (long long)max_it + block) {
             set_error("PCG driver: samples still active after %lld iterations", done);
             return MSA_ERR_STATE;
         }
-        const int it = active < total && tail < block ? tail : block;
+        if (part && cycle && done > 0 && c[2] == 0) {
+            cycle = false;
+            total = active;
+        }
+        const bool full = active >= total || tail >= block;
+        const int it = full ? block : tail;
         if (use_graph) {
-            MSA_HIP(hipGraphLaunch(it == block ? b->graph : b->graph_tail, b->ctx->stream));
+            hipGraphExec_t *g = cycle ? full ? &b->graph : &b->graph_tail : &b->graph_flat[full ? 0 : 1];
+            if (!*g) MSA_TRY(capture(b, g, [&] { return launch_block(b, kind, it, tol, max_it, false); }));
+            MSA_HIP(hipGraphLaunch(*g, b->ctx->stream));
             b->graph_replays++;
         } else {
-            MSA_TRY(launch_block(b, kind, it, tol, max_it));
+            MSA_TRY(launch_block(b, kind, it, tol, max_it, cycle));
         }
         done += it;
     }

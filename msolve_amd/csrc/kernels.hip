@@ -1961,6 +1961,26 @@ __global__ void k_set_int(int *p, int n, int v)
     if (i < n) p[i] = v;
 }
 
+// One workgroup; a few thousand loads at most (one launch per block of
+// iterations, 3 us).
+__global__ __launch_bounds__(256) void k_mg_count(const ClassDev *__restrict__ cls, int ncls,
+                                                  int kind, int *out)
+{
+    __shared__ int sum;
+    if (threadIdx.x == 0) sum = 0;
+    __syncthreads();
+    int n = 0;
+    for (int c = 0; c < ncls; c++) {
+        const ClassDev &C = cls[c];
+        if (C.mg_coarse < 0) continue;
+        for (int k = threadIdx.x; k < C.nsamp; k += 256)
+            n += kind == 1 ? C.st[k].ir_active != 0 : C.st[k].active != 0;
+    }
+    if (n) atomicAdd(&sum, n);
+    __syncthreads();
+    if (threadIdx.x == 0) *out = sum;
+}
+
 __global__ void k_step_advance(int *step)
 {
     if (blockIdx.x == 0 && threadIdx.x == 0) *step += 1;
@@ -5347,6 +5367,12 @@ hipError_t launch_set_int(hipStream_t s, int *p, int n, int v)
 {
     if (n <= 0) return hipSuccess;
     hipLaunchKernelGGL(k_set_int, dim3((n + 255) / 256), dim3(256), 0, s, p, n, v);
+    return hipGetLastError();
+}
+
+hipError_t launch_mg_count(hipStream_t s, const ClassDev *d_cls, int ncls, int kind, int *out)
+{
+    hipLaunchKernelGGL(k_mg_count, dim3(1), dim3(256), 0, s, d_cls, ncls, kind, out);
     return hipGetLastError();
 }
 

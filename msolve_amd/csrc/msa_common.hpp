@@ -409,6 +409,9 @@ hipError_t launch_ru_restart(hipStream_t s, int T, const ClassDev *d_cls, const 
                              int nitems);
 hipError_t launch_spmv(hipStream_t s, bool mixed, int T, const ClassDev *d_cls, const int4 *items,
                        int nitems, const double *x, double *y);
+// samples of classes with a hierarchy that are still active (kind 0) or still
+// refining (kind 1)
+hipError_t launch_mg_count(hipStream_t s, const ClassDev *d_cls, int ncls, int kind, int *out);
 hipError_t launch_reduce(hipStream_t s, int T, const ClassDev *d_cls, const int2 *tiles,
                          int ntiles, const ReduceArgs &a);
 // direct solver (band Cholesky); cp = the class's device ClassDev

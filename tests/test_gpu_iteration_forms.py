@@ -1,0 +1,59 @@
+"""Forms of the PCG iteration: a multigrid batch in which one class does not
+coarsen leaves the cycle out once only that class's samples are active; every
+sample then follows the recurrence it follows in a batch of its own."""
+import numpy as np
+import pytest
+
+import msolve_amd as msa
+from msolve_amd import _lib as L
+from msolve_amd.model import box_mesh
+
+pytestmark = pytest.mark.gpu
+
+
+def solve(ctx, shapes, nsamp, precision, method, tol, **kw):
+    meshes, rng = [], np.random.default_rng(2)
+    data = {}
+    for k, sh in enumerate([(8, 8, 8), (7, 5, 9)]):
+        xyz, conn = box_mesh(*sh, *[float(v) for v in sh])
+        cons = np.zeros((xyz.shape[0], 3), bool)
+        cons[xyz[:, 2] < 1e-12] = True
+        dof, nf = msa.enumerate_dofs(cons)
+        data[sh] = (xyz, conn, dof, nf, rng.standard_normal(nf),
+                    rng.uniform(1.0, 3.0, (nsamp[k], conn.shape[0])))
+    for sh in shapes:
+        meshes.append(msa.Mesh(ctx, *data[sh][:4]))
+    b = msa.Batch(ctx, meshes, [data[sh][5].shape[0] for sh in shapes], precision, 1)
+    b.set_preconditioner(L.MSA_PRECOND_MULTIGRID)
+    if precision == L.MSA_MIXED:
+        b.set_refinement(method)
+    for c, sh in enumerate(shapes):
+        b.set_modulus(c, data[sh][5])
+        b.set_rhs(c, data[sh][4])
+    b.assemble(0.3)
+    b.solve(tol=tol, max_it=5000, **kw)
+    out = {}
+    for c, sh in enumerate(shapes):
+        st = b.stats(c)
+        assert (st["status"] == msa.MSA_OK).all()
+        out[sh] = (st["iters"], [b.solution(c, s) for s in range(len(st["iters"]))])
+    replays = b.graph_info()["replays"]
+    b.close()
+    for m in meshes:
+        m.close()
+    return out, replays
+
+
+@pytest.mark.parametrize("graph_iters", [0, 2, 12])
+@pytest.mark.parametrize("precision,method", [(L.MSA_FP64, 0), (L.MSA_MIXED, L.MSA_REFINE_RELIABLE),
+                                              (L.MSA_MIXED, L.MSA_REFINE_RESTART)])
+def test_partial_hierarchy_equals_separate_batches(ctx, precision, method, graph_iters):
+    cube, odd = (8, 8, 8), (7, 5, 9)
+    kw = dict(nsamp=(3, 2), precision=precision, method=method, tol=1e-10, graph_iters=graph_iters)
+    both, _ = solve(ctx, [cube, odd], **kw)
+    for sh in (cube, odd):
+        alone, _ = solve(ctx, [sh], **kw)
+        assert np.array_equal(both[sh][0], alone[sh][0])
+        for u, v in zip(both[sh][1], alone[sh][1]):
+            assert np.array_equal(u, v)
+    assert both[odd][0].min() > 2 * both[cube][0].max()  # the cycle was left out for a while
