@@ -400,6 +400,7 @@ int setup_class(msa_batch *b, ClassHost &C, msa_mesh *mesh, int nsamp)
         D.f = (const double *)p;
         A((void **)&D.E, (size_t)C.ntiles * h.n_elem * T * sizeof(double));
         A((void **)&D.st, (size_t)C.ntiles * T * sizeof(SampleState));
+        A((void **)&D.st_b, (size_t)C.ntiles * T * sizeof(SampleState));
         A((void **)&D.partial, (size_t)C.ntiles * C.nchunks * 3 * T * sizeof(double));
         A((void **)&D.negdet, sizeof(int));
         A((void **)&D.due, (1 + (size_t)C.ntiles * T) * sizeof(int));
@@ -439,8 +440,8 @@ int timed(msa_batch *b, int kind, F &&launch)
     return MSA_OK;
 }
 
-int reduce(msa_batch *b, int op, double tol = 0.0, int max_it = 0, int max_outer = 0,
-           double ru_drop = 0.0, double ru_tol = 0.0)
+ReduceArgs reduce_args(const msa_batch *b, int op, double tol = 0.0, int max_it = 0,
+                       int max_outer = 0, double ru_drop = 0.0, double ru_tol = 0.0)
 {
     ReduceArgs a{};
     a.op = op;
@@ -451,9 +452,19 @@ int reduce(msa_batch *b, int op, double tol = 0.0, int max_it = 0, int max_outer
     a.ru_tol = ru_tol;
     a.active_count = b->d_counts;
     a.ir_count = b->d_counts + 1;
+    return a;
+}
+
+int reduce(msa_batch *b, const ReduceArgs &a)
+{
     return timed(b, KK_OTHER, [&] {
         return launch_reduce(b->ctx->stream, b->T, b->d_cls, b->d_tiles, (int)b->tiles.size(), a);
     });
+}
+
+int reduce(msa_batch *b, int op, double tol = 0.0, int max_it = 0, int max_outer = 0)
+{
+    return reduce(b, reduce_args(b, op, tol, max_it, max_outer));
 }
 
 void drop_graph(msa_batch *b)
@@ -504,36 +515,49 @@ int precond_values(msa_batch *b);
 
 // q = K p with p = z + beta p_old for every class: the stored-value product
 // and, for the classes whose product is matrix-free, k_pcg_a_mf.
-hipError_t launch_product(msa_batch *b, int pbuf)
+hipError_t launch_product(msa_batch *b, int pbuf, const PcgFuse &fz)
 {
     hipStream_t s = b->ctx->stream;
     if (b->n_items_mf == 0)
         return launch_pcg_a(s, is_mixed(b), b->T, b->unroll, b->d_cls, b->d_items,
-                            (int)b->items.size(), pbuf, b->d_counts);
+                            (int)b->items.size(), pbuf, fz);
     const hipError_t e = launch_pcg_a(s, is_mixed(b), b->T, b->unroll, b->d_cls, b->d_items_st,
-                                      b->n_items_st, pbuf, b->d_counts);
+                                      b->n_items_st, pbuf, fz);
     return e != hipSuccess ? e : launch_pcg_a_mf(s, is_mixed(b), b->dyn, b->d_cls, b->d_items_mf,
-                                                     b->n_items_mf, pbuf);
+                                                     b->n_items_mf, pbuf, fz);
 }
 
-// ru_tol > 0: reliable-update mode (inner test off, replacement triggers on).
-// cycle: with the preconditioner's own launches.
-int launch_iteration_pair(msa_batch *b, int pbuf, double tol, int max_it, double ru_tol, bool cycle)
+// One iteration.  ru_tol > 0: reliable-update mode (inner stopping test off,
+// replacement triggers on).  cycle: with the preconditioner's own launches.
+// fold: the update applies the product's reduction itself and the product
+// that of the update before it; the first iteration of a run of them finds
+// that applied already, and the last one's is applied by k_reduce.
+struct IterForm {
+    bool cycle = true, fold = false, first = true, last = true;
+};
+int launch_iteration_pair(msa_batch *b, int pbuf, double tol, int max_it, double ru_tol,
+                          const IterForm &f)
 {
     const bool mx = is_mixed(b);
     hipStream_t s = b->ctx->stream;
-    MSA_TRY(timed(b, KK_SPMV, [&] { return launch_product(b, pbuf); }));
-    MSA_TRY(reduce(b, OP_A));
+    PcgFuse fa, fb;
+    ReduceArgs rb = ru_tol > 0 ? reduce_args(b, OP_B, 0.0, max_it, 0, b->drop, ru_tol)
+                               : reduce_args(b, OP_B, tol, max_it);
+    if (f.fold) {
+        fa.fold = !f.first;
+        fa.slot = 2;
+        fa.red = rb;
+        fb.fold = 1;
+        fb.red = reduce_args(b, OP_A);
+        rb.folded = 1;
+    }
+    MSA_TRY(timed(b, KK_SPMV, [&] { return launch_product(b, pbuf, fa); }));
+    if (!f.fold) MSA_TRY(reduce(b, OP_A));
     MSA_TRY(timed(b, KK_UPDATE, [&] {
-        return launch_pcg_b(s, mx, b->T, b->d_cls, b->d_items, (int)b->items.size(), pbuf, tol,
-                            max_it, b->d_counts);
+        return launch_pcg_b(s, mx, b->T, b->d_cls, b->d_items, (int)b->items.size(), pbuf, fb);
     }));
-    if (cycle) MSA_TRY(mg_vcycle(b, pbuf, 1));
-    if (ru_tol > 0)
-        MSA_TRY(reduce(b, OP_B, 0.0, max_it, 0, b->drop, ru_tol));
-    else
-        MSA_TRY(reduce(b, OP_B, tol, max_it));
-    return MSA_OK;
+    if (f.cycle) MSA_TRY(mg_vcycle(b, pbuf, 1));
+    return f.fold && !f.last ? MSA_OK : reduce(b, rb);
 }
 
 // Classes an element-by-element (coloured) launch leaves to a matrix-free
@@ -609,16 +633,40 @@ bool part_hierarchy(const msa_batch *b)
     return false;
 }
 
+// Whether the iterations apply their reductions inside the product and the
+// update (reduced_state): one-sample tiles, no preconditioner launches between
+// update and reduction, at most kFoldChunks chunks a sample.  An iteration of
+// short launches is then two instead of four: 10^3 FP64 (5 chunks) 20.7 -> 16
+// us an iteration, 32 mixed 24^3 samples (59 chunks) 47.5 -> 43.4 ms, 64 FP64
+// 32^3 (137 chunks) 139 -> 134 ms.  Samples of more chunks keep k_reduce, two
+// 5 us launches of an iteration of 100 us and up (64^3: 1057 chunks), where
+// every workgroup would read more partials than rows.
+bool fold_reductions(const msa_batch *b, bool cycle)
+{
+    if (b->T != 1) return false;
+    if (cycle && (b->precond == MSA_PRECOND_FIRST_SAMPLE ||
+                  (b->precond == MSA_PRECOND_MULTIGRID && b->mg_depth > 0)))
+        return false;
+    for (auto &C : b->cls)
+        if (C.nchunks > kFoldChunks) return false;
+    return true;
+}
+
 // One block of `iters` PCG iterations; kind 1 adds a residual replacement
 // after every b->period iterations (inner stopping test disabled).  In a
 // batch with a partial hierarchy it ends with the count of samples that still
 // need the cycle; at zero the following blocks go without it (cycle false).
 int launch_block(msa_batch *b, int kind, int iters, double tol, int max_it, bool cycle = true)
 {
+    IterForm f;
+    f.cycle = cycle;
+    f.fold = fold_reductions(b, cycle);
     for (int k = 0; k < iters; k++) {
-        MSA_TRY(launch_iteration_pair(b, k & 1, kind == 1 ? 0.0 : tol, max_it, kind == 1 ? tol : 0.0,
-                                      cycle));
-        if (kind == 1 && (k + 1) % b->period == 0) MSA_TRY(launch_replacement(b, tol, max_it, cycle));
+        const bool rep = kind == 1 && (k + 1) % b->period == 0;
+        f.last = rep || k + 1 == iters;
+        MSA_TRY(launch_iteration_pair(b, k & 1, kind == 1 ? 0.0 : tol, max_it, kind == 1 ? tol : 0.0, f));
+        f.first = f.last;
+        if (rep) MSA_TRY(launch_replacement(b, tol, max_it, cycle));
     }
     if (cycle && part_hierarchy(b))
         MSA_TRY(timed(b, KK_OTHER, [&] {
@@ -3393,9 +3441,9 @@ int msa_batch_time_spmv(msa_batch *b, int reps, double *ms_per_launch)
     MSA_TRY(timed(b, KK_OTHER, [&] { return launch_pcg_init(s, mx, b->T, b->d_cls, b->d_items, ni, 0, b->d_counts); }));
     MSA_TRY(reduce(b, OP_INIT0));
     // pbuf 0 reads z and p1, writes p0 and q: every launch does the same work
-    MSA_HIP(launch_product(b, 0));
+    MSA_HIP(launch_product(b, 0, PcgFuse{}));
     MSA_HIP(hipEventRecord(b->timing.e0, s));
-    for (int r = 0; r < reps; r++) MSA_HIP(launch_product(b, 0));
+    for (int r = 0; r < reps; r++) MSA_HIP(launch_product(b, 0, PcgFuse{}));
     MSA_HIP(hipEventRecord(b->timing.e1, s));
     MSA_HIP(hipEventSynchronize(b->timing.e1));
     float ms = 0;
@@ -3560,11 +3608,11 @@ int msa_autotune_tile(msa_ctx *ctx, msa_mesh *mesh, int n_samples, int precision
             // warm-up, then 10 timed products (pbuf 0 keeps every sample active)
             const int reps = 10;
             hipError_t e = launch_pcg_a(s, precision == MSA_MIXED, b->T, 3, b->d_cls, b->d_items, ni, 0,
-                                        b->d_counts);
+                                        PcgFuse{});
             if (e == hipSuccess) e = hipEventRecord(b->timing.e0, s);
             for (int r = 0; r < reps && e == hipSuccess; r++)
                 e = launch_pcg_a(s, precision == MSA_MIXED, b->T, 3, b->d_cls, b->d_items, ni, 0,
-                                 b->d_counts);
+                                 PcgFuse{});
             if (e == hipSuccess) e = hipEventRecord(b->timing.e1, s);
             if (e == hipSuccess) e = hipEventSynchronize(b->timing.e1);
             float ms = 0;

@@ -1159,16 +1159,21 @@ __device__ __forceinline__ void mf_product(const ClassDev &C, const MSA_GLOBAL f
                                            const double *Es, int br, float &y0, float &y1,
                                            float &y2, float *pown = nullptr);
 
+// A sample's state with the reduction of the preceding phase applied to it
+// (defined with the reductions below).
+__device__ __forceinline__ SampleState reduced_state(const ClassDev &C, int smp, bool writer,
+                                                     const PcgFuse &fz);
+
 // Search direction + product + curvature (SolverPCGSimpleSearchVectorCalculator
 // .cs:18-41, MCPCGDirect.cs:48-51): p = z + beta p_old on the fly for every
 // gathered column, q = K p, own rows of p written to the other buffer,
-// pq = p.q per sample; the last workgroup of each tile sets alpha = rz/pq.
+// pq = p.q per sample; the reduction that follows sets alpha = rz/pq.
 // Stencil classes of one-sample tiles take the symmetric product above.
 // U: slots per group of a row (the loads of a group issue together; the
 // schedule the autotuner picks); every U sums the slots in the same order.
 template <typename real, int T, int U = 3>
 __device__ __forceinline__ void pcg_a_item(const ClassDev *__restrict__ cls, const int4 it,
-                                           int pbuf)
+                                           int pbuf, const PcgFuse &fz)
 {
     constexpr int R = 64 / T;
     const ClassDev &C = cls[it.x];
@@ -1177,8 +1182,18 @@ __device__ __forceinline__ void pcg_a_item(const ClassDev *__restrict__ cls, con
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int rr = lane / T, s = lane % T;
     const int sample = tile * T + s;
-    const bool act = sample < C.nsamp && C.st[sample].active;
-    const real beta = act ? (real)C.st[sample].beta : (real)0;
+    bool act = sample < C.nsamp;
+    real beta = 0;
+    if (T == 1 && fz.fold) {
+        if (act) {
+            const SampleState S = reduced_state(C, sample, chunk == 0, fz);
+            act = S.active;
+            beta = (real)S.beta;
+        }
+    } else {
+        act = act && C.st[sample].active;
+        if (act) beta = (real)C.st[sample].beta;
+    }
     const size_t vb = (size_t)tile * C.tile_vec;
     using V3 = vec3<real>;
     const MSA_GLOBAL real *__restrict__ z = gbl((const real *)C.z + vb);
@@ -1278,17 +1293,17 @@ __device__ __forceinline__ void pcg_a_item(const ClassDev *__restrict__ cls, con
         }
     }
     double acc[1] = {(double)pq};
-    block_partials<T, 1>(acc, C.partial + ((size_t)tile * C.nchunks + chunk) * 3 * T);
+    block_partials<T, 1>(acc, C.partial + ((size_t)tile * C.nchunks + chunk) * 3 * T + fz.slot * T);
 }
 
 template <typename real, int T, int U = 3>
 __global__ __launch_bounds__(256) void k_pcg_a(const ClassDev *__restrict__ cls,
                                                const int4 *__restrict__ items, int nitems,
-                                               int pbuf, int *active_count)
+                                               int pbuf, PcgFuse fz)
 {
     const int item = xcd_item(nitems);
     if (item < 0) return;
-    pcg_a_item<real, T, U>(cls, items[item], pbuf);
+    pcg_a_item<real, T, U>(cls, items[item], pbuf, fz);
 }
 
 // The same step for box-grid classes whose product is matrix-free
@@ -1299,12 +1314,21 @@ __global__ __launch_bounds__(256) void k_pcg_a(const ClassDev *__restrict__ cls,
 // products) with one gather per node, and the p.q partials.  No stored value
 // is read.  An item covers max(1, it.w) consecutive chunks.
 template <typename real>
-__device__ __forceinline__ void pcg_p_item(const ClassDev *__restrict__ cls, const int4 it, int pbuf)
+__device__ __forceinline__ void pcg_p_item(const ClassDev *__restrict__ cls, const int4 it, int pbuf,
+                                           const PcgFuse &fz)
 {
     const ClassDev &C = cls[it.x];
     const int tile = it.y, nch = max(1, it.w);
-    if (tile >= C.nsamp || !C.st[tile].active) return;  // one sample per tile
-    const real beta = (real)C.st[tile].beta;
+    if (tile >= C.nsamp) return;  // one sample per tile
+    real beta;
+    if (fz.fold) {
+        const SampleState S = reduced_state(C, tile, it.z == 0, fz);
+        if (!S.active) return;
+        beta = (real)S.beta;
+    } else {
+        if (!C.st[tile].active) return;
+        beta = (real)C.st[tile].beta;
+    }
     const size_t vb = (size_t)tile * C.tile_vec;
     const MSA_GLOBAL real *__restrict__ z = gbl((const real *)C.z + vb);
     const MSA_GLOBAL real *__restrict__ po = gbl((const real *)(pbuf ? C.p1 : C.p0) + vb);
@@ -1319,16 +1343,16 @@ __device__ __forceinline__ void pcg_p_item(const ClassDev *__restrict__ cls, con
 template <typename real>
 __global__ __launch_bounds__(256) void k_pcg_p(const ClassDev *__restrict__ cls,
                                                const int4 *__restrict__ items, int nitems,
-                                               int pbuf)
+                                               int pbuf, PcgFuse fz)
 {
     const int item = xcd_item(nitems);
     if (item < 0) return;
-    pcg_p_item<real>(cls, items[item], pbuf);
+    pcg_p_item<real>(cls, items[item], pbuf, fz);
 }
 
 __global__ __launch_bounds__(256) void k_pcg_a_mf(const ClassDev *__restrict__ cls,
                                                   const int4 *__restrict__ items, int nitems,
-                                                  int pbuf)
+                                                  int pbuf, int slot)
 {
     const int item = xcd_item(nitems);
     if (item < 0) return;
@@ -1364,7 +1388,7 @@ __global__ __launch_bounds__(256) void k_pcg_a_mf(const ClassDev *__restrict__ c
             }
         }
         double acc[1] = {(double)pq};
-        block_partials<1, 1>(acc, C.partial + ((size_t)tile * C.nchunks + ck) * 3);
+        block_partials<1, 1>(acc, C.partial + ((size_t)tile * C.nchunks + ck) * 3 + slot);
         // the next chunk's partials reuse the same LDS rows
         if (ck + 1 < chunk + nch) __syncthreads();
     }
@@ -1379,7 +1403,7 @@ __device__ __forceinline__ void mf64_product(const ClassDev &C, const MSA_GLOBAL
 
 template <bool DYN>
 __device__ __forceinline__ void pcg_a_mf64_item(const ClassDev *__restrict__ cls, const int4 it,
-                                                int pbuf)
+                                                int pbuf, int slot)
 {
     const ClassDev &C = cls[it.x];
     const int tile = it.y, chunk = it.z, nch = max(1, it.w);
@@ -1404,7 +1428,7 @@ __device__ __forceinline__ void pcg_a_mf64_item(const ClassDev *__restrict__ cls
             }
         }
         double acc[1] = {pq};
-        block_partials<1, 1>(acc, C.partial + ((size_t)tile * C.nchunks + ck) * 3);
+        block_partials<1, 1>(acc, C.partial + ((size_t)tile * C.nchunks + ck) * 3 + slot);
         // the next chunk's partials reuse the same LDS rows
         if (ck + 1 < chunk + nch) __syncthreads();
     }
@@ -1413,19 +1437,19 @@ __device__ __forceinline__ void pcg_a_mf64_item(const ClassDev *__restrict__ cls
 template <bool DYN>
 __global__ __launch_bounds__(256) void k_pcg_a_mf64(const ClassDev *__restrict__ cls,
                                                     const int4 *__restrict__ items, int nitems,
-                                                    int pbuf)
+                                                    int pbuf, int slot)
 {
     const int item = xcd_item(nitems);
     if (item < 0) return;
-    pcg_a_mf64_item<DYN>(cls, items[item], pbuf);
+    pcg_a_mf64_item<DYN>(cls, items[item], pbuf, slot);
 }
 
 // Update + preconditioner + stopping test (SolverPCG.cs:122-136):
-// x += alpha p, r -= alpha q, z = D^-1 r, rz = r.z, rr = r.r; the last
-// workgroup of each tile checks |r|/|b| < tol and forms beta.
+// x += alpha p, r -= alpha q, z = D^-1 r, rz = r.z, rr = r.r; the
+// reduction that follows checks |r|/|b| < tol and forms beta.
 template <typename real, int T>
 __device__ __forceinline__ void pcg_b_item(const ClassDev *__restrict__ cls, const int4 it,
-                                           int pbuf)
+                                           int pbuf, const PcgFuse &fz)
 {
     constexpr int R = 64 / T;
     const ClassDev &C = cls[it.x];
@@ -1433,8 +1457,18 @@ __device__ __forceinline__ void pcg_b_item(const ClassDev *__restrict__ cls, con
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int rr = lane / T, s = lane % T;
     const int sample = tile * T + s;
-    const bool act = sample < C.nsamp && C.st[sample].active;
-    const real alpha = act ? (real)C.st[sample].alpha : (real)0;
+    bool act = sample < C.nsamp;
+    real alpha = 0;
+    if (T == 1 && fz.fold) {
+        if (act) {
+            const SampleState S = reduced_state(C, sample, chunk == 0, fz);
+            act = S.active;
+            alpha = (real)S.alpha;
+        }
+    } else {
+        act = act && C.st[sample].active;
+        if (act) alpha = (real)C.st[sample].alpha;
+    }
     const size_t vb = (size_t)tile * C.tile_vec;
     MSA_GLOBAL real *__restrict__ x = gbl((real *)C.x + vb);
     MSA_GLOBAL real *__restrict__ r = gbl((real *)C.r + vb);
@@ -1484,12 +1518,11 @@ __device__ __forceinline__ void pcg_b_item(const ClassDev *__restrict__ cls, con
 template <typename real, int T>
 __global__ __launch_bounds__(256) void k_pcg_b(const ClassDev *__restrict__ cls,
                                                const int4 *__restrict__ items, int nitems,
-                                               int pbuf, double tol, int max_it,
-                                               int *active_count)
+                                               int pbuf, PcgFuse fz)
 {
     const int item = xcd_item(nitems);
     if (item < 0) return;
-    pcg_b_item<real, T>(cls, items[item], pbuf);
+    pcg_b_item<real, T>(cls, items[item], pbuf, fz);
 }
 
 // y = K x for every lane of one tile (tests and the single-product entry).
@@ -2602,16 +2635,22 @@ __global__ void k_kl_eval(const ClassDev *__restrict__ cp, int ntiles, int n_ele
 // 1, so the list never exceeds nsamp entries).  The list is reset by the
 // reductions that clear every flag (OP_INIT*, OP_RURESTART); no sample is
 // appended by those.
-__device__ __forceinline__ void set_due(const ClassDev &C, SampleState &S, int smp)
+__device__ __forceinline__ void set_due(const ClassDev &C, SampleState &S, int smp, bool side)
 {
     if (S.ru_due) return;
     S.ru_due = 1;
-    C.due[1 + atomicAdd(C.due, 1)] = smp;
+    if (side) C.due[1 + atomicAdd(C.due, 1)] = smp;
 }
 
-__device__ void apply_op(const ClassDev &C, int smp, const double *v, const ReduceArgs &a)
+// The state update of a.op on S, a copy or the sample's own; the counters and
+// the due list move only with `side`.
+
+__device__ __forceinline__ void apply_op(const ClassDev &C, int smp, SampleState &S, const double *v,
+                                         const ReduceArgs &a, bool side)
 {
-    SampleState &S = C.st[smp];
+    auto count = [&](int *p, int d) {
+        if (side) atomicAdd(p, d);
+    };
     switch (a.op) {
     case OP_INIT0:
     case OP_INIT1: {  // start of a PCG solve: rz = r.z, |b|
@@ -2632,7 +2671,7 @@ __device__ void apply_op(const ClassDev &C, int smp, const double *v, const Redu
         } else if (S.bnorm > 1e-25) {
             S.status = MSA_NOT_CONVERGED;
             S.active = 1;
-            atomicAdd(a.active_count, 1);
+            count(a.active_count, 1);
         } else {
             S.status = MSA_OK;
             S.relres = 0;
@@ -2654,7 +2693,7 @@ __device__ void apply_op(const ClassDev &C, int smp, const double *v, const Redu
         } else if (S.fnorm > 1e-25 && !(err < a.tol)) {
             S.status = MSA_NOT_CONVERGED;
             S.active = 1;
-            atomicAdd(a.active_count, 1);
+            count(a.active_count, 1);
         } else {
             S.status = MSA_OK;
             S.active = 0;
@@ -2680,8 +2719,8 @@ __device__ void apply_op(const ClassDev &C, int smp, const double *v, const Redu
         if (!(v[0] > 0) || !isfinite(v[0])) {
             S.status = MSA_BREAKDOWN;
             S.active = 0;
-            atomicSub(a.active_count, 1);
-            if (S.ir_active) set_due(C, S, smp);  // reliable updates: final fold + test
+            count(a.active_count, -1);
+            if (S.ir_active) set_due(C, S, smp, side);  // reliable updates: final fold + test
         } else {
             S.alpha = S.rz / v[0];
         }
@@ -2695,17 +2734,17 @@ __device__ void apply_op(const ClassDev &C, int smp, const double *v, const Redu
         if (!isfinite(err) || !isfinite(v[0])) {
             S.status = MSA_BREAKDOWN;
             S.active = 0;
-            atomicSub(a.active_count, 1);
-            if (a.ru_drop > 0) set_due(C, S, smp);  // final fold of the correction
+            count(a.active_count, -1);
+            if (a.ru_drop > 0) set_due(C, S, smp, side);  // final fold of the correction
         } else if (err < a.tol) {
             S.status = MSA_OK;
             S.active = 0;
-            atomicSub(a.active_count, 1);
+            count(a.active_count, -1);
         } else if (S.iters >= a.max_it) {
             S.status = MSA_NOT_CONVERGED;
             S.active = 0;
-            atomicSub(a.active_count, 1);
-            if (a.ru_drop > 0) set_due(C, S, smp);
+            count(a.active_count, -1);
+            if (a.ru_drop > 0) set_due(C, S, smp, side);
         } else {
             S.beta = v[0] / S.rz;
             S.rz = v[0];
@@ -2713,7 +2752,7 @@ __device__ void apply_op(const ClassDev &C, int smp, const double *v, const Redu
             // replacement) fell by ru_drop, or the FP64 stopping test may pass
             if (a.ru_drop > 0) {
                 const double rn = sqrt(v[1]);
-                if (rn < a.ru_drop || rn * S.scale < a.ru_tol * fnorm_of(C, S)) set_due(C, S, smp);
+                if (rn < a.ru_drop || rn * S.scale < a.ru_tol * fnorm_of(C, S)) set_due(C, S, smp, side);
             }
         }
         break;
@@ -2729,15 +2768,15 @@ __device__ void apply_op(const ClassDev &C, int smp, const double *v, const Redu
         if (!isfinite(err)) {
             S.status = MSA_BREAKDOWN;
             S.ir_active = 0;
-            atomicSub(a.ir_count, 1);
+            count(a.ir_count, -1);
         } else if (err < a.tol) {
             S.status = MSA_OK;
             S.ir_active = 0;
-            atomicSub(a.ir_count, 1);
+            count(a.ir_count, -1);
         } else if (S.outer >= a.max_outer) {
             S.status = MSA_NOT_CONVERGED;
             S.ir_active = 0;
-            atomicSub(a.ir_count, 1);
+            count(a.ir_count, -1);
         } else {
             S.scale = nr;
         }
@@ -2765,10 +2804,10 @@ __device__ void apply_op(const ClassDev &C, int smp, const double *v, const Redu
         if (done) {
             S.ir_active = 0;
             S.ru_due = 0;
-            atomicSub(a.ir_count, 1);
+            count(a.ir_count, -1);
             if (S.active) {
                 S.active = 0;
-                atomicSub(a.active_count, 1);
+                count(a.active_count, -1);
             }
         } else {
             S.pq = S.scale / nr;  // rescale ratio of the search direction
@@ -2837,12 +2876,62 @@ __device__ __forceinline__ void reduce_tile(const ClassDev *__restrict__ cls, co
         const int t = threadIdx.x;
         const int smp = tile * T + t;
         const double v[2] = {red[0][t], red[1][t]};
-        if (smp < C.nsamp) apply_op(C, smp, v, a);
+        if (smp < C.nsamp) {
+            SampleState &S = C.st[smp];
+            if (a.folded) S = C.st_b[smp];
+            apply_op(C, smp, S, v, a, true);
+        }
     }
     // these ops clear every replacement flag of the class and append none
     if ((a.op == OP_INIT0 || a.op == OP_INIT1 || a.op == OP_INIT2 || a.op == OP_RURESTART) &&
         tile == 0 && threadIdx.x == 0)
         *C.due = 0;
+}
+
+// The reduction of the preceding phase, formed by every workgroup that needs
+// it instead of a launch of its own: in batches of small classes an iteration
+// is a chain of short launches, and the two reductions are two of the four
+// (launch_block has the rule and the figures).  Each wave sums the sample's
+// partials in reduce_tile's order (thread v of 1024 holds chunk v; up to
+// kFoldChunks = 256 of them, the others zero: the lane holds chunks lane,
+// lane + 64, ..), so the bits are those of k_reduce.  All workgroups compute
+// the same new state; the workgroup of the sample's first chunk stores it
+// and moves the counters.  No workgroup reads what another one writes in the
+// same launch: the product reads st_b and partial slots 0 and 1 and writes st
+// and slot 2, the update reads st and slot 2 and writes st_b and slots 0, 1.
+__device__ __forceinline__ SampleState reduced_state(const ClassDev &C, int smp, bool writer,
+                                                     const PcgFuse &fz)
+{
+    static_assert(kFoldChunks == 256, "four partials per lane");
+    const int lane = threadIdx.x & 63;
+    const bool upd = fz.red.op == OP_A;  // the reader is the update
+    const double *base = C.partial + (size_t)smp * C.nchunks * 3 + (upd ? 2 : 0);
+    double p[2][4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int c = lane + 64 * j;
+        p[0][j] = p[1][j] = 0.0;
+        if (c < C.nchunks) {
+            p[0][j] = base[(size_t)c * 3];
+            if (!upd) p[1][j] = base[(size_t)c * 3 + 1];
+        }
+    }
+    double v[2];
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        v[k] = (p[k][0] + p[k][2]) + (p[k][1] + p[k][3]);
+#pragma unroll
+        for (int st = 32; st >= 1; st >>= 1) v[k] += __shfl_down(v[k], st);
+        v[k] = __shfl(v[k], 0);
+    }
+    SampleState S = upd ? C.st[smp] : C.st_b[smp];
+    if (writer && threadIdx.x == 0) {
+        SampleState W = S;
+        apply_op(C, smp, W, v, fz.red, true);
+        (upd ? C.st_b : C.st)[smp] = W;
+    }
+    apply_op(C, smp, S, v, fz.red, false);
+    return S;
 }
 
 template <int T>
@@ -2887,16 +2976,16 @@ __global__ __launch_bounds__(256) void k_pcg_persist(const ClassDev *__restrict_
         const int pbuf = (pbuf0 + k) & 1;
         if constexpr (MF != 0) {
             for (int i = i0; i < i1; i += gx)
-                if (cls[items[i].x].mf_pcg) pcg_p_item<real>(cls, items[i], pbuf);
+                if (cls[items[i].x].mf_pcg) pcg_p_item<real>(cls, items[i], pbuf, PcgFuse{});
             barrier();
         }
         for (int i = i0; i < i1; i += gx) {
             bool mf = false;
             if constexpr (MF != 0) mf = cls[items[i].x].mf_pcg != 0;
             if (!mf) {
-                pcg_a_item<real, T, U>(cls, items[i], pbuf);
+                pcg_a_item<real, T, U>(cls, items[i], pbuf, PcgFuse{});
             } else {
-                if constexpr (MF != 0) pcg_a_mf64_item<MF == 2>(cls, items[i], pbuf);
+                if constexpr (MF != 0) pcg_a_mf64_item<MF == 2>(cls, items[i], pbuf, 0);
             }
             __syncthreads();
         }
@@ -2907,7 +2996,7 @@ __global__ __launch_bounds__(256) void k_pcg_persist(const ClassDev *__restrict_
         }
         barrier();
         for (int i = i0; i < i1; i += gx) {
-            pcg_b_item<real, T>(cls, items[i], pbuf);
+            pcg_b_item<real, T>(cls, items[i], pbuf, PcgFuse{});
             __syncthreads();
         }
         barrier();
@@ -5137,48 +5226,51 @@ hipError_t launch_pcg_init(hipStream_t s, bool mixed, int T, const ClassDev *d_c
 
 template <typename real>
 static hipError_t pcg_a_unrolled(hipStream_t s, int U, dim3 grid, const ClassDev *d_cls,
-                                 const int4 *items, int nitems, int pbuf, int *active_count)
+                                 const int4 *items, int nitems, int pbuf, const PcgFuse &fz)
 {
     switch (U) {
-    case 1: hipLaunchKernelGGL((k_pcg_a<real, 1, 1>), grid, dim3(256), 0, s, d_cls, items, nitems, pbuf, active_count); break;
-    case 2: hipLaunchKernelGGL((k_pcg_a<real, 1, 2>), grid, dim3(256), 0, s, d_cls, items, nitems, pbuf, active_count); break;
-    case 3: hipLaunchKernelGGL((k_pcg_a<real, 1, 3>), grid, dim3(256), 0, s, d_cls, items, nitems, pbuf, active_count); break;
-    case 4: hipLaunchKernelGGL((k_pcg_a<real, 1, 4>), grid, dim3(256), 0, s, d_cls, items, nitems, pbuf, active_count); break;
+    case 1: hipLaunchKernelGGL((k_pcg_a<real, 1, 1>), grid, dim3(256), 0, s, d_cls, items, nitems, pbuf, fz); break;
+    case 2: hipLaunchKernelGGL((k_pcg_a<real, 1, 2>), grid, dim3(256), 0, s, d_cls, items, nitems, pbuf, fz); break;
+    case 3: hipLaunchKernelGGL((k_pcg_a<real, 1, 3>), grid, dim3(256), 0, s, d_cls, items, nitems, pbuf, fz); break;
+    case 4: hipLaunchKernelGGL((k_pcg_a<real, 1, 4>), grid, dim3(256), 0, s, d_cls, items, nitems, pbuf, fz); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
 }
 
 hipError_t launch_pcg_a(hipStream_t s, bool mixed, int T, int U, const ClassDev *d_cls,
-                        const int4 *items, int nitems, int pbuf, int *active_count)
+                        const int4 *items, int nitems, int pbuf, const PcgFuse &fz)
 {
     if (T == 1 && U != 3) {
         if (nitems <= 0) return hipSuccess;
         const dim3 grid(xcd_grid(nitems));
-        return mixed ? pcg_a_unrolled<float>(s, U, grid, d_cls, items, nitems, pbuf, active_count)
-                     : pcg_a_unrolled<double>(s, U, grid, d_cls, items, nitems, pbuf, active_count);
+        return mixed ? pcg_a_unrolled<float>(s, U, grid, d_cls, items, nitems, pbuf, fz)
+                     : pcg_a_unrolled<double>(s, U, grid, d_cls, items, nitems, pbuf, fz);
     }
     if (U != 3) return hipErrorInvalidValue;  // lane tiles T > 1 use groups of 3 slots
-    MSA_PCG_LAUNCH(k_pcg_a, d_cls, items, nitems, pbuf, active_count);
+    MSA_PCG_LAUNCH(k_pcg_a, d_cls, items, nitems, pbuf, fz);
 }
 
 hipError_t launch_pcg_a_mf(hipStream_t s, bool mixed, bool dyn, const ClassDev *d_cls,
-                           const int4 *items, int nitems, int pbuf)
+                           const int4 *items, int nitems, int pbuf, const PcgFuse &fz)
 {
     if (nitems <= 0) return hipSuccess;
     const dim3 grid(xcd_grid(nitems)), block(256);
     if (mixed)
-        hipLaunchKernelGGL(k_pcg_p<float>, grid, block, 0, s, d_cls, items, nitems, pbuf);
+        hipLaunchKernelGGL(k_pcg_p<float>, grid, block, 0, s, d_cls, items, nitems, pbuf, fz);
     else
-        hipLaunchKernelGGL(k_pcg_p<double>, grid, block, 0, s, d_cls, items, nitems, pbuf);
+        hipLaunchKernelGGL(k_pcg_p<double>, grid, block, 0, s, d_cls, items, nitems, pbuf, fz);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (mixed)
-        hipLaunchKernelGGL(k_pcg_a_mf, grid, block, 0, s, d_cls, items, nitems, pbuf);
+        hipLaunchKernelGGL(k_pcg_a_mf, grid, block, 0, s, d_cls, items, nitems, pbuf,
+                           fz.slot);
     else if (dyn)
-        hipLaunchKernelGGL(k_pcg_a_mf64<true>, grid, block, 0, s, d_cls, items, nitems, pbuf);
+        hipLaunchKernelGGL(k_pcg_a_mf64<true>, grid, block, 0, s, d_cls, items, nitems, pbuf,
+                           fz.slot);
     else
-        hipLaunchKernelGGL(k_pcg_a_mf64<false>, grid, block, 0, s, d_cls, items, nitems, pbuf);
+        hipLaunchKernelGGL(k_pcg_a_mf64<false>, grid, block, 0, s, d_cls, items, nitems, pbuf,
+                           fz.slot);
     return hipGetLastError();
 }
 
@@ -5234,9 +5326,9 @@ hipError_t launch_pcg_persist(hipStream_t s, bool mixed, int U, const ClassDev *
 }
 
 hipError_t launch_pcg_b(hipStream_t s, bool mixed, int T, const ClassDev *d_cls, const int4 *items,
-                        int nitems, int pbuf, double tol, int max_it, int *active_count)
+                        int nitems, int pbuf, const PcgFuse &fz)
 {
-    MSA_PCG_LAUNCH(k_pcg_b, d_cls, items, nitems, pbuf, tol, max_it, active_count);
+    MSA_PCG_LAUNCH(k_pcg_b, d_cls, items, nitems, pbuf, fz);
 }
 
 hipError_t launch_spmv(hipStream_t s, bool mixed, int T, const ClassDev *d_cls, const int4 *items,

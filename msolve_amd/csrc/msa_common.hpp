@@ -176,6 +176,7 @@ struct ClassDev {
     double *phi;          // [n_elem][M]
     double *xi;           // [ntiles*T][M]
     SampleState *st;      // [ntiles*T]
+    SampleState *st_b;  // its other copy while reductions fold into the phases
     double *partial;      // [ntiles][nchunks][3][T]
     int *negdet;          // [1]
     int *due;             // [1 + nsamp]: count, then samples with a pending replacement
@@ -334,13 +335,22 @@ struct ReduceArgs {
     int op;
     int max_it;
     int max_outer;
-    int pad;
+    int folded;  // 1: the sample's state comes from st_b (see PcgFuse)
     double tol;
     double ru_drop;  // > 0: reliable-update mode of OP_B (trigger factor)
     double ru_tol;   // FP64 stopping tolerance seen by OP_B in that mode
     int *active_count;
     int *ir_count;
 };
+
+// How a PCG phase gets the reduction before it.  fold 0: from the sample's
+// state, k_reduce has run; fold 1: the phase applies `red` itself.  slot: the
+// partial slot the product writes (2 where the next phase folds).
+struct PcgFuse {
+    int fold = 0, slot = 0;
+    ReduceArgs red{};
+};
+constexpr int kFoldChunks = 256;  // most chunks of a sample whose reductions fold
 
 enum KernelKind { KK_SPMV = 0, KK_UPDATE = 1, KK_ASSEMBLE = 2, KK_RES64 = 3, KK_OTHER = 4, KK_MG = 5 };
 constexpr int kKernelKinds = 6;
@@ -384,7 +394,7 @@ hipError_t launch_pcg_init(hipStream_t s, bool mixed, int T, const ClassDev *d_c
                            const int4 *items, int nitems, int mode, int *active_count);
 // U: slots per group of a row (1..4 at T = 1, 3 for T > 1)
 hipError_t launch_pcg_a(hipStream_t s, bool mixed, int T, int U, const ClassDev *d_cls,
-                        const int4 *items, int nitems, int pbuf, int *active_count);
+                        const int4 *items, int nitems, int pbuf, const PcgFuse &fz);
 // need_due 1: the samples due for a replacement, 0: every refining one
 hipError_t launch_residual64_mf_box(hipStream_t s, bool dyn, const ClassDev *d_cls,
                                    const int4 *items, int nitems, int need_due);
@@ -392,9 +402,9 @@ hipError_t launch_dyn_rhs_mf(hipStream_t s, bool stiff, const ClassDev *d_cls, c
                              int nitems);
 // mixed: FP32 vectors and product, else FP64; dyn: with the consistent mass
 hipError_t launch_pcg_a_mf(hipStream_t s, bool mixed, bool dyn, const ClassDev *d_cls,
-                           const int4 *items, int nitems, int pbuf);
+                           const int4 *items, int nitems, int pbuf, const PcgFuse &fz);
 hipError_t launch_pcg_b(hipStream_t s, bool mixed, int T, const ClassDev *d_cls, const int4 *items,
-                        int nitems, int pbuf, double tol, int max_it, int *active_count);
+                        int nitems, int pbuf, const PcgFuse &fz);
 hipError_t launch_ir_begin(hipStream_t s, int T, const ClassDev *d_cls, const int4 *items,
                            int nitems, int *ir_count, int warm);
 hipError_t launch_ir_update(hipStream_t s, int T, const ClassDev *d_cls, const int4 *items,
