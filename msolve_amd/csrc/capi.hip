@@ -171,7 +171,7 @@ struct msa_batch {
     int mg_nlv_gitems = 0;
     int4 *mg_co_items = nullptr;        // the coarsest levels
     int mg_nco_items = 0;
-    int4 *mf_items = nullptr;           // solved classes with matrix-free products
+    int4 *mf_items = nullptr;           // solved classes with matrix-free residuals (mf_r)
     int n_mf_items = 0;                 //   (general grids; box grids: runs of chunks below)
     int4 *mf_box_items = nullptr;
     int n_mf_box_items = 0;
@@ -576,13 +576,9 @@ int max_tiles(const msa_batch *b)
     return m;
 }
 
-// Whether uniform-grid classes of a MIXED batch have their FP64 residual
-// formed matrix-free (multigrid set up), and those launches.
-bool mf_residual(const msa_batch *b)
-{
-    return is_mixed(b) && b->precond == MSA_PRECOND_MULTIGRID && b->mg_ready &&
-           b->n_mf_items + b->n_mf_box_items > 0;
-}
+// Whether classes of a MIXED batch have their FP64 residual formed
+// matrix-free (sync_mf_residual), and those launches.
+bool mf_residual(const msa_batch *b) { return is_mixed(b) && b->n_mf_items + b->n_mf_box_items > 0; }
 int launch_residual_mf(msa_batch *b, int need_due)
 {
     hipStream_t s = b->ctx->stream;
@@ -601,7 +597,7 @@ int launch_replacement(msa_batch *b, double tol, int max_it, bool cycle)
     hipStream_t s = b->ctx->stream;
     const int T = b->T, ni = (int)b->items.size();
     MSA_TRY(timed(b, KK_OTHER, [&] { return launch_ru_fold(s, T, b->d_cls, b->d_items, ni); }));
-    // matrix-free residual of the uniform-grid classes (multigrid set up),
+    // matrix-free residual of the classes that take it (sync_mf_residual),
     // the coloured element scatter for the others
     const bool mfres = mf_residual(b);
     if (mfres) MSA_TRY(launch_residual_mf(b, 1));
@@ -852,8 +848,8 @@ ColourLaunch colour_launch(const msa_batch *b, int colour, int *nblocks, ColourS
         const MeshHost &m = b->cls[c].mesh->h;
         int cnt = colour < m.ncolours ? m.colour_ptr[colour + 1] - m.colour_ptr[colour] : 0;
         const ClassDev &D = b->cls[c].dev;
-        const bool box = is_mixed(b) ? D.mf && D.mf_box : D.mf_pcg != 0;
-        if ((skip == SKIP_MF && D.mf) || (skip == SKIP_MF_EXACT && D.mf && D.mf_exact) ||
+        const bool box = is_mixed(b) ? D.mf_r && D.mf_box : D.mf_pcg != 0;
+        if ((skip == SKIP_MF && D.mf_r) || (skip == SKIP_MF_EXACT && D.mf_r && D.mf_exact) ||
             (skip == SKIP_MF_RHS && box && D.mf_exact))
             cnt = 0;
         cl.prefix[c + 1] = cl.prefix[c] + cnt;
@@ -1196,6 +1192,14 @@ void class_run_items(const ClassHost &C, int ci, std::vector<int4> &out, int run
 // 21.9 / 24.6, 16 x 16^3 (304) 34.2 / 24.1, 32^3 (133) 27.2 / 20.1.
 bool mf64_large(const msa_batch *b) { return !is_mixed(b) && b->items.size() >= 128; }
 
+// MIXED batches that form the FP64 residual matrix-free also without a
+// hierarchy, on box grids of equal cells: from 128 chunks on, the size from
+// which the eight coloured launches are more than launches (32 samples of
+// 24^3, 1888 chunks: 8 x 14 us each replacement; 17 samples of four meshes,
+// 391: 8 x 2.5 us) and repay the grid tables that a batch then uploads when
+// it is created.
+bool mf_res_large(const msa_batch *b) { return is_mixed(b) && b->items.size() >= 128; }
+
 int sync_mf_pcg(msa_batch *b)
 {
     bool changed = false, any = false;
@@ -1229,6 +1233,34 @@ int sync_mf_pcg(msa_batch *b)
     return upload_class_table(b);
 }
 
+// Which classes of a MIXED batch form the FP64 residual matrix-free: uniform
+// grids with the multigrid tables set up, and box grids of equal cells
+// (mf_res).  Called with sync_mf_pcg.
+int sync_mf_residual(msa_batch *b)
+{
+    if (!is_mixed(b)) return MSA_OK;
+    const bool mg = b->precond == MSA_PRECOND_MULTIGRID && b->mg_ready;
+    bool changed = false;
+    for (auto &C : b->cls) {
+        const int want = (mg && C.dev.mf) || C.dev.mf_res;
+        changed |= C.dev.mf_r != want;
+        C.dev.mf_r = want;
+    }
+    if (!changed) return MSA_OK;
+    std::vector<int4> general, box;
+    for (int c = 0; c < (int)b->cls.size(); c++) {
+        const ClassDev &D = b->cls[c].dev;
+        if (D.mf_r && D.mf_box)
+            class_run_items(b->cls[c], c, box);
+        else if (D.mf_r)
+            class_items(b->cls[c], c, general);
+    }
+    MSA_TRY(items_to_device(b, general, &b->mf_items, &b->n_mf_items));
+    MSA_TRY(items_to_device(b, box, &b->mf_box_items, &b->n_mf_box_items));
+    drop_graph(b);
+    return upload_class_table(b);
+}
+
 // Work items of the grouped gather assembly: tiles in groups of kAsmGroup.
 void class_group_items(const ClassHost &C, int ci, std::vector<int4> &out)
 {
@@ -1252,12 +1284,16 @@ int assemble_items(msa_batch *b, const int4 *items, int nitems, const int4 *gite
 // batches take box grids whose cells are equal up to the rounding of the
 // coordinates: the shared element matrix then is every element's to FP64
 // rounding (MIXED: cells equal to 1e-9, FP32 products).
-int mf_setup(msa_batch *b, ClassHost &C)
+int mf_setup(msa_batch *b, ClassHost &C, bool residual_only)
 {
     const GridInfo &g = C.grid;
-    if (b->T != 1 || C.dev.mf || C.dev.mf64 || g.nx == 0) return MSA_OK;
-    if (!is_mixed(b) && !(g.box && g.exact)) return MSA_OK;
     ClassDev &D = C.dev;
+    if (b->T != 1 || D.mf || D.mf64 || g.nx == 0) return MSA_OK;
+    if ((!is_mixed(b) || residual_only) && !(g.box && g.exact)) return MSA_OK;
+    if (D.mf_res) {  // the tables are there
+        D.mf = !residual_only;
+        return MSA_OK;
+    }
     MSA_TRY(upload_vec(b, g.gblock, &D.mf_gblock));
     MSA_TRY(upload_vec(b, g.cell_elem, &D.mf_cell));
     MSA_TRY(upload_vec(b, g.bpos, &D.mf_bpos));
@@ -1281,7 +1317,9 @@ int mf_setup(msa_batch *b, ClassHost &C)
     D.mf_free = 1;
     for (int bb = 0; bb < m.nb; bb++)
         if (m.node_free[m.block_node[bb]] != 7) D.mf_free = 0;
-    if (is_mixed(b))
+    if (residual_only)
+        D.mf_res = 1;
+    else if (is_mixed(b))
         D.mf = 1;
     else
         D.mf64 = 1;
@@ -1333,7 +1371,7 @@ int mg_build(msa_batch *b, int max_levels)
         if (meshes.empty() || meshes.back().n_free > kMgCoarsestMax) continue;
         b->mg_nlev[c] = (int)meshes.size();
         depth_classes[0].push_back(c);
-        MSA_TRY(mf_setup(b, b->cls[c]));
+        MSA_TRY(mf_setup(b, b->cls[c], false));
         int parent = c;
         for (size_t l = 0; l < meshes.size(); l++) {
             msa_mesh *m = new msa_mesh();
@@ -1346,7 +1384,7 @@ int mg_build(msa_batch *b, int max_levels)
             ClassHost &L = b->lv.back();
             MSA_TRY(setup_class(b, L, m, b->cls[c].nsamp));
             L.has_E = true;
-            MSA_TRY(mf_setup(b, L));
+            MSA_TRY(mf_setup(b, L, false));
             ClassDev &D = L.dev;
             D.mg_root = c;
             D.mg_st = b->cls[c].dev.st;
@@ -1475,18 +1513,6 @@ int mg_build(msa_batch *b, int max_levels)
         if (d > 0) MSA_TRY(items_to_device(b, re, &b->mg_restr[d], &b->mg_nrestr[d]));
     }
     MSA_TRY(items_to_device(b, all, &b->mg_lv_items, &b->mg_nlv_items));
-    {
-        std::vector<int4> mfi, mfb;
-        for (int c = 0; c < ncls; c++)
-            if (b->cls[c].dev.mf) {
-                if (b->cls[c].dev.mf_box)
-                    class_run_items(b->cls[c], c, mfb);
-                else
-                    class_items(b->cls[c], c, mfi);
-            }
-        MSA_TRY(items_to_device(b, mfi, &b->mf_items, &b->n_mf_items));
-        MSA_TRY(items_to_device(b, mfb, &b->mf_box_items, &b->n_mf_box_items));
-    }
     std::vector<int4> gall;
     for (size_t l = 0; l < b->lv.size(); l++)
         class_group_items(b->lv[l], (int)(b->cls.size() + l), gall);
@@ -2235,7 +2261,8 @@ int msa_batch_create(msa_ctx *ctx, int n_classes, msa_mesh *const *meshes, const
             for (int k = 0; k < C.nchunks; k++) b->items.push_back(make_int4(c, t, k, 0));
         }
     }
-    for (int c = 0; c < n_classes && rc == MSA_OK && mf64_large(b); c++) rc = mf_setup(b, b->cls[c]);
+    for (int c = 0; c < n_classes && rc == MSA_OK && (mf64_large(b) || mf_res_large(b)); c++)
+        rc = mf_setup(b, b->cls[c], is_mixed(b));
     if (rc != MSA_OK) return fail(rc);
     void *p = nullptr;
     rc = dalloc(b, &p, sizeof(ClassDev) * n_classes);
@@ -2419,7 +2446,7 @@ int msa_batch_assemble(msa_batch *b, double nu)
             MSA_TRY(timed(b, KK_ASSEMBLE, [&] {
                 return launch_khat_cache(s, b->d_cls + c, C.mesh->h.n_elem, nu, C.dev.dyn);
             }));
-            if (C.dev.mf64)
+            if (C.dev.mf64 || C.dev.mf_res)
                 MSA_TRY(timed(b, KK_ASSEMBLE, [&] { return launch_mf_khat(s, b->d_cls + c); }));
             C.kc_nu = nu;
             C.kc_mass = C.dev.dyn;
@@ -2481,6 +2508,7 @@ int msa_batch_solve(msa_batch *b, double tol, int max_it, double inner_tol, int 
     const int T = b->T, ni = (int)b->items.size();
     if (!b->mg_ready) MSA_TRY(precond_values(b));
     MSA_TRY(sync_mf_pcg(b));
+    MSA_TRY(sync_mf_residual(b));
     if (b->dyn) {
         // static solve with the effective matrix: per-sample right-hand side = f
         MSA_TRY(timed(b, KK_OTHER, [&] { return launch_fs_static(s, T, b->d_cls, b->d_items, ni); }));
@@ -2770,6 +2798,7 @@ int msa_batch_newmark(msa_batch *b, int nsteps, const double *acc, int acc_dir, 
     const int T = b->T, ni = (int)b->items.size();
     if (b->solver != MSA_SOLVER_DIRECT && !b->mg_ready) MSA_TRY(precond_values(b));
     MSA_TRY(sync_mf_pcg(b));
+    MSA_TRY(sync_mf_residual(b));
     if (acc_dir >= 0) {
         if (b->acc_cap < nsteps) {
             void *p = nullptr;

@@ -258,6 +258,10 @@ struct ClassDev {
     // the rounding of the coordinates (mf stays 0; the mf_ tables and mf_k64
     // are set).  mf_free: every block fully free.
     int mf64, mf_free;
+    // MIXED: the FP64 residual matrix-free without the multigrid tables (mf
+    // stays 0; a box grid of equal cells, the tables as for mf64); mf_r: the
+    // class takes it in this solve (mf_res, or mf with multigrid set up)
+    int mf_res, mf_r;
     int mf_exact;  // mf / mf64 class whose cells are equal up to coordinate rounding
     // FP64 copy of the stored values (same layout as a one-sample-tile FP64
     // batch) for the coarsest multigrid level of a MIXED batch: the band

@@ -57,3 +57,44 @@ def test_partial_hierarchy_equals_separate_batches(ctx, precision, method, graph
         for u, v in zip(both[sh][1], alone[sh][1]):
             assert np.array_equal(u, v)
     assert both[odd][0].min() > 2 * both[cube][0].max()  # the cycle was left out for a while
+
+
+@pytest.mark.parametrize("dyn", [False, True])
+@pytest.mark.parametrize("shape,lengths,roller", [((5, 4, 3), (5.0, 4.0, 3.0), False),
+                                                  ((70, 2, 2), (35.0, 1.5, 1.0), True),
+                                                  ((1, 9, 8), (1.0, 4.5, 8.0), False)])
+def test_mixed_residual_without_hierarchy(ctx, shape, lengths, roller, dyn):
+    """Jacobi MIXED batches from 128 chunks on form the FP64 residual
+    matrix-free: the first samples against a batch of those alone (too few
+    chunks: the coloured residual).  Both stop at a true relative residual of
+    1e-11; the blocks' condition is below 1e4 (70 x 2 x 2: clamped along the
+    side)."""
+    xyz, conn = box_mesh(*shape, *lengths)
+    cons = np.zeros((xyz.shape[0], 3), bool)
+    cons[xyz[:, 1] < 1e-12] = True
+    if roller:
+        cons[xyz[:, 0] > lengths[0] * (1 - 1e-12), 2] = True
+    dof, nf = msa.enumerate_dofs(cons)
+    rng = np.random.default_rng(4)
+    f, E = rng.standard_normal(nf), rng.uniform(1.0, 3.0, (130, conn.shape[0]))
+    out = []
+    for ns in (130, 3):
+        mesh = msa.Mesh(ctx, xyz, conn, dof, nf)
+        b = msa.Batch(ctx, [mesh], [ns], L.MSA_MIXED, 1)
+        b.set_modulus(0, E[:ns])
+        b.set_rhs(0, f)
+        if dyn:
+            b.set_dynamics(1e-2, 0.5, 1e-3, 0.25, 0.5, 1e-2)
+        b.assemble(0.25)
+        b.assemble(0.3)  # the tables follow a new Poisson ratio
+        b.solve(tol=1e-11, max_it=5000, graph_iters=8)
+        assert (b.stats(0)["status"] == msa.MSA_OK).all()
+        u = [b.solution(0, s) for s in range(3)]
+        if dyn:
+            b.newmark(np.linspace(1.0, 0.5, 4), acc_dir=0, tol=1e-11, max_it=5000, graph_iters=8)
+            u += [v for s in range(3) for v in b.dynamic_state(0, s)[:3]]
+        out.append(u)
+        b.close()
+        mesh.close()
+    for a, c in zip(*out):
+        assert np.linalg.norm(a - c) <= 1e-7 * np.linalg.norm(c)
