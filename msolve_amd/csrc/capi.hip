@@ -96,6 +96,8 @@ struct msa_batch {
     std::vector<void *> allocs;
     long long bytes = 0;
     bool assembled = false;
+    bool small = false;       // one-sample tiles, few slices of 64 rows in all (kSmallSlices)
+    long long chunks4 = 0;    // chunks of four slices in all
     bool loaded = false;      // values set by msa_batch_set_matrix_csr, not assembled
     bool factored = false;    // band Cholesky factors match the assembled values
     double zem_tol = 0.0;     // zero-energy-mode pivot tolerance (0: off)
@@ -259,7 +261,10 @@ int setup_class(msa_batch *b, ClassHost &C, msa_mesh *mesh, int nsamp)
         C.nsamp = nsamp;
         C.ntiles = (C.nsamp + T - 1) / T;
         C.nslices = (h.nb + R - 1) / R;
-        C.chunk = kWaves * std::max(1, 16 / R);
+        // small batches: a slice per workgroup (few compute units would stream
+        // the whole matrix otherwise); larger samples keep fewer partials than
+        // the phases fold
+        C.chunk = b->small && C.nslices <= kFoldChunks ? 1 : kWaves * std::max(1, 16 / R);
         C.nchunks = (C.nslices + C.chunk - 1) / C.chunk;
         C.R = R;
         int sy = 0, sz = 0;
@@ -514,17 +519,22 @@ int mg_lanczos(msa_batch *b);
 int precond_values(msa_batch *b);
 
 // q = K p with p = z + beta p_old for every class: the stored-value product
-// and, for the classes whose product is matrix-free, k_pcg_a_mf.
-hipError_t launch_product(msa_batch *b, int pbuf, const PcgFuse &fz)
+// and, for the classes whose product is matrix-free, k_pcg_a_mf.  Stored
+// products of symmetric classes in small batches take the split form.  cycle:
+// false once no sample with a hierarchy is active, and MIXED matrix-free
+// products have one.
+hipError_t launch_product(msa_batch *b, int pbuf, const PcgFuse &fz, bool cycle = true)
 {
     hipStream_t s = b->ctx->stream;
-    if (b->n_items_mf == 0)
-        return launch_pcg_a(s, is_mixed(b), b->T, b->unroll, b->d_cls, b->d_items,
-                            (int)b->items.size(), pbuf, fz);
-    const hipError_t e = launch_pcg_a(s, is_mixed(b), b->T, b->unroll, b->d_cls, b->d_items_st,
-                                      b->n_items_st, pbuf, fz);
-    return e != hipSuccess ? e : launch_pcg_a_mf(s, is_mixed(b), b->dyn, b->d_cls, b->d_items_mf,
-                                                     b->n_items_mf, pbuf, fz);
+    const bool mx = is_mixed(b), some = b->n_items_mf > 0;
+    const int4 *items = some ? b->d_items_st : b->d_items;
+    const int ni = some ? b->n_items_st : (int)b->items.size();
+    bool split = true;
+    for (auto &C : b->cls) split = split && (C.dev.mf_pcg || (C.dev.sym && C.chunk == 1));
+    const hipError_t e = split ? launch_pcg_a_split(s, mx, b->d_cls, items, ni, pbuf, fz)
+                               : launch_pcg_a(s, mx, b->T, b->unroll, b->d_cls, items, ni, pbuf, fz);
+    if (e != hipSuccess || !some || (mx && !cycle)) return e;
+    return launch_pcg_a_mf(s, mx, b->dyn, b->d_cls, b->d_items_mf, b->n_items_mf, pbuf, fz);
 }
 
 // One iteration.  ru_tol > 0: reliable-update mode (inner stopping test off,
@@ -551,7 +561,7 @@ int launch_iteration_pair(msa_batch *b, int pbuf, double tol, int max_it, double
         fb.red = reduce_args(b, OP_A);
         rb.folded = 1;
     }
-    MSA_TRY(timed(b, KK_SPMV, [&] { return launch_product(b, pbuf, fa); }));
+    MSA_TRY(timed(b, KK_SPMV, [&] { return launch_product(b, pbuf, fa, f.cycle); }));
     if (!f.fold) MSA_TRY(reduce(b, OP_A));
     MSA_TRY(timed(b, KK_UPDATE, [&] {
         return launch_pcg_b(s, mx, b->T, b->d_cls, b->d_items, (int)b->items.size(), pbuf, fb);
@@ -1190,7 +1200,7 @@ void class_run_items(const ClassHost &C, int ci, std::vector<int4> &out, int run
 // 128 chunks every kernel lasts as long as its launch, and the p pass is one
 // launch more: us per iteration, stored / matrix-free, 24^3 (60 chunks)
 // 21.9 / 24.6, 16 x 16^3 (304) 34.2 / 24.1, 32^3 (133) 27.2 / 20.1.
-bool mf64_large(const msa_batch *b) { return !is_mixed(b) && b->items.size() >= 128; }
+bool mf64_large(const msa_batch *b) { return !is_mixed(b) && b->chunks4 >= 128; }
 
 // MIXED batches that form the FP64 residual matrix-free also without a
 // hierarchy, on box grids of equal cells: from 128 chunks on, the size from
@@ -1198,7 +1208,7 @@ bool mf64_large(const msa_batch *b) { return !is_mixed(b) && b->items.size() >= 
 // 24^3, 1888 chunks: 8 x 14 us each replacement; 17 samples of four meshes,
 // 391: 8 x 2.5 us) and repay the grid tables that a batch then uploads when
 // it is created.
-bool mf_res_large(const msa_batch *b) { return is_mixed(b) && b->items.size() >= 128; }
+bool mf_res_large(const msa_batch *b) { return is_mixed(b) && b->chunks4 >= 128; }
 
 int sync_mf_pcg(msa_batch *b)
 {
@@ -2251,6 +2261,13 @@ int msa_batch_create(msa_ctx *ctx, int n_classes, msa_mesh *const *meshes, const
         msa_batch_destroy(b);
         return code;
     };
+    long long slices = 0;
+    for (int c = 0; c < n_classes; c++) {
+        const long long ns = (meshes[c]->h.nb + b->R - 1) / b->R, nt = (n_samples[c] + tile - 1) / tile;
+        slices += ns * nt;
+        b->chunks4 += (ns + kWaves - 1) / kWaves * nt;
+    }
+    b->small = tile == 1 && slices <= (is_mixed(b) ? kSmallSlices : kSmallSlices / 2);
     for (int c = 0; c < n_classes && rc == MSA_OK; c++) {
         rc = setup_class(b, b->cls[c], meshes[c], n_samples[c]);
         if (rc != MSA_OK) break;

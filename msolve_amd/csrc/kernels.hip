@@ -1025,6 +1025,108 @@ __device__ __forceinline__ real dpp_wave(real old, real src)
 }
 constexpr int kDppWaveShl1 = 0x130, kDppWaveShr1 = 0x138;
 
+// One row of the symmetric product (pcg_a_sym_rows) per lane.
+template <typename real>
+struct SymRow {
+    const MSA_GLOBAL real *z, *po, *val;
+    real beta;
+    int sy, sz, nb1, rr, brc;
+
+    // the roundings are written out: every kernel gives the same bits
+    static __device__ __forceinline__ real fma3(real a, real b, real c)
+    {
+        if constexpr (sizeof(real) == 4)
+            return __builtin_fmaf(a, b, c);
+        else
+            return __builtin_fma(a, b, c);
+    }
+    static __device__ __forceinline__ real dot(real a0, real a1, real a2, real b0, real b1, real b2)
+    {
+        return fma3(a2, b2, fma3(a0, b0, a1 * b1));
+    }
+
+    // p at stencil column m = (dy+1) + 3 (dz+1): c[0] at x - 1, c[1] at x,
+    // c[2] at x + 1
+    __device__ __forceinline__ void column(int m, real (&c)[3][3]) const
+    {
+        using V3 = vec3<real>;
+        const int mo = sy * (m % 3 - 1) + sz * (m / 3 - 1);
+        const V3 zc = ld3(z, min(max(brc + mo, 0), nb1));
+        const V3 pc = ld3(po, min(max(brc + mo, 0), nb1));
+        const real own[3] = {fma3(beta, pc.x, zc.x), fma3(beta, pc.y, zc.y), fma3(beta, pc.z, zc.z)};
+        real edge[3] = {0, 0, 0};
+        if (rr == 0 || rr == 63) {
+            const int r1 = min(max(brc + mo + (rr == 0 ? -1 : 1), 0), nb1);
+            const V3 ze = ld3(z, r1), pe = ld3(po, r1);
+            edge[0] = fma3(beta, pe.x, ze.x);
+            edge[1] = fma3(beta, pe.y, ze.y);
+            edge[2] = fma3(beta, pe.z, ze.z);
+        }
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            c[1][d] = own[d];
+            c[0][d] = dpp_wave<kDppWaveShr1>(edge[d], own[d]);
+            c[2][d] = dpp_wave<kDppWaveShl1>(edge[d], own[d]);
+        }
+    }
+
+    // the block of stencil position n times v (transposed for n < 13)
+    __device__ __forceinline__ void term(int n, const real (&v)[3], real (&r)[3]) const
+    {
+        const int su = n >= 13 ? n : 26 - n;
+        const int off = (n % 3 - 1) + sy * ((n / 3) % 3 - 1) + sz * (n / 9 - 1);
+        const int j = n >= 13 ? brc : brc + off;
+        const int jc = max(j, 0);
+        real m[9];
+        load_block<real, 1, false>(val, (size_t)(jc >> 6) * 27 + su, jc & 63, 0, m);
+        const real w0 = j >= 0 ? v[0] : (real)0, w1 = j >= 0 ? v[1] : (real)0,
+                   w2 = j >= 0 ? v[2] : (real)0;
+        if (n < 13) {
+            r[0] = dot(m[0], m[3], m[6], w0, w1, w2);
+            r[1] = dot(m[1], m[4], m[7], w0, w1, w2);
+            r[2] = dot(m[2], m[5], m[8], w0, w1, w2);
+        } else {
+            r[0] = dot(m[0], m[1], m[2], w0, w1, w2);
+            r[1] = dot(m[3], m[4], m[5], w0, w1, w2);
+            r[2] = dot(m[6], m[7], m[8], w0, w1, w2);
+        }
+    }
+
+    // the middle column: pair k = 1 and the diagonal d, both from zero; the
+    // row's own p
+    __device__ __forceinline__ void middle(real (&a)[3], real (&d)[3], real (&own)[3]) const
+    {
+        real c[3][3], t12[3], t14[3];
+        column(4, c);
+        term(14, c[2], t14);
+        term(12, c[0], t12);
+        term(13, c[1], d);
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            a[k] = 0;
+            a[k] += t14[k] + t12[k];
+            own[k] = c[1][k];
+        }
+    }
+
+    // column m and its mirror: the pairs by ascending distance, dx = 2, 1, 0
+    __device__ __forceinline__ void pairs(int m, real (&s)[3][3]) const
+    {
+        real cl[3][3], ch[3][3], rl[3][3], rh[3][3];
+        column(m, cl);
+        column(8 - m, ch);
+#pragma unroll
+        for (int dx = 2; dx >= 0; dx--) {
+            term(3 * m + dx, cl[dx], rl[dx]);
+            term(26 - 3 * m - dx, ch[2 - dx], rh[dx]);
+        }
+#pragma unroll
+        for (int dx = 2; dx >= 0; dx--)
+#pragma unroll
+            for (int k = 0; k < 3; k++) s[dx][k] = rh[dx][k] + rl[dx][k];
+    }
+};
+
 // Rows [s0, s1) slices of a stencil class (one-sample tiles) in the
 // symmetric product q = K p, p = z + beta p_old: every row's 14 upper
 // blocks (slots 13..26) times p at br + off, and its 13 lower blocks as the
@@ -1063,90 +1165,29 @@ __device__ __forceinline__ real pcg_a_sym_rows(const ClassDev &C, int s0, int s1
                                                MSA_GLOBAL real *__restrict__ q,
                                                const MSA_GLOBAL real *__restrict__ val)
 {
-    using V3 = vec3<real>;
-    const int sy = C.sym_sy, sz = C.sym_sz, nb1 = C.nb - 1;
     real pq = 0;
     if (!act) return pq;  // one sample per tile: uniform over the wave
+    SymRow<real> R{z, po, val, beta, C.sym_sy, C.sym_sz, C.nb - 1, rr, 0};
     for (int slice = s0 + wave; slice < s1; slice += kWaves) {
         const int br = slice * 64 + rr;
-        const int brc = min(br, nb1);
-        // p at stencil column m = (dy+1) + 3 (dz+1): c[0] at x - 1, c[1] at x,
-        // c[2] at x + 1
-        auto column = [&](int m, real (&c)[3][3]) {
-            const int mo = sy * (m % 3 - 1) + sz * (m / 3 - 1);
-            const V3 zc = ld3(z, min(max(brc + mo, 0), nb1));
-            const V3 pc = ld3(po, min(max(brc + mo, 0), nb1));
-            const real own[3] = {zc.x + beta * pc.x, zc.y + beta * pc.y, zc.z + beta * pc.z};
-            real edge[3] = {0, 0, 0};
-            if (rr == 0 || rr == 63) {
-                const int r1 = min(max(brc + mo + (rr == 0 ? -1 : 1), 0), nb1);
-                const V3 ze = ld3(z, r1), pe = ld3(po, r1);
-                edge[0] = ze.x + beta * pe.x;
-                edge[1] = ze.y + beta * pe.y;
-                edge[2] = ze.z + beta * pe.z;
-            }
-#pragma unroll
-            for (int d = 0; d < 3; d++) {
-                c[1][d] = own[d];
-                c[0][d] = dpp_wave<kDppWaveShr1>(edge[d], own[d]);
-                c[2][d] = dpp_wave<kDppWaveShl1>(edge[d], own[d]);
-            }
-        };
-        // the block of stencil position n times v (transposed for n < 13)
-        auto term = [&](int n, const real (&v)[3], real (&r)[3]) {
-            const int su = n >= 13 ? n : 26 - n;
-            const int off = (n % 3 - 1) + sy * ((n / 3) % 3 - 1) + sz * (n / 9 - 1);
-            const int j = n >= 13 ? brc : brc + off;
-            const int jc = max(j, 0);
-            real m[9];
-            load_block<real, 1, false>(val, (size_t)(jc >> 6) * 27 + su, jc & 63, 0, m);
-            const real w0 = j >= 0 ? v[0] : (real)0, w1 = j >= 0 ? v[1] : (real)0,
-                       w2 = j >= 0 ? v[2] : (real)0;
-            if (n < 13) {
-                r[0] = m[0] * w0 + m[3] * w1 + m[6] * w2;
-                r[1] = m[1] * w0 + m[4] * w1 + m[7] * w2;
-                r[2] = m[2] * w0 + m[5] * w1 + m[8] * w2;
-            } else {
-                r[0] = m[0] * w0 + m[1] * w1 + m[2] * w2;
-                r[1] = m[3] * w0 + m[4] * w1 + m[5] * w2;
-                r[2] = m[6] * w0 + m[7] * w1 + m[8] * w2;
-            }
-        };
+        R.brc = min(br, R.nb1);
         real a[3], d[3], own[3];
-        {
-            real c[3][3], t12[3], t14[3];
-            column(4, c);
-            term(14, c[2], t14);
-            term(12, c[0], t12);
-            term(13, c[1], d);
-#pragma unroll
-            for (int k = 0; k < 3; k++) {
-                a[k] = 0;
-                a[k] += t14[k] + t12[k];
-                own[k] = c[1][k];
-            }
-        }
+        R.middle(a, d, own);
 #pragma unroll 1
         for (int m = 3; m >= 0; m--) {
-            real cl[3][3], ch[3][3], rl[3][3], rh[3][3];
-            column(m, cl);
-            column(8 - m, ch);
-#pragma unroll
-            for (int dx = 2; dx >= 0; dx--) {
-                term(3 * m + dx, cl[dx], rl[dx]);
-                term(26 - 3 * m - dx, ch[2 - dx], rh[dx]);
-            }
+            real s[3][3];
+            R.pairs(m, s);
 #pragma unroll
             for (int dx = 2; dx >= 0; dx--)
 #pragma unroll
-                for (int k = 0; k < 3; k++) a[k] += rh[dx][k] + rl[dx][k];
+                for (int k = 0; k < 3; k++) a[k] += s[dx][k];
         }
 #pragma unroll
         for (int k = 0; k < 3; k++) a[k] += d[k];
         if (br < C.nb) {
             st3(pn, br, own[0], own[1], own[2]);
             st3(q, br, a[0], a[1], a[2]);
-            pq += own[0] * a[0] + own[1] * a[1] + own[2] * a[2];
+            pq += SymRow<real>::dot(own[0], own[1], own[2], a[0], a[1], a[2]);
         }
     }
     return pq;
@@ -1304,6 +1345,80 @@ __global__ __launch_bounds__(256) void k_pcg_a(const ClassDev *__restrict__ cls,
     const int item = xcd_item(nitems);
     if (item < 0) return;
     pcg_a_item<real, T, U>(cls, items[item], pbuf, fz);
+}
+
+// The symmetric product in chunks of one slice (small batches): the four
+// waves share the slice, each forming the pairs of one column and its mirror,
+// and the wave of column 3 adds them up in pcg_a_sym_rows' order (same bits).
+// A wave of k_pcg_a streams its slice's 124 KB of FP64 values alone, four of
+// them on one CU, which is what a 10^3 product (19 slices) waits for: an
+// iteration takes 16.3 us so and 11.5 us with the slices on 19 CUs.
+template <typename real>
+__global__ __launch_bounds__(256) void k_pcg_a_split(const ClassDev *__restrict__ cls,
+                                                     const int4 *__restrict__ items, int nitems,
+                                                     int pbuf, PcgFuse fz)
+{
+    const int item = xcd_item(nitems);
+    if (item < 0) return;
+    __shared__ real part[3][9][64];
+    const int4 it = items[item];
+    const ClassDev &C = cls[it.x];
+    const int tile = it.y, slice = it.z;  // one sample per tile
+    const int lane = threadIdx.x & 63;
+    const int m = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    bool act = tile < C.nsamp;
+    real beta = 0;
+    if (act) {
+        if (fz.fold) {
+            const SampleState S = reduced_state(C, tile, slice == 0, fz);
+            act = S.active;
+            beta = (real)S.beta;
+        } else {
+            act = C.st[tile].active;
+            beta = (real)C.st[tile].beta;
+        }
+    }
+    double *out = C.partial + ((size_t)tile * C.nchunks + slice) * 3 + fz.slot;
+    if (!act) {  // the same in every wave
+        if (threadIdx.x == 0) *out = 0.0;
+        return;
+    }
+    const size_t vb = (size_t)tile * C.tile_vec;
+    const int br = slice * 64 + lane;
+    SymRow<real> R{gbl((const real *)C.z + vb),
+                   gbl((const real *)(pbuf ? C.p1 : C.p0) + vb),
+                   gbl((const real *)C.val + (size_t)tile * C.tile_vals),
+                   beta, C.sym_sy, C.sym_sz, C.nb - 1, lane, min(br, C.nb - 1)};
+    real s[3][3], a[3], d[3], own[3];
+    R.pairs(m, s);
+    if (m == 3) {
+        R.middle(a, d, own);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 9; e++) part[m][e][lane] = s[e / 3][e % 3];
+    }
+    __syncthreads();
+    if (m != 3) return;
+#pragma unroll
+    for (int dx = 2; dx >= 0; dx--)
+#pragma unroll
+        for (int k = 0; k < 3; k++) a[k] += s[dx][k];
+#pragma unroll
+    for (int mm = 2; mm >= 0; mm--)
+#pragma unroll
+        for (int dx = 2; dx >= 0; dx--)
+#pragma unroll
+            for (int k = 0; k < 3; k++) a[k] += part[mm][3 * dx + k][lane];
+#pragma unroll
+    for (int k = 0; k < 3; k++) a[k] += d[k];
+    real pq = 0;
+    if (br < C.nb) {
+        st3(gbl((real *)(pbuf ? C.p0 : C.p1) + vb), br, own[0], own[1], own[2]);
+        st3(gbl((real *)C.q + vb), br, a[0], a[1], a[2]);
+        pq += SymRow<real>::dot(own[0], own[1], own[2], a[0], a[1], a[2]);
+    }
+    const double w = reduce_rows<1>((double)pq);
+    if (lane == 0) *out = w;
 }
 
 // The same step for box-grid classes whose product is matrix-free
@@ -5249,6 +5364,18 @@ hipError_t launch_pcg_a(hipStream_t s, bool mixed, int T, int U, const ClassDev 
     }
     if (U != 3) return hipErrorInvalidValue;  // lane tiles T > 1 use groups of 3 slots
     MSA_PCG_LAUNCH(k_pcg_a, d_cls, items, nitems, pbuf, fz);
+}
+
+hipError_t launch_pcg_a_split(hipStream_t s, bool mixed, const ClassDev *d_cls, const int4 *items,
+                              int nitems, int pbuf, const PcgFuse &fz)
+{
+    if (nitems <= 0) return hipSuccess;
+    const dim3 grid(xcd_grid(nitems)), block(256);
+    if (mixed)
+        hipLaunchKernelGGL(k_pcg_a_split<float>, grid, block, 0, s, d_cls, items, nitems, pbuf, fz);
+    else
+        hipLaunchKernelGGL(k_pcg_a_split<double>, grid, block, 0, s, d_cls, items, nitems, pbuf, fz);
+    return hipGetLastError();
 }
 
 hipError_t launch_pcg_a_mf(hipStream_t s, bool mixed, bool dyn, const ClassDev *d_cls,

@@ -354,6 +354,12 @@ struct PcgFuse {
     int fold = 0, slot = 0;
     ReduceArgs red{};
 };
+// Most slices of a MIXED batch (FP64: half) that gets one-slice chunks and the
+// split product, two to four workgroups a CU.  us per Jacobi iteration, chunks
+// of four / of one: FP64 10^3 (19 slices) 16.3 / 11.5, 24^3 (235) 16.5 / 11.8,
+// 2 x 24^3 (470) 19.8 / 15.8, 16 x 14^3 (800) 22.0 / 23.0; MIXED 4 x 20^3
+// (552) 17.7 / 14.9, 7 x 20^3 (966) 19.9 / 18.6, 12 x 20^3 (1656) 24.4 / 26.9.
+constexpr int kSmallSlices = 1024;
 constexpr int kFoldChunks = 256;  // most chunks of a sample whose reductions fold
 
 enum KernelKind { KK_SPMV = 0, KK_UPDATE = 1, KK_ASSEMBLE = 2, KK_RES64 = 3, KK_OTHER = 4, KK_MG = 5 };
@@ -399,6 +405,9 @@ hipError_t launch_pcg_init(hipStream_t s, bool mixed, int T, const ClassDev *d_c
 // U: slots per group of a row (1..4 at T = 1, 3 for T > 1)
 hipError_t launch_pcg_a(hipStream_t s, bool mixed, int T, int U, const ClassDev *d_cls,
                         const int4 *items, int nitems, int pbuf, const PcgFuse &fz);
+// the same product for symmetric classes of one-slice chunks
+hipError_t launch_pcg_a_split(hipStream_t s, bool mixed, const ClassDev *d_cls, const int4 *items,
+                              int nitems, int pbuf, const PcgFuse &fz);
 // need_due 1: the samples due for a replacement, 0: every refining one
 hipError_t launch_residual64_mf_box(hipStream_t s, bool dyn, const ClassDev *d_cls,
                                    const int4 *items, int nitems, int need_due);

@@ -98,3 +98,39 @@ def test_mixed_residual_without_hierarchy(ctx, shape, lengths, roller, dyn):
         mesh.close()
     for a, c in zip(*out):
         assert np.linalg.norm(a - c) <= 1e-7 * np.linalg.norm(c)
+
+
+@pytest.mark.parametrize("precision", [L.MSA_FP64, L.MSA_MIXED])
+@pytest.mark.parametrize("shape", [(1, 1, 1), (4, 4, 3), (63, 1, 1), (64, 2, 1), (3, 9, 70)])
+def test_small_batch_forms(ctx, shape, precision):
+    """One-slice chunks with the split product and folded reductions (a batch
+    of one sample) against the form of larger batches, the sample repeated
+    beside others past the limit, and the persistent launch.  Same terms in
+    the same order but for the partial sums, so the solves agree to their
+    stopping residual of 1e-11 times the condition (below 1e5)."""
+    xyz, conn = box_mesh(*shape, *[float(v) for v in shape])
+    cons = np.zeros((xyz.shape[0], 3), bool)
+    cons[xyz[:, 1] < 1e-12] = True
+    dof, nf = msa.enumerate_dofs(cons)
+    rng = np.random.default_rng(6)
+    f, E = rng.standard_normal(nf), rng.uniform(1.0, 3.0, conn.shape[0])
+    slices = -(-(nf // 3) // 64)
+    out = []
+    for ns, persistent in ((1, False), (1, True), (1024 // slices + 1, False)):
+        mesh = msa.Mesh(ctx, xyz, conn, dof, nf)
+        b = msa.Batch(ctx, [mesh], [ns], precision, 1)
+        b.set_matrix_free_product(False)
+        b.set_persistent(persistent)
+        b.set_modulus(0, np.tile(E, (ns, 1)))
+        b.set_rhs(0, f)
+        b.assemble(0.3)
+        b.solve(tol=1e-11, max_it=5000, graph_iters=8)
+        assert (b.stats(0)["status"] == msa.MSA_OK).all()
+        out.append((b.solution(0, 0), b.solution(0, ns - 1)))
+        b.close()
+        mesh.close()
+    if precision == L.MSA_FP64:  # the persistent launch serves FP64 and inner solves
+        assert np.array_equal(out[0][0], out[1][0])
+    assert np.array_equal(*out[2])
+    for o in out[1:]:
+        assert np.linalg.norm(o[0] - out[0][0]) <= 1e-6 * np.linalg.norm(out[0][0])
