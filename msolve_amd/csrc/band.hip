@@ -446,14 +446,9 @@ __device__ __forceinline__ bool served(const ClassDev &C, int smp, int mode)
 // side lives in LDS (slot = block modulo the window), every wave holds 64
 // rows of the current panel in registers, loaded before the diagonal product
 // they wait for.  sweeps: bit 0 forward, bit 1 backward.
-__global__ __launch_bounds__(64 * kSweepWaves) void k_band_sweep_one(const ClassDev *__restrict__ cp,
-                                                                     int mode, int sweeps)
+__device__ __forceinline__ void sweep_sample(const ClassDev &C, int smp, int sweeps,
+                                             double *yw /* bW */, double *xb /* kBandNB */)
 {
-    extern __shared__ double yw[];  // bW
-    __shared__ double xb[kBandNB];
-    const ClassDev &C = *cp;
-    const int smp = blockIdx.x;
-    if (!served(C, smp, mode)) return;
     const int n = C.bn, W = C.bW, nblk = (n + kBandNB - 1) / kBandNB, nwb = W / kBandNB;
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -513,6 +508,47 @@ __global__ __launch_bounds__(64 * kSweepWaves) void k_band_sweep_one(const Class
             if (wave == kSweepWaves - 1) yw[slot + lane] = yin;
             __syncthreads();
         }
+    }
+}
+
+__global__ __launch_bounds__(64 * kSweepWaves) void k_band_sweep_one(const ClassDev *__restrict__ cp,
+                                                                     int mode, int sweeps)
+{
+    extern __shared__ double yw[];
+    __shared__ double xb[kBandNB];
+    const ClassDev &C = *cp;
+    const int smp = blockIdx.x;
+    if (!served(C, smp, mode)) return;
+    sweep_sample(C, smp, sweeps, yw, xb);
+}
+
+// Coarsest multigrid levels, all classes of the batch at once: items are
+// (class, sample), one workgroup each, which also moves the level's
+// right-hand side into band order and the solution back.  A sample's sweeps
+// are a serial chain of 2.8 us a block, so a batch's classes one after the
+// other waited for the sum of their chains instead of the longest: 17 samples
+// over four meshes (coarsest chains of 53, 23 and 9 blocks) 31.1 -> 26.4 ms.
+template <typename real>
+__global__ __launch_bounds__(64 * kSweepWaves) void k_mg_band_solve(const ClassDev *__restrict__ cls,
+                                                                    const int2 *__restrict__ items,
+                                                                    int T, int mode)
+{
+    extern __shared__ double yw[];
+    __shared__ double xb[kBandNB];
+    const ClassDev &C = cls[items[blockIdx.x].x];
+    const int smp = items[blockIdx.x].y, n = C.bn, t = threadIdx.x;
+    if (!served(C, smp, mode)) return;
+    const size_t vb = (size_t)(smp / T) * C.tile_vec + smp % T;
+    GLOB double *y = glob(C.by + (size_t)smp * n);
+    const GLOB real *r = glob((const real *)C.r + vb);
+    GLOB real *z = glob((real *)C.z + vb);
+    for (int i = t; i < n; i += 64 * kSweepWaves) y[i] = (double)r[(size_t)C.bperm[i] * T];
+    __syncthreads();
+    sweep_sample(C, smp, 3, yw, xb);
+    __syncthreads();
+    for (int row = t; row < 3 * C.nb; row += 64 * kSweepWaves) {
+        const int i = C.binv[row];
+        z[(size_t)row * T] = i >= 0 ? (real)y[i] : (real)0;
     }
 }
 
@@ -627,6 +663,20 @@ hipError_t launch_band_sweep_one(hipStream_t s, const ClassDev *cp, int nsamp, i
     if (!band_one_launch(bn, bW)) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_band_sweep_one, dim3(nsamp), dim3(64 * kSweepWaves), bW * sizeof(double), s,
                        cp, mode, sweeps);
+    return hipGetLastError();
+}
+
+hipError_t launch_mg_band_solve(hipStream_t s, bool mixed, int T, const ClassDev *d_cls,
+                                const int2 *items, int nitems, int max_bW, int mode)
+{
+    if (nitems <= 0) return hipSuccess;
+    if (max_bW > kBandOneMax) return hipErrorInvalidValue;
+    const dim3 grid(nitems), block(64 * kSweepWaves);
+    const size_t lds = max_bW * sizeof(double);
+    if (mixed)
+        hipLaunchKernelGGL(k_mg_band_solve<float>, grid, block, lds, s, d_cls, items, T, mode);
+    else
+        hipLaunchKernelGGL(k_mg_band_solve<double>, grid, block, lds, s, d_cls, items, T, mode);
     return hipGetLastError();
 }
 

@@ -178,6 +178,11 @@ struct msa_batch {
     int4 *mf_box_items = nullptr;
     int n_mf_box_items = 0;
     std::vector<int> mg_coarsest;       // class table indices of the coarsest levels
+    // their solves, (class, sample): dense inverses, one-launch bands; the
+    // classes of wide bands
+    int2 *mg_co_dense = nullptr, *mg_co_band = nullptr;
+    int mg_nco_dense = 0, mg_nco_band = 0, mg_co_dense_n = 0, mg_co_band_W = 0;
+    std::vector<int> mg_co_wide;
     int mg_max_levels = 0;              // max_levels the hierarchy was built with
     size_t d_cls_cap = 0;               // ClassDev entries allocated at d_cls
     bool mg_ready = false;              // level matrices match the assembled classes
@@ -1523,6 +1528,34 @@ int mg_build(msa_batch *b, int max_levels)
         if (d > 0) MSA_TRY(items_to_device(b, re, &b->mg_restr[d], &b->mg_nrestr[d]));
     }
     MSA_TRY(items_to_device(b, all, &b->mg_lv_items, &b->mg_nlv_items));
+    {
+        std::vector<int> order = b->mg_coarsest;  // the longest chains start first
+        std::stable_sort(order.begin(), order.end(),
+                         [&](int i, int k) { return tab(b, i).dev.bn > tab(b, k).dev.bn; });
+        std::vector<int2> dense, band;
+        b->mg_co_dense_n = b->mg_co_band_W = 0;
+        b->mg_co_wide.clear();
+        for (int ci : order) {
+            const ClassHost &C = tab(b, ci);
+            const bool inv = C.dev.binvd != nullptr;
+            if (!inv && !band_one_launch(C.dev.bn, C.dev.bW)) {
+                b->mg_co_wide.push_back(ci);
+                continue;
+            }
+            if (inv)
+                b->mg_co_dense_n = std::max(b->mg_co_dense_n, C.dev.bn);
+            else
+                b->mg_co_band_W = std::max(b->mg_co_band_W, C.dev.bW);
+            for (int k = 0; k < C.nsamp; k++) (inv ? dense : band).push_back(make_int2(ci, k));
+        }
+        const int2 *p = nullptr;
+        MSA_TRY(upload_vec(b, dense, &p));
+        b->mg_co_dense = (int2 *)p;
+        MSA_TRY(upload_vec(b, band, &p));
+        b->mg_co_band = (int2 *)p;
+        b->mg_nco_dense = (int)dense.size();
+        b->mg_nco_band = (int)band.size();
+    }
     std::vector<int4> gall;
     for (size_t l = 0; l < b->lv.size(); l++)
         class_group_items(b->lv[l], (int)(b->cls.size() + l), gall);
@@ -1855,14 +1888,17 @@ int mg_vcycle(msa_batch *b, int pbuf, int mode)
                                       pbuf, mode);
         }));
     }
-    for (int ci : b->mg_coarsest) {
+    MSA_TRY(timed(b, KK_OTHER, [&] {
+        const hipError_t e = launch_mg_dense_solve(s, mx, T, b->d_cls, b->mg_co_dense,
+                                                   b->mg_nco_dense, b->mg_co_dense_n, mode);
+        return e != hipSuccess ? e
+                               : launch_mg_band_solve(s, mx, T, b->d_cls, b->mg_co_band,
+                                                      b->mg_nco_band, b->mg_co_band_W, mode);
+    }));
+    for (int ci : b->mg_co_wide) {
         ClassHost &C = tab(b, ci);
         const ClassDev *cp = b->d_cls + ci;
         const int n = C.dev.bn, W = C.dev.bW, ns = C.nsamp;
-        if (C.dev.binvd) {
-            MSA_TRY(timed(b, KK_OTHER, [&] { return launch_mg_dense_solve(s, mx, T, cp, ns, n, mode); }));
-            continue;
-        }
         MSA_TRY(timed(b, KK_OTHER, [&] { return launch_mg_band_in(s, mx, T, cp, ns, n, mode); }));
         MSA_TRY(band_sweeps(b, cp, n, W, ns, mode));
         MSA_TRY(timed(b, KK_OTHER, [&] { return launch_mg_band_out(s, mx, T, cp, ns, 3 * C.dev.nb, mode); }));

@@ -5060,14 +5060,15 @@ __global__ __launch_bounds__(64) void k_band_inverse(const ClassDev *__restrict_
 }
 
 // Coarsest solve by the dense inverse: z[bperm[i]] = sum_j X[j][i] b[bperm[j]]
-// (X symmetric: lane i reads row j at column i, so loads are coalesced).
+// (X symmetric: lane i reads row j at column i, so loads are coalesced).  Items
+// are (class, sample) of all classes, grid.x covers the largest order.
 template <typename real, int T>
-__global__ __launch_bounds__(64) void k_mg_dense_solve(const ClassDev *__restrict__ cp, int mode)
+__global__ __launch_bounds__(64) void k_mg_dense_solve(const ClassDev *__restrict__ cls,
+                                                       const int2 *__restrict__ items, int mode)
 {
-    const ClassDev &C = *cp;
-    const int smp = blockIdx.y;
-    if (!mg_act(C.mg_st[smp], mode)) return;
-    const int n = C.bn;
+    const ClassDev &C = cls[items[blockIdx.y].x];
+    const int smp = items[blockIdx.y].y, n = C.bn;
+    if ((int)blockIdx.x * 64 >= n || !mg_act(C.mg_st[smp], mode)) return;
     const int i = blockIdx.x * 64 + threadIdx.x;
     const int tile = smp / T, s = smp % T;
     const size_t vb = (size_t)tile * C.tile_vec;
@@ -5860,17 +5861,17 @@ hipError_t launch_band_inverse(hipStream_t s, const ClassDev *cp, int nsamp, int
     return hipGetLastError();
 }
 
-hipError_t launch_mg_dense_solve(hipStream_t s, bool mixed, int T, const ClassDev *cp, int nsamp,
-                                 int bn, int mode)
+hipError_t launch_mg_dense_solve(hipStream_t s, bool mixed, int T, const ClassDev *d_cls,
+                                 const int2 *items, int nitems, int max_bn, int mode)
 {
-    if (bn <= 0) return hipSuccess;
-    const dim3 grid((bn + 63) / 64, nsamp);
+    if (nitems <= 0) return hipSuccess;
+    const dim3 grid((max_bn + 63) / 64, nitems);
     if (mixed) {
-        MSA_DISPATCH_T(T, hipLaunchKernelGGL((k_mg_dense_solve<float, TT>), grid, dim3(64), 0, s, cp,
-                                             mode));
+        MSA_DISPATCH_T(T, hipLaunchKernelGGL((k_mg_dense_solve<float, TT>), grid, dim3(64), 0, s,
+                                             d_cls, items, mode));
     } else {
-        MSA_DISPATCH_T(T, hipLaunchKernelGGL((k_mg_dense_solve<double, TT>), grid, dim3(64), 0, s, cp,
-                                             mode));
+        MSA_DISPATCH_T(T, hipLaunchKernelGGL((k_mg_dense_solve<double, TT>), grid, dim3(64), 0, s,
+                                             d_cls, items, mode));
     }
     return hipGetLastError();
 }

@@ -497,8 +497,11 @@ hipError_t launch_residual64_mf(hipStream_t s, const ClassDev *d_cls, const int4
                                 int need_due);
 // coarsest multigrid level: dense inverse from the band factor, and its use
 hipError_t launch_band_inverse(hipStream_t s, const ClassDev *cp, int nsamp, int bn);
-hipError_t launch_mg_dense_solve(hipStream_t s, bool mixed, int T, const ClassDev *cp, int nsamp,
-                                 int bn, int mode);
+hipError_t launch_mg_dense_solve(hipStream_t s, bool mixed, int T, const ClassDev *d_cls,
+                                 const int2 *items, int nitems, int max_bn, int mode);
+// coarsest levels of narrow bands, items (class, sample)
+hipError_t launch_mg_band_solve(hipStream_t s, bool mixed, int T, const ClassDev *d_cls,
+                                const int2 *items, int nitems, int max_bW, int mode);
 hipError_t launch_mg_load(hipStream_t s, bool mixed, int T, const ClassDev *cp, const double *src,
                           size_t nrows, int tile, int lane);
 hipError_t launch_band_scatter_any(hipStream_t s, bool mixed, int T, const ClassDev *d_cls,
