@@ -1201,10 +1201,12 @@ void class_run_items(const ClassHost &C, int ci, std::vector<int4> &out, int run
 //
 // FP64, why: the stored product is bound by its values (64 x 32^3: 0.54 ms
 // per launch, 64^3: 65 us), the matrix-free one reads 24 bytes a node and
-// runs on the FP64 VALU (98 + 32 us with its p pass, 17.5 + 6 us).  Under
-// 128 chunks every kernel lasts as long as its launch, and the p pass is one
-// launch more: us per iteration, stored / matrix-free, 24^3 (60 chunks)
-// 21.9 / 24.6, 16 x 16^3 (304) 34.2 / 24.1, 32^3 (133) 27.2 / 20.1.
+// runs on the FP64 VALU (98 + 32 us with its p pass, 17.5 + 6 us).  In small
+// batches every kernel lasts as long as its launch, and the p pass is one
+// launch more: us per iteration, stored / matrix-free, by chunks of four
+// slices, 24^3 (59) 11.9 / 14.2, 6 x 16^3 (114) 14.5 / 15.2, 2 x 24^3 (118)
+// 15.8 / 15.7, 7 x 16^3 (133) 16.1 / 15.4, 32^3 (137) 20.4 / 15.2, 16 x 16^3
+// (304) 29.4 / 18.5.
 bool mf64_large(const msa_batch *b) { return !is_mixed(b) && b->chunks4 >= 128; }
 
 // MIXED batches that form the FP64 residual matrix-free also without a

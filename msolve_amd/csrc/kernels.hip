@@ -7,8 +7,9 @@
 // rows (rr) times T samples (s).  Every value load reads 64 consecutive words;
 // every gathered vector load reads T consecutive words of one block column.
 // Per-sample dot products are reduced wave -> workgroup -> a partial per
-// work item; k_reduce, launched next, sums the partials of a (class, tile) in
-// a fixed order, so results do not depend on scheduling.
+// work item; k_reduce, launched next, or the next phase (reduced_state) sums
+// the partials of a (class, tile) in a fixed order, so results do not depend
+// on scheduling.
 #include <algorithm>
 #include <cmath>
 
