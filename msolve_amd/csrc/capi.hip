@@ -2734,6 +2734,8 @@ int msa_batch_set_dynamics(msa_batch *b, double rho, double rayleigh_alpha, doub
         D.cM = (c.a0 + c.a1 * rayleigh_alpha) * rho;  // a0 M + a1 alphaR M
         D.rho = rho;
     }
+    // the captured iteration blocks hold kernels of the static matrix
+    if (!b->dyn) drop_graph(b);
     b->dyn = true;
     b->assembled = false;
     return upload_class_table(b);
