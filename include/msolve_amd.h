@@ -255,7 +255,8 @@ int msa_batch_set_symmetric_product(msa_batch *b, int enable);
  *   matrix in FP32; the FP64 residual replacements (also matrix-free) fix
  *   the accuracy;
  *   FP64 with any preconditioner, in FP64 throughout, on grids whose cells
- *   are equal up to the rounding of the coordinates, in batches of at least
+ *   are equal up to rounding (4 units in the last place of the grid's extent
+ *   per axis: not grids far from the origin), in batches of at least
  *   128 chunks of 256 block rows (below that the launches dominate and the
  *   stored product needs one less), unless matrices were loaded
  *   (msa_batch_set_matrix_csr) or the full image is selected
@@ -458,8 +459,8 @@ int msa_batch_set_matrix_cores(msa_batch *b, int enable);
  * These count the FP32 form: MIXED batches with one-sample tiles on grids of
  * equal, equally oriented cells (all elements share one element matrix): K v
  * from the cell moduli and that matrix, without reading the stored values.
- * FP64 batches report 0; on box grids of cells equal up to coordinate
- * rounding (one-sample tiles, upper-triangle storage) their smoothing
+ * FP64 batches report 0; on box grids of cells equal up to
+ * rounding (msa_batch_set_matrix_free_product; one-sample tiles, upper-triangle storage) their smoothing
  * products have the same form in FP64. */
 int msa_batch_mg_info(msa_batch *b, int cls, long long *info);
 /* Upper end lam of each level's Chebyshev smoothing interval [lam/ratio,

@@ -577,7 +577,7 @@ int launch_iteration_pair(msa_batch *b, int pbuf, double tol, int max_it, double
 
 // Classes an element-by-element (coloured) launch leaves to a matrix-free
 // kernel: none; those whose replacement residual is matrix-free; of these
-// the ones whose cells are equal up to coordinate rounding (residual at the
+// the ones whose cells are equal up to rounding (GridInfo::exact; residual at the
 // start of a Newmark step); the box grids among the latter (its right-hand
 // side).
 enum ColourSkip { SKIP_NONE = 0, SKIP_MF, SKIP_MF_EXACT, SKIP_MF_RHS };
@@ -1299,8 +1299,8 @@ int assemble_items(msa_batch *b, const int4 *items, int nitems, const int4 *gite
 // Tables of the matrix-free products for a class on a uniform structured
 // grid (one-sample tiles); other classes keep the stored values.  FP64
 // batches take box grids whose cells are equal up to the rounding of the
-// coordinates: the shared element matrix then is every element's to FP64
-// rounding (MIXED: cells equal to 1e-9, FP32 products).
+// grid's extent (GridInfo::exact): the shared element matrix then is every
+// element's to FP64 rounding (MIXED: cells equal to 1e-9, FP32 products).
 int mf_setup(msa_batch *b, ClassHost &C, bool residual_only)
 {
     const GridInfo &g = C.grid;

@@ -132,7 +132,7 @@ struct GridInfo {
     std::vector<int> gblock, cell_elem, bpos;
     int corner_node[8] = {0, 0, 0, 0, 0, 0, 0, 0};
     int cell_identity = 0;  // element number == cell number
-    int exact = 0;          // equal cells up to the rounding of the coordinates
+    int exact = 0;          // equal cells up to the rounding of the grid's own extent
     int box = 0;            // the blocks are exactly the grid points of [box_lo, box_hi],
     int box_lo[3] = {0, 0, 0}, box_hi[3] = {0, 0, 0};  // numbered lexicographically
 };
@@ -255,14 +255,14 @@ struct ClassDev {
     // mf64)
     int mf_pcg;
     // FP64 batches, one-sample tiles: a box grid whose cells are equal up to
-    // the rounding of the coordinates (mf stays 0; the mf_ tables and mf_k64
+    // the rounding of its extent (GridInfo::exact; mf stays 0; the mf_ tables and mf_k64
     // are set).  mf_free: every block fully free.
     int mf64, mf_free;
     // MIXED: the FP64 residual matrix-free without the multigrid tables (mf
     // stays 0; a box grid of equal cells, the tables as for mf64); mf_r: the
     // class takes it in this solve (mf_res, or mf with multigrid set up)
     int mf_res, mf_r;
-    int mf_exact;  // mf / mf64 class whose cells are equal up to coordinate rounding
+    int mf_exact;  // mf / mf64 class whose cells are equal up to rounding (GridInfo::exact)
     // FP64 copy of the stored values (same layout as a one-sample-tile FP64
     // batch) for the coarsest multigrid level of a MIXED batch: the band
     // factor is computed from these, not from the FP32 values (null: none)

@@ -197,3 +197,55 @@ def test_fp64_cycle_forms(ctx, grid, dyn):
         assert rel(z[0][s], z[1][s]) < 1e-11
     b.close()
     mesh.close()
+
+
+def residual_launches(b, run):
+    """FP64 residual and right-hand side launches of run() (eager)."""
+    b.set_kernel_timing(True)
+    run()
+    n = b.kernel_timing()["residual64"]["launches"]
+    b.set_kernel_timing(False)
+    return n
+
+
+@pytest.mark.parametrize("offset,free", [(0.0, True), (-0.3, True), (0.5, True), (100.0, False),
+                                         (1e4, False), (1e5, False)])
+def test_grids_off_the_origin(ctx, offset, free):
+    """Far from the origin the rounding of the coordinates makes the cells
+    differ, and the forms with one shared element matrix are left out: the
+    solution's residual on the assembled matrix stays at the 1e-12 of the
+    stopping test plus the recurrence's own drift, a few eps times the
+    condition number (below 1e4)."""
+    h, n = 0.1, 6
+    xyz, conn, dof, nf, f = block((n, n, n), [h * n] * 3)
+    mesh = msa.Mesh(ctx, xyz + offset, conn, dof, nf)
+    E = 2.1e5 * np.exp(0.3 * np.random.default_rng(2).standard_normal((NS, conn.shape[0])))
+    b = msa.Batch(ctx, [mesh], [NS], L.MSA_FP64, 1)
+    b.set_modulus(0, E)
+    b.set_rhs(0, f)
+    b.assemble(0.3)
+    b.solve(tol=1e-12, max_it=5000, graph_iters=8)
+    assert (b.stats(0)["status"] == msa.MSA_OK).all()
+    assert b.product_form(0) == ("matrix_free" if free else "upper_triangle")
+    rp, col, val = b.matrix_csr(0, 3)
+    u = b.solution(0, 3)
+    r = f - np.array([val[rp[i]:rp[i + 1]] @ u[col[rp[i]:rp[i + 1]]] for i in range(nf)])
+    print(f"\n[case] offset {offset}: true residual {np.linalg.norm(r) / np.linalg.norm(f):.2e}",
+          flush=True)
+    assert np.linalg.norm(r) < 5e-12 * np.linalg.norm(f)
+    # right-hand side of a Newmark step, and the MIXED residuals: one
+    # matrix-free launch each, or one per colour
+    b.set_dynamics(1e-2, 0.5, 1e-3, 0.25, 0.5, 1e-2)
+    b.assemble(0.3)
+    step = lambda: b.newmark(np.array([1.0]), 1, 1e-8, 5000, 0)  # noqa: E731
+    assert residual_launches(b, step) == (1 if free else 8)
+    b.close()
+    b = msa.Batch(ctx, [mesh], [NS], L.MSA_MIXED, 1)
+    b.set_modulus(0, E)
+    b.set_rhs(0, f)
+    b.assemble(0.3)
+    k = residual_launches(b, lambda: b.solve(tol=1e-10, max_it=5000, graph_iters=0))
+    outer = b.stats(0)["outer"].max()
+    assert outer >= 2 and (k < 8 * outer if free else k % 8 == 0)
+    b.close()
+    mesh.close()
