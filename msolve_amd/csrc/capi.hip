@@ -90,6 +90,8 @@ struct msa_batch {
     int n_gitems = 0;
     std::vector<int2> tiles;  // (class, tile) pairs, one reduction workgroup each
     int2 *d_tiles = nullptr;
+    int4 *d_items_run = nullptr;  // the persistent launch's: one-slice chunks in runs of kWaves
+    int n_items_run = 0;
     // [0] PCG active samples, [1] refinement active samples, [2] those of the
     // classes with a hierarchy after the last block (launch_block)
     int *d_counts = nullptr;
@@ -791,8 +793,8 @@ int pcg_loop(msa_batch *b, int kind, double tol, int max_it, int graph_iters)
         ra.active_count = rb.active_count = b->d_counts;
         ra.ir_count = rb.ir_count = b->d_counts + 1;
         int G = 0;
-        MSA_HIP(launch_pcg_persist(b->ctx->stream, is_mixed(b), b->unroll, b->d_cls, b->d_items,
-                                   (int)b->items.size(), b->d_tiles, (int)b->tiles.size(), ra, rb,
+        MSA_HIP(launch_pcg_persist(b->ctx->stream, is_mixed(b), b->unroll, b->d_cls, b->d_items_run,
+                                   b->n_items_run, b->d_tiles, (int)b->tiles.size(), ra, rb,
                                    max_it + 1, b->n_items_mf > 0, b->dyn, &G));
         b->persist_launches++;
         b->persist_grid = G;
@@ -2992,6 +2994,17 @@ int msa_batch_set_persistent(msa_batch *b, int enable)
     MSA_CHECK(b, MSA_ERR_ARG, "null batch");
     MSA_CHECK(!enable || b->T == 1, MSA_ERR_STATE,
               "the persistent launch takes one-sample tiles (the batch has lane tile %d)", b->T);
+    if (enable && !b->d_items_run) {
+        MSA_HIP(hipSetDevice(b->ctx->device));
+        std::vector<int4> items;
+        for (int c = 0; c < (int)b->cls.size(); c++) {
+            if (b->cls[c].chunk == 1)
+                class_run_items(b->cls[c], c, items, kWaves);
+            else
+                class_items(b->cls[c], c, items);
+        }
+        MSA_TRY(items_to_device(b, items, &b->d_items_run, &b->n_items_run));
+    }
     b->persistent = enable != 0;
     return MSA_OK;
 }

@@ -74,6 +74,17 @@ __device__ __forceinline__ void block_partials(double (&v)[NV], double *out)
     }
 }
 
+// The same sums of one wave alone (one-sample tiles): the bits block_partials
+// gives for a chunk that only this wave works on.
+template <int NV>
+__device__ __forceinline__ void wave_partials(double (&v)[NV], double *out)
+{
+#pragma unroll
+    for (int k = 0; k < NV; k++) {
+        v[k] = reduce_rows<1>(v[k]);
+        if ((threadIdx.x & 63) == 0) out[k] = v[k];
+    }
+}
 
 // Three components of one node in one-sample tiles (T = 1 layout: v[3*block
 // + d]) move as a single 12- or 24-byte access.
@@ -1213,7 +1224,9 @@ __device__ __forceinline__ SampleState reduced_state(const ClassDev &C, int smp,
 // Stencil classes of one-sample tiles take the symmetric product above.
 // U: slots per group of a row (the loads of a group issue together; the
 // schedule the autotuner picks); every U sums the slots in the same order.
-template <typename real, int T, int U = 3>
+// RUN: an item of w > 1 covers w one-slice chunks, one per wave (the
+// persistent launch).
+template <typename real, int T, int U = 3, bool RUN = false>
 __device__ __forceinline__ void pcg_a_item(const ClassDev *__restrict__ cls, const int4 it,
                                            int pbuf, const PcgFuse &fz)
 {
@@ -1246,7 +1259,8 @@ __device__ __forceinline__ void pcg_a_item(const ClassDev *__restrict__ cls, con
     const MSA_GLOBAL int *__restrict__ cidx = gbl(C.cidx);
     const MSA_GLOBAL int *__restrict__ sptr = gbl(C.slice_ptr);
     real pq = 0;
-    const int s0 = chunk * C.chunk, s1 = min(s0 + C.chunk, C.nslices);
+    const int run = RUN ? max(1, it.w) : 1;
+    const int s0 = chunk * C.chunk, s1 = min(s0 + run * C.chunk, C.nslices);
     // One slot: gathered p = z + beta p_old of block column col, then the 3x3
     // block times it.  Padding slots (cidx < 0) hold zero values; they read
     // block 0 instead of branching, so the loads of several slots overlap.
@@ -1335,7 +1349,11 @@ __device__ __forceinline__ void pcg_a_item(const ClassDev *__restrict__ cls, con
         }
     }
     double acc[1] = {(double)pq};
-    block_partials<T, 1>(acc, C.partial + ((size_t)tile * C.nchunks + chunk) * 3 * T + fz.slot * T);
+    if (RUN && run > 1) {
+        if (wave < run) wave_partials(acc, C.partial + ((size_t)tile * C.nchunks + chunk + wave) * 3);
+    } else {
+        block_partials<T, 1>(acc, C.partial + ((size_t)tile * C.nchunks + chunk) * 3 * T + fz.slot * T);
+    }
 }
 
 template <typename real, int T, int U = 3>
@@ -1452,7 +1470,8 @@ __device__ __forceinline__ void pcg_p_item(const ClassDev *__restrict__ cls, con
     const int r0 = it.z * C.chunk * 64, r1 = min((it.z + nch) * C.chunk * 64, C.nb);
     for (int br = r0 + (int)threadIdx.x; br < r1; br += blockDim.x) {
         const vec3<real> zc = ld3(z, br), pc = ld3(po, br);
-        st3(pn, br, zc.x + beta * pc.x, zc.y + beta * pc.y, zc.z + beta * pc.z);
+        st3(pn, br, SymRow<real>::fma3(beta, pc.x, zc.x), SymRow<real>::fma3(beta, pc.y, zc.y),
+            SymRow<real>::fma3(beta, pc.z, zc.z));
     }
 }
 
@@ -1511,11 +1530,12 @@ __global__ __launch_bounds__(256) void k_pcg_a_mf(const ClassDev *__restrict__ c
 }
 
 // y = K v for block row br of a box-grid class in FP64 (defined with the
-// smoothing kernels below).
-template <bool DYN>
+// smoothing kernels below).  SUM: v = v + beta v2, formed on the fly.
+template <bool DYN, bool SUM = false>
 __device__ __forceinline__ void mf64_product(const ClassDev &C, const MSA_GLOBAL double *v,
                                              const double *Es, int br, double (&y)[3],
-                                             double (&own)[3]);
+                                             double (&own)[3], const MSA_GLOBAL double *v2 = nullptr,
+                                             double beta = 0.0);
 
 template <bool DYN>
 __device__ __forceinline__ void pcg_a_mf64_item(const ClassDev *__restrict__ cls, const int4 it,
@@ -1550,6 +1570,46 @@ __device__ __forceinline__ void pcg_a_mf64_item(const ClassDev *__restrict__ cls
     }
 }
 
+// The same in the persistent launch: p = z + beta p_old on the fly (same bits
+// as the p pass), since a pass of its own costs a grid-wide barrier, which is
+// most of an iteration there: 32^3 (137 chunks) 106 ms a solve with the
+// pass, 86 without.
+template <bool DYN>
+__device__ __forceinline__ void pcg_a_mf64_run(const ClassDev *__restrict__ cls, const int4 it, int pbuf)
+{
+    const ClassDev &C = cls[it.x];
+    const int tile = it.y, chunk = it.z, run = max(1, it.w);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const bool act = tile < C.nsamp && C.st[tile].active;  // one sample per tile
+    const double beta = act ? C.st[tile].beta : 0.0;
+    const size_t vb = (size_t)tile * C.tile_vec;
+    const MSA_GLOBAL double *__restrict__ z = gbl((const double *)C.z + vb);
+    const MSA_GLOBAL double *__restrict__ po = gbl((const double *)(pbuf ? C.p1 : C.p0) + vb);
+    MSA_GLOBAL double *__restrict__ pn = gbl((double *)(pbuf ? C.p0 : C.p1) + vb);
+    MSA_GLOBAL double *__restrict__ q = gbl((double *)C.q + vb);
+    const double *Es = C.E + (size_t)tile * C.n_elem;
+    double pq = 0.0;
+    const int s0 = chunk * C.chunk, s1 = min(s0 + run * C.chunk, C.nslices);
+    if (act) {
+        for (int slice = s0 + wave; slice < s1; slice += kWaves) {
+            const int br = slice * 64 + lane;
+            if (br >= C.nb) continue;
+            double y[3], own[3];
+            mf64_product<DYN, true>(C, z, Es, br, y, own, po, beta);
+            st3(pn, br, own[0], own[1], own[2]);
+            st3(q, br, y[0], y[1], y[2]);
+            pq += own[0] * y[0] + own[1] * y[1] + own[2] * y[2];
+        }
+    }
+    double acc[1] = {pq};
+    if (run > 1) {
+        if (wave < run) wave_partials(acc, C.partial + ((size_t)tile * C.nchunks + chunk + wave) * 3);
+    } else {
+        block_partials<1, 1>(acc, C.partial + ((size_t)tile * C.nchunks + chunk) * 3);
+    }
+}
+
 template <bool DYN>
 __global__ __launch_bounds__(256) void k_pcg_a_mf64(const ClassDev *__restrict__ cls,
                                                     const int4 *__restrict__ items, int nitems,
@@ -1563,7 +1623,7 @@ __global__ __launch_bounds__(256) void k_pcg_a_mf64(const ClassDev *__restrict__
 // Update + preconditioner + stopping test (SolverPCG.cs:122-136):
 // x += alpha p, r -= alpha q, z = D^-1 r, rz = r.z, rr = r.r; the
 // reduction that follows checks |r|/|b| < tol and forms beta.
-template <typename real, int T>
+template <typename real, int T, bool RUN = false>
 __device__ __forceinline__ void pcg_b_item(const ClassDev *__restrict__ cls, const int4 it,
                                            int pbuf, const PcgFuse &fz)
 {
@@ -1593,7 +1653,8 @@ __device__ __forceinline__ void pcg_b_item(const ClassDev *__restrict__ cls, con
     const MSA_GLOBAL real *__restrict__ q = gbl((const real *)C.q + vb);
     const MSA_GLOBAL real *__restrict__ dinv = gbl((const real *)C.dinv + vb);
     real rz = 0, rr2 = 0;
-    const int s0 = chunk * C.chunk, s1 = min(s0 + C.chunk, C.nslices);
+    const int run = RUN ? max(1, it.w) : 1;
+    const int s0 = chunk * C.chunk, s1 = min(s0 + run * C.chunk, C.nslices);
     if (act) {
 #pragma unroll 2
         for (int slice = s0 + wave; slice < s1; slice += kWaves) {
@@ -1628,7 +1689,11 @@ __device__ __forceinline__ void pcg_b_item(const ClassDev *__restrict__ cls, con
         }
     }
     double acc[2] = {(double)rz, (double)rr2};
-    block_partials<T, 2>(acc, C.partial + ((size_t)tile * C.nchunks + chunk) * 3 * T);
+    if (RUN && run > 1) {
+        if (wave < run) wave_partials(acc, C.partial + ((size_t)tile * C.nchunks + chunk + wave) * 3);
+    } else {
+        block_partials<T, 2>(acc, C.partial + ((size_t)tile * C.nchunks + chunk) * 3 * T);
+    }
 }
 
 template <typename real, int T>
@@ -3065,8 +3130,10 @@ __global__ __launch_bounds__(1024) void k_reduce(const ClassDev *__restrict__ cl
 // (so the same bits).  Work items go to XCDs in contiguous ranges, as
 // xcd_item does.  Every workgroup reads the active-sample count after the
 // same barrier, so all leave the loop together; `iters` bounds it.
-// MF (FP64 batches with matrix-free classes; 2: with the consistent mass):
-// the p pass and its barrier come first.
+// Items of one-slice chunks hold up to kWaves of them (one per wave): a
+// barrier's cost grows with the workgroups, and chunks of one slice would make
+// four times as many (24^3, 235 slices: 97 ms a solve with 240, 32 with
+// 64).  MF: FP64 batches with matrix-free classes (2: with the consistent mass).
 template <typename real, int T, int U, int MF>
 __global__ __launch_bounds__(256) void k_pcg_persist(const ClassDev *__restrict__ cls,
                                                      const int4 *__restrict__ items, int nitems,
@@ -3090,18 +3157,13 @@ __global__ __launch_bounds__(256) void k_pcg_persist(const ClassDev *__restrict_
                                                              __HIP_MEMORY_SCOPE_AGENT)) <= 0)
             break;
         const int pbuf = (pbuf0 + k) & 1;
-        if constexpr (MF != 0) {
-            for (int i = i0; i < i1; i += gx)
-                if (cls[items[i].x].mf_pcg) pcg_p_item<real>(cls, items[i], pbuf, PcgFuse{});
-            barrier();
-        }
         for (int i = i0; i < i1; i += gx) {
             bool mf = false;
             if constexpr (MF != 0) mf = cls[items[i].x].mf_pcg != 0;
             if (!mf) {
-                pcg_a_item<real, T, U>(cls, items[i], pbuf, PcgFuse{});
+                pcg_a_item<real, T, U, true>(cls, items[i], pbuf, PcgFuse{});
             } else {
-                if constexpr (MF != 0) pcg_a_mf64_item<MF == 2>(cls, items[i], pbuf, 0);
+                if constexpr (MF != 0) pcg_a_mf64_run<MF == 2>(cls, items[i], pbuf);
             }
             __syncthreads();
         }
@@ -3112,7 +3174,7 @@ __global__ __launch_bounds__(256) void k_pcg_persist(const ClassDev *__restrict_
         }
         barrier();
         for (int i = i0; i < i1; i += gx) {
-            pcg_b_item<real, T>(cls, items[i], pbuf, PcgFuse{});
+            pcg_b_item<real, T, true>(cls, items[i], pbuf, PcgFuse{});
             __syncthreads();
         }
         barrier();
@@ -3698,10 +3760,11 @@ __device__ __forceinline__ cdouble *mf_khat64(const ClassDev &C)
 // launch, 26 TFLOP/s at 1152 flop a node; 126 us with the element matrix
 // reloaded per (cell, component) in 24 groups of scalar loads.  DYN adds the consistent mass.  Rows of constrained components
 // are zero, as in the stored matrix.
-template <bool DYN>
+template <bool DYN, bool SUM>
 __device__ __forceinline__ void mf64_product(const ClassDev &C, const MSA_GLOBAL double *v,
                                              const double *Es, int br, double (&y)[3],
-                                             double (&own)[3])
+                                             double (&own)[3], const MSA_GLOBAL double *v2,
+                                             double beta)
 {
     const int lane = threadIdx.x & 63;
     const int nx = __builtin_amdgcn_readfirstlane(C.mf_nx);
@@ -3718,6 +3781,13 @@ __device__ __forceinline__ void mf64_product(const ClassDev &C, const MSA_GLOBAL
     const int ne = __builtin_amdgcn_readfirstlane(C.n_elem);
     const __amdgpu_buffer_rsrc_t ub = wave_buffer((const void *)v, (unsigned)nb * 24u);
     const __amdgpu_buffer_rsrc_t eb = wave_buffer((const void *)Es, (unsigned)ne * 8u);
+    __amdgpu_buffer_rsrc_t vb2 = ub;
+    if constexpr (SUM) vb2 = wave_buffer((const void *)v2, (unsigned)nb * 24u);
+    auto load = [&](unsigned o) {
+        double x = buffer_load_f64(ub, (int)o, 0, 0);
+        if constexpr (SUM) x = __builtin_fma(beta, buffer_load_f64(vb2, (int)o, 0, 0), x);
+        return x;
+    };
     const unsigned uout = (unsigned)nb * 24u, eout = (unsigned)ne * 8u;
     const int g = gbl(C.mf_bpos)[br];
     const int i = g & 1023, j = (g >> 10) & 1023, k = g >> 20;
@@ -3764,7 +3834,7 @@ __device__ __forceinline__ void mf64_product(const ClassDev &C, const MSA_GLOBAL
         double xq[9], xm[9], xp[9], ym = 0.0;
 #pragma unroll
         for (int m = 0; m < 9; m++)
-            xq[m] = buffer_load_f64(ub, (int)(off[m] + 8u * q), 0, 0);
+            xq[m] = load(off[m] + 8u * q);
         // lane 0: the column at x - 1, lane 63: at x + 1 (the other lanes'
         // values are replaced by the shifts)
 #pragma unroll
@@ -3774,8 +3844,7 @@ __device__ __forceinline__ void mf64_product(const ClassDev &C, const MSA_GLOBAL
             const unsigned sh = lane == 0 ? (unsigned)-24 : 24u;
 #pragma unroll
             for (int m = 0; m < 9; m++)
-                xm[m] = buffer_load_f64(
-                    ub, (int)((okx && off[m] != uout) ? off[m] + sh + 8u * q : uout), 0, 0);
+                xm[m] = load((okx && off[m] != uout) ? off[m] + sh + 8u * q : uout);
         }
         cdouble *ks = mf_khat64(C) + kMfK64S + 16 * q;
         double kv[16];

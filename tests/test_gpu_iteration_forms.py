@@ -134,3 +134,44 @@ def test_small_batch_forms(ctx, shape, precision):
     assert np.array_equal(*out[2])
     for o in out[1:]:
         assert np.linalg.norm(o[0] - out[0][0]) <= 1e-6 * np.linalg.norm(out[0][0])
+
+
+@pytest.mark.parametrize("dyn", [False, True])
+@pytest.mark.parametrize("shape,ns,form", [((24, 24, 24), 1, "upper_triangle"),
+                                           ((6, 6, 6), 60, "upper_triangle"),
+                                           ((5, 6, 6), 128, "matrix_free"),
+                                           ((6, 6, 6), 100, "matrix_free")])
+def test_persistent_runs_of_one_slice_chunks(ctx, shape, ns, form, dyn):
+    """The persistent launch takes four one-slice chunks per workgroup (its
+    barriers cost by the workgroup) and gives the bits of the captured
+    blocks, with the stored and with the matrix-free product (235, 5, 4 and 5
+    slices a sample)."""
+    xyz, conn = box_mesh(*shape, *[float(v) for v in shape])
+    cons = np.zeros((xyz.shape[0], 3), bool)
+    cons[xyz[:, 0] < 1e-12] = True
+    dof, nf = msa.enumerate_dofs(cons)
+    rng = np.random.default_rng(7)
+    f, E = rng.standard_normal(nf), rng.uniform(1.0, 3.0, (ns, conn.shape[0]))
+    out = []
+    for persistent in (False, True):
+        mesh = msa.Mesh(ctx, xyz, conn, dof, nf)
+        b = msa.Batch(ctx, [mesh], [ns], L.MSA_FP64, 1)
+        b.set_persistent(persistent)
+        b.set_modulus(0, E)
+        b.set_rhs(0, f)
+        if dyn:
+            b.set_dynamics(1e-2, 0.5, 1e-3, 0.25, 0.5, 1e-2)
+        b.assemble(0.3)
+        b.solve(tol=1e-10, max_it=5000, graph_iters=8)
+        assert (b.stats(0)["status"] == msa.MSA_OK).all()
+        assert b.product_form(0) == form
+        out.append((b.stats(0)["iters"], [b.solution(0, s) for s in (0, ns // 2, ns - 1)]))
+        if persistent:
+            slices = -(-(nf // 3) // 64)
+            assert b.persistent_info()["launches"] == 1
+            assert b.persistent_info()["workgroups"] <= 8 * -(-(-(-slices // 4) * ns) // 8)
+        b.close()
+        mesh.close()
+    assert np.array_equal(out[0][0], out[1][0])
+    for u, v in zip(out[0][1], out[1][1]):
+        assert np.array_equal(u, v)
