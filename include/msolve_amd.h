@@ -529,8 +529,8 @@ int msa_batch_get_dynamic_state(msa_batch *b, int cls, int sample, double *u,
                                 double *v, double *a, long long *iters);
 
 /* ----------------------------------------------------------- autotuner
- * Times the SpMV+dot kernel of mesh `mesh` for every lane tile
- * (1..64 samples per wave) with n_samples synthetic samples and writes the
+ * Times the PCG product (SpMV + dot, in the form a Jacobi solve takes) of
+ * mesh `mesh` for every lane tile (1..64 samples per wave) with n_samples synthetic samples and writes the
  * fastest tile to *best_tile; ms_per_tile[7] receives the timings (tiles
  * 1, 2, 4, 8, 16, 32, 64; negative = skipped). */
 int msa_autotune_tile(msa_ctx *ctx, msa_mesh *mesh, int n_samples,

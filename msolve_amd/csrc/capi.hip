@@ -3703,15 +3703,14 @@ int msa_autotune_tile(msa_ctx *ctx, msa_mesh *mesh, int n_samples, int precision
                 rc = MSA_ERR_HIP;
             if (rc == MSA_OK) rc = reduce(b, OP_INIT0);
         }
+        if (rc == MSA_OK) rc = sync_mf_pcg(b);
         if (rc == MSA_OK) {
-            // warm-up, then 10 timed products (pbuf 0 keeps every sample active)
+            // warm-up, then 10 timed products, in the form a Jacobi solve of the
+            // batch takes (pbuf 0 keeps every sample active)
             const int reps = 10;
-            hipError_t e = launch_pcg_a(s, precision == MSA_MIXED, b->T, 3, b->d_cls, b->d_items, ni, 0,
-                                        PcgFuse{});
+            hipError_t e = launch_product(b, 0, PcgFuse{});
             if (e == hipSuccess) e = hipEventRecord(b->timing.e0, s);
-            for (int r = 0; r < reps && e == hipSuccess; r++)
-                e = launch_pcg_a(s, precision == MSA_MIXED, b->T, 3, b->d_cls, b->d_items, ni, 0,
-                                 PcgFuse{});
+            for (int r = 0; r < reps && e == hipSuccess; r++) e = launch_product(b, 0, PcgFuse{});
             if (e == hipSuccess) e = hipEventRecord(b->timing.e1, s);
             if (e == hipSuccess) e = hipEventSynchronize(b->timing.e1);
             float ms = 0;

@@ -97,3 +97,23 @@ def test_back_to_back_spmv_timing(ctx):
         assert np.array_equal(b.solution(0, s), u0[s])
     b.close()
     mesh.close()
+
+
+def test_tile_autotuner_times_the_product_that_runs(ctx):
+    """Tile 1 of msa_autotune_tile on an FP64 box grid (8 samples of 32^3:
+    matrix-free) takes what the batch's own product takes (the stored product
+    is more than three times that); a factor of 2 covers timing noise."""
+    model = msa.cantilever(32, 32, 32, load=-100.0)
+    mesh = msa.Mesh(ctx, model.xyz, model.conn, model.dof, model.n_free)
+    _, table = msa.autotune_tile(ctx, mesh, 8, L.MSA_FP64)
+    b = msa.Batch(ctx, [mesh], [8], L.MSA_FP64, 1)
+    b.set_modulus(0, np.full((8, model.conn.shape[0]), 2.1e5))
+    b.set_rhs(0, model.f)
+    b.assemble(0.3)
+    b.solve(tol=1e-1, max_it=50)
+    assert b.product_form(0) == "matrix_free"
+    own = min(b.time_spmv(10) for _ in range(3))
+    print(f"\n[case] tile 1: {table[1]:.4f} ms, the batch's product {own:.4f} ms", flush=True)
+    assert table[1] < 2.0 * own
+    b.close()
+    mesh.close()
