@@ -12,14 +12,16 @@
 // A sweep walks the factor in blocks of kBandNB = 64 columns, and a block
 // depends on the one before: the time is the number of blocks times the
 // latency of one.  So the 64 x 64 diagonal blocks are inverted once per
-// factorization (k_band_linv, all blocks at once), which turns each serial
-// 64-step substitution into a 64 x 64 product of one parallel step, and both
-// sweeps push a solved block's contribution outwards (forward: the rows
-// below; backward: the rows above), so no block waits on a reduction over
-// rows that another workgroup holds.
+// factorization (in k_chol_block, whose panel needs the inverse too; with
+// zero-energy modes by k_band_linv, all blocks at once), which turns each
+// serial 64-step substitution into a 64 x 64 product of one parallel step.
+// The inverse takes the block's place in the band, so a factor is n W doubles
+// and nothing beside it.  Both sweeps push a solved block's contribution
+// outwards (forward: the rows below; backward: the rows above), so no block
+// waits on a reduction over rows that another workgroup holds.
 //
 // Measured, factorization (MI355X, one 16^3 sample, 217 blocks of width 960):
-// 218 -> 43 us per block, 47 -> 9.3 ms: the diagonal block 137 -> 27 us (the
+// 218 -> 41 us per block, 47 -> 8.9 ms: the diagonal block 137 -> 26 us (the
 // chain of 64 pivots; it was a 64-step loop with two barriers a step), the
 // panel 58 -> 5 us (a product with the inverse instead of a column sweep),
 // the update 23 -> 10.6 us (matrix cores instead of 4 x 4 register tiles
@@ -42,7 +44,6 @@ namespace msa {
 
 namespace {
 
-constexpr int kLinvBlock = 2 * kBandNB * kBandNB;  // doubles per inverted block: by row, by column
 constexpr int kSweepWaves = 8;
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
@@ -129,11 +130,15 @@ __device__ __forceinline__ void invert_lower(const Tile64 &L, Tile64 &X, const d
     __syncthreads();
 }
 
-__device__ __forceinline__ void store_inverse(const Tile64 &X, GLOB double *out, int t)
+// The inverse takes the block's place in the band: it is a lower triangle too,
+// and nothing reads the block itself once its panel is formed.
+__device__ __forceinline__ void store_inverse(const ClassDev &C, GLOB double *AB, int k0, const Tile64 &X,
+                                              int t)
 {
+    const int nk = min(kBandNB, C.bn - k0);
     for (int e = t; e < kBandNB * kBandNB; e += 256) {
-        out[e] = X[e >> 6][e & 63];                      // by row
-        out[kBandNB * kBandNB + e] = X[e & 63][e >> 6];  // by column
+        const int c = e >> 6, r = e & 63;
+        if (r >= c && r < nk) AB[(size_t)(k0 + c) * C.bW + (r - c)] = X[r][c];
     }
 }
 
@@ -149,19 +154,22 @@ __device__ __forceinline__ void load_diag(const ClassDev &C, const GLOB double *
     }
 }
 
-// Inverse of every diagonal block of every factor: grid (block, sample).
+// Inverse of every diagonal block of every factor, in place: grid (block,
+// sample).
 __global__ __launch_bounds__(256) void k_band_linv(const ClassDev *__restrict__ cp)
 {
     __shared__ Tile64 L, X;
     __shared__ double rd[kBandNB];
     const ClassDev &C = *cp;
     const int t = threadIdx.x, smp = blockIdx.y;
-    load_diag(C, glob((const double *)C.band + (size_t)smp * C.band_ss), blockIdx.x * kBandNB, L, t);
+    const int k0 = blockIdx.x * kBandNB;
+    GLOB double *AB = glob(C.band + (size_t)smp * C.band_ss);
+    load_diag(C, AB, k0, L, t);
     __syncthreads();
     if (t < kBandNB) rd[t] = 1.0 / L[t][t];
     __syncthreads();
     invert_lower(L, X, rd, t);
-    store_inverse(X, glob(C.linv + (size_t)smp * C.linv_ss + (size_t)blockIdx.x * kLinvBlock), t);
+    store_inverse(C, AB, k0, X, t);
 }
 
 // ------------------------------------------------------------ factorization
@@ -185,7 +193,6 @@ __global__ __launch_bounds__(256) void k_chol_block(const ClassDev *__restrict__
     __shared__ double rd[kBandNB];
     const ClassDev &C = *cp;
     const int smp = blockIdx.y, t = threadIdx.x, lane = t & 63, wave = t >> 6;
-    const int nk = min(kBandNB, C.bn - k0);
     GLOB double *AB = glob(C.band + (size_t)smp * C.band_ss);
     load_diag(C, AB, k0, L, t);
     __syncthreads();
@@ -239,12 +246,8 @@ __global__ __launch_bounds__(256) void k_chol_block(const ClassDev *__restrict__
         __syncthreads();
     }
     if (t == 0 && fail) C.bfail[smp] = 1;
-    for (int e = t; e < kBandNB * kBandNB; e += 256) {
-        const int c = e >> 6, rr = e & 63;
-        if (rr >= c && rr < nk) AB[(size_t)(k0 + c) * C.bW + (rr - c)] = L[rr][c];
-    }
     invert_lower(L, X, rd, t);
-    store_inverse(X, glob(C.linv + (size_t)smp * C.linv_ss + (size_t)(k0 / kBandNB) * kLinvBlock), t);
+    store_inverse(C, AB, k0, X, t);
 }
 
 // Panel rows [r0, r0 + m), r0 = k0 + 64: L21 = A21 L11^-T as a product with
@@ -259,8 +262,8 @@ __global__ __launch_bounds__(256) void k_chol_panel_inv(const ClassDev *__restri
     const int i0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 16;  // row - r0
     if (i0 >= m) return;
     GLOB double *P = glob(C.band + (size_t)smp * C.band_ss) + (size_t)k0 * W + kBandNB + i0 + r;
-    const GLOB double *LI = glob((const double *)C.linv + (size_t)smp * C.linv_ss +
-                                 (size_t)(k0 / kBandNB) * kLinvBlock + kBandNB * kBandNB);
+    // entry (row, col) of the inverse (col <= row) at LI[col (W - 1) + row]
+    const GLOB double *LI = glob((const double *)C.band + (size_t)smp * C.band_ss) + (size_t)k0 * W;
     double a[16];  // A21[row][4 q + g]
 #pragma unroll
     for (int q = 0; q < 16; q++) a[q] = P[(size_t)(4 * q + g) * (W - 1)];
@@ -269,8 +272,11 @@ __global__ __launch_bounds__(256) void k_chol_panel_inv(const ClassDev *__restri
     for (int ct = 0; ct < 4; ct++) {
         s[ct] = f64x4{0, 0, 0, 0};
 #pragma unroll
-        for (int q = 0; q < 4 * (ct + 1); q++)
-            s[ct] = MFMA64(LI[(4 * q + g) * kBandNB + 16 * ct + r], a[q], s[ct]);
+        for (int q = 0; q < 4 * (ct + 1); q++) {
+            const double l = LI[(size_t)(4 * q + g) * (W - 1) + 16 * ct + r];
+            const bool low = q < 4 * ct || r >= 4 * (q - 4 * ct) + g;
+            s[ct] = MFMA64(low ? l : 0.0, a[q], s[ct]);
+        }
     }
     if (i0 + r >= m) return;
 #pragma unroll
@@ -327,32 +333,6 @@ __global__ __launch_bounds__(256) void k_chol_update_mfma(const ClassDev *__rest
 
 // ------------------------------------------------------------------- sweeps
 
-// Row `t / P` (P = threads / 64 lanes per row) of the inverted block times
-// the block's right-hand side y: a thread takes 64 / P columns, the P lanes
-// of a row sum by DPP.  m: the block's inverse, by row (forward) or by
-// column (backward, the transpose).
-struct LinvRow {
-    f64x2 v[4];
-};
-__device__ __forceinline__ LinvRow load_linv(const GLOB double *m, int t)
-{
-    LinvRow r;
-    const GLOB f64x2 *p = (const GLOB f64x2 *)(m + (t >> 3) * kBandNB + (t & 7) * 8);
-#pragma unroll
-    for (int k = 0; k < 4; k++) r.v[k] = p[k];
-    return r;
-}
-__device__ __forceinline__ double linv_times(const LinvRow &r, const double *y, int t)
-{
-    double s = 0.0;
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        s += r.v[k].x * y[(t & 7) * 8 + 2 * k];
-        s += r.v[k].y * y[(t & 7) * 8 + 2 * k + 1];
-    }
-    return sum8(s);
-}
-
 // Range-checked view of `bytes` bytes at p (the same in the whole wave):
 // loads past the end return zeros.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t wave_view(const GLOB double *p, unsigned bytes)
@@ -362,6 +342,50 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t wave_view(const GLOB double *p
     const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(a >> 32));
     return __builtin_amdgcn_make_buffer_rsrc((void *)(((unsigned long long)hi << 32) | lo), (short)0,
                                              (int)__builtin_amdgcn_readfirstlane(bytes), 0x00020000);
+}
+
+// Row t / 8 of the inverted block (backward: of its transpose) times the
+// block's right-hand side y: lane p of the 8 of a row takes columns 2 p + 16 j
+// (+ 1), so that a backward load covers 128 contiguous bytes, and the 8 lanes
+// sum by DPP.  The block lies in the band at byte `base` of the view `ab`,
+// entry (row, col) at col (W - 1) + row; `out` is an offset past the view.
+// Backward, the entries of the other triangle are the unused (zero) end of
+// the column before; columns past the band's end (a last, partial block) are
+// out of range.
+struct LinvRow {
+    f64x2 v[4];
+};
+template <bool FWD>
+__device__ __forceinline__ LinvRow load_linv(__amdgpu_buffer_rsrc_t ab, unsigned base, unsigned out, int W,
+                                             int t)
+{
+    LinvRow l;
+    const unsigned i = (unsigned)t >> 3, w1 = (unsigned)W - 1;
+#pragma unroll
+    for (unsigned k = 0; k < 4; k++) {
+        const unsigned j = 2 * (t & 7) + 16 * k;
+        if constexpr (FWD) {
+            const unsigned o = base + (j * w1 + i) * 8u;
+            l.v[k].x = __builtin_bit_cast(
+                double, __builtin_amdgcn_raw_buffer_load_b64(ab, (int)(j <= i ? o : out), 0, 0));
+            l.v[k].y = __builtin_bit_cast(
+                double, __builtin_amdgcn_raw_buffer_load_b64(ab, (int)(j < i ? o + w1 * 8u : out), 0, 0));
+        } else {
+            l.v[k] = __builtin_bit_cast(
+                f64x2, __builtin_amdgcn_raw_buffer_load_b128(ab, (int)(base + (i * w1 + j) * 8u), 0, 0));
+        }
+    }
+    return l;
+}
+__device__ __forceinline__ double linv_times(const LinvRow &r, const double *y, int t)
+{
+    double s = 0.0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        s += r.v[k].x * y[2 * (t & 7) + 16 * k];
+        s += r.v[k].y * y[2 * (t & 7) + 16 * k + 1];
+    }
+    return sum8(s);
 }
 
 // A wave's share of a panel: the 64 rows of row block rb next to solved
@@ -452,13 +476,14 @@ __device__ __forceinline__ void sweep_sample(const ClassDev &C, int smp, int swe
     const int n = C.bn, W = C.bW, nblk = (n + kBandNB - 1) / kBandNB, nwb = W / kBandNB;
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    // bytes of the factor and of a block of columns
+    const unsigned nw = (unsigned)n * (unsigned)W * 8u, bw = kBandNB * (unsigned)W * 8u;
     const __amdgpu_buffer_rsrc_t ab =
-        wave_view(glob((const double *)C.band + (size_t)smp * C.band_ss), (unsigned)n * (unsigned)W * 8u);
-    const GLOB double *LI = glob((const double *)C.linv + (size_t)smp * C.linv_ss);
+        wave_view(glob((const double *)C.band + (size_t)smp * C.band_ss), nw);
     GLOB double *y = glob(C.by + (size_t)smp * n);
     if (sweeps & 1) {
         for (int i = t; i < W; i += 64 * kSweepWaves) yw[i] = i < n ? y[i] : 0.0;
-        LinvRow li = load_linv(LI, t);
+        LinvRow li = load_linv<true>(ab, 0, nw, W, t);
         __syncthreads();
         for (int k = 0; k < nblk; k++) {
             const int k0 = k * kBandNB, slot = (k % nwb) * kBandNB;
@@ -472,7 +497,7 @@ __device__ __forceinline__ void sweep_sample(const ClassDev &C, int smp, int swe
                 xb[t >> 3] = x;
                 if (k0 + (t >> 3) < n) y[k0 + (t >> 3)] = x;
             }
-            if (k + 1 < nblk) li = load_linv(LI + (size_t)(k + 1) * kLinvBlock, t);
+            if (k + 1 < nblk) li = load_linv<true>(ab, (k + 1) * bw, nw, W, t);
             __syncthreads();
             if (wave < nrb) yw[((k + 1 + wave) % nwb) * kBandNB + lane] -= panel_times<true>(p, xb, lane);
             if (wave == kSweepWaves - 1) yw[slot + lane] = yin;
@@ -481,12 +506,12 @@ __device__ __forceinline__ void sweep_sample(const ClassDev &C, int smp, int swe
     }
     if (sweeps & 2) {
         __syncthreads();
-        const int kl = nblk - 1, ow = kBandNB * kBandNB;
+        const int kl = nblk - 1;
         for (int j = wave; j < min(nwb, nblk); j += kSweepWaves) {
             const int i = (kl - j) * kBandNB + lane;
             yw[((kl - j) % nwb) * kBandNB + lane] = i < n ? y[i] : 0.0;
         }
-        LinvRow li = load_linv(LI + (size_t)kl * kLinvBlock + ow, t);
+        LinvRow li = load_linv<false>(ab, kl * bw, nw, W, t);
         __syncthreads();
         for (int k = kl; k >= 0; k--) {
             const int k0 = k * kBandNB, slot = (k % nwb) * kBandNB;
@@ -500,7 +525,7 @@ __device__ __forceinline__ void sweep_sample(const ClassDev &C, int smp, int swe
                 xb[t >> 3] = x;
                 if (k0 + (t >> 3) < n) y[k0 + (t >> 3)] = x;
             }
-            if (k > 0) li = load_linv(LI + (size_t)(k - 1) * kLinvBlock + ow, t);
+            if (k > 0) li = load_linv<false>(ab, (k - 1) * bw, nw, W, t);
             __syncthreads();
             if (wave < nrb)
                 yw[((k - 1 - wave) % nwb) * kBandNB + (lane & 7) * 8 + (lane >> 3)] -=
@@ -552,18 +577,32 @@ __global__ __launch_bounds__(64 * kSweepWaves) void k_mg_band_solve(const ClassD
     }
 }
 
+// Sums of two rows spread over the two halves of a wave: lane l < 32 gets a of
+// lanes l and l + 32, lane l + 32 gets b of them.
+__device__ __forceinline__ double sum_halves(double a, double b)
+{
+    const unsigned long long ua = __builtin_bit_cast(unsigned long long, a);
+    const unsigned long long ub = __builtin_bit_cast(unsigned long long, b);
+    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)ua, (unsigned)ub, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(ua >> 32), (unsigned)(ub >> 32), false, false);
+    return __builtin_bit_cast(double, ((unsigned long long)hi[0] << 32) | lo[0]) +
+           __builtin_bit_cast(double, ((unsigned long long)hi[1] << 32) | lo[1]);
+}
+
 // One block of a sweep over many workgroups (wide bands, where one
 // workgroup cannot stream a panel fast enough): every workgroup forms the
 // block's solution from the right-hand side in `src` and subtracts its
 // share of 64 rows there; workgroup 0 writes the solution to `dst`, another
 // buffer, since the others still read the block.  The 8 waves split the
-// panel's columns (forward) or rows (backward).
+// panel's columns (forward) or rows (backward).  Forward, loads of 16 bytes
+// along the columns: 3.6 us a launch (8 samples of 12^3), 4.1 with the 8-byte
+// loads of sweep_sample.
 // Forward: by -> bx, backward: bx -> by.
 template <bool FWD>
 __global__ __launch_bounds__(64 * kSweepWaves) void k_band_sweep_step(
     const ClassDev *__restrict__ cp, int k, int mode)
 {
-    __shared__ double yb[kBandNB], xb[kBandNB], red[FWD ? kSweepWaves : 1][kBandNB];
+    __shared__ double yb[kBandNB], xb[kBandNB], red[FWD ? 2 : 1][FWD ? kSweepWaves : 1][kBandNB];
     const ClassDev &C = *cp;
     const int smp = blockIdx.y;
     if (!served(C, smp, mode)) return;
@@ -571,49 +610,92 @@ __global__ __launch_bounds__(64 * kSweepWaves) void k_band_sweep_step(
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
     const GLOB double *AB = glob((const double *)C.band + (size_t)smp * C.band_ss);
-    const GLOB double *LI = glob((const double *)C.linv + (size_t)smp * C.linv_ss);
     GLOB double *src = glob((FWD ? C.by : C.bx) + (size_t)smp * n);
     GLOB double *dst = glob((FWD ? C.bx : C.by) + (size_t)smp * n);
     const int k0 = k * kBandNB, rb = blockIdx.x;
     const bool rows = rb < (FWD ? min(nblk - 1 - k, nwb - 1) : min(k, nwb - 1));
-    const LinvRow li =
-        load_linv(LI + (size_t)k * kLinvBlock + (FWD ? 0 : kBandNB * kBandNB), t);
-    if (t < kBandNB) yb[t] = k0 + t < n ? src[k0 + t] : 0.0;
+    const unsigned nw = (unsigned)min(kBandNB, n - k0) * (unsigned)W * 8u;  // bytes of the block's columns
+    const __amdgpu_buffer_rsrc_t ab = wave_view(AB + (size_t)k0 * W, nw);
     constexpr int kc = kBandNB / kSweepWaves;
-    double pv[kc];
-    f64x2 pt[4];
-    const int i = FWD ? k0 + kBandNB * (1 + rb) + lane
+    LinvRow li;
+    f64x2 lc[4], pt[4];
+    double ys[4];
+    // Forward, a wave takes 8 columns, each half of it every other one, a lane
+    // two rows: 16-byte loads along the band's columns
+    const int half = lane >> 5, l2 = 2 * (lane & 31), row = l2 + half;
+    const int i = FWD ? k0 + kBandNB * (1 + rb) + row
                       : k0 - kBandNB * (1 + rb) + kc * wave + (lane >> 3);
-    if (rows) {
-        if constexpr (FWD) {
-            const GLOB double *a =
-                AB + (size_t)k0 * W + (i - k0) + (size_t)(kc * wave) * (W - 1);
+    if constexpr (FWD) {
+        // right-hand sides by scalar loads (past the band's end any value:
+        // there the inverse's columns read as zeros)
+        const auto *sp = (__attribute__((address_space(4))) const double *)(unsigned long long)src;
 #pragma unroll
-            for (int c = 0; c < kc; c++) pv[c] = a[(size_t)c * (W - 1)];
-        } else {
-            const GLOB double *a = AB + (size_t)i * W + (k0 - i) + 2 * (lane & 7);
-#pragma unroll
-            for (int j = 0; j < 4; j++) pt[j] = *(const GLOB f64x2u *)(a + 16 * j);
+        for (int j = 0; j < 4; j++) {
+            const int col = kc * wave + 2 * j;
+            lc[j] = __builtin_bit_cast(
+                f64x2, __builtin_amdgcn_raw_buffer_load_b128(
+                           ab, (int)(col + half <= l2 + 1 ? (unsigned)((col + half) * (W - 1) + l2) * 8u : nw),
+                           0, 0));
+            const double y0 = sp[min(k0 + col, n - 1)], y1 = sp[min(k0 + col + 1, n - 1)];
+            ys[j] = half ? y1 : y0;
         }
+    } else {
+        li = load_linv<false>(ab, 0, nw, W, t);
+        if (t < kBandNB) yb[t] = k0 + t < n ? src[k0 + t] : 0.0;
     }
-    __syncthreads();
-    const double x = linv_times(li, yb, t);
-    if ((t & 7) == 0) {
-        xb[t >> 3] = x;
-        if (rb == 0 && k0 + (t >> 3) < n) dst[k0 + (t >> 3)] = x;
+    if (rows) {
+        const GLOB double *a = FWD ? AB + (size_t)k0 * W + kBandNB * (1 + rb) + l2 +
+                                         (size_t)(kc * wave + half) * (W - 1)
+                                   : AB + (size_t)i * W + (k0 - i) + 2 * (lane & 7);
+#pragma unroll
+        for (int j = 0; j < 4; j++) pt[j] = *(const GLOB f64x2u *)(a + (FWD ? (size_t)2 * j * (W - 1) : 16 * j));
     }
-    __syncthreads();
+    // the block's solution: forward, row `row` in every wave, backward in xb
+    double x = 0.0;
+    if constexpr (FWD) {
+        double a = 0.0, b = 0.0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            a += lc[j].x * ys[j];
+            b += lc[j].y * ys[j];
+        }
+        red[0][wave][lane] = sum_halves(a, b);
+        __syncthreads();
+        const auto &p = red[0];
+        x = ((p[0][lane] + p[1][lane]) + (p[2][lane] + p[3][lane])) +
+            ((p[4][lane] + p[5][lane]) + (p[6][lane] + p[7][lane]));
+        if (rb == 0 && wave == 0 && k0 + row < n) dst[k0 + row] = x;
+    } else {
+        __syncthreads();
+        x = linv_times(li, yb, t);
+        if ((t & 7) == 0) {
+            xb[t >> 3] = x;
+            if (rb == 0 && k0 + (t >> 3) < n) dst[k0 + (t >> 3)] = x;
+        }
+        __syncthreads();
+    }
     if (!rows) return;  // the whole workgroup
     double s = 0.0;
     if constexpr (FWD) {
+        double xs[4];
 #pragma unroll
-        for (int c = 0; c < kc; c++) s += pv[c] * xb[kc * wave + c];
-        red[wave][lane] = s;
+        for (int j = 0; j < 4; j++) {
+            const double x0 = lane_f64(x, 4 * wave + j), x1 = lane_f64(x, 4 * wave + j + 32);
+            xs[j] = half ? x1 : x0;
+        }
+        double a = 0.0, b = 0.0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            a += pt[j].x * xs[j];
+            b += pt[j].y * xs[j];
+        }
+        s = sum_halves(a, b);
+        red[1][wave][lane] = s;
         __syncthreads();
         if (wave > 0 || i >= n) return;
-        s = red[0][lane];
+        s = red[1][0][lane];
 #pragma unroll
-        for (int w = 1; w < kSweepWaves; w++) s += red[w][lane];
+        for (int w = 1; w < kSweepWaves; w++) s += red[1][w][lane];
         src[i] -= s;
     } else {
 #pragma unroll

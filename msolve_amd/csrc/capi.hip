@@ -947,13 +947,10 @@ int band_setup(msa_batch *b, ClassHost &C, bool *changed, bool shared = false)
     }
     const size_t per = (size_t)C.dev.bn * C.dev.bW;
     const size_t need = shared ? per : (size_t)C.nsamp * per;
-    const size_t lper = (size_t)((C.dev.bn + kBandNB - 1) / kBandNB) * 2 * kBandNB * kBandNB;
     if (C.band_cap < need) {
         void *p = nullptr;
         MSA_TRY(dalloc(b, &p, need * sizeof(double)));
         C.dev.band = (double *)p;
-        MSA_TRY(dalloc(b, &p, (shared ? 1 : C.nsamp) * lper * sizeof(double)));
-        C.dev.linv = (double *)p;
         C.band_cap = need;
         upload = true;
     }
@@ -972,7 +969,6 @@ int band_setup(msa_batch *b, ClassHost &C, bool *changed, bool shared = false)
     const long long ss = shared ? 0 : (long long)per;
     if (C.dev.band_ss != ss) {
         C.dev.band_ss = ss;
-        C.dev.linv_ss = shared ? 0 : (long long)lper;
         upload = true;
     }
     if (upload) *changed = true;
@@ -987,8 +983,8 @@ int prepare_band(msa_batch *b)
     return MSA_OK;
 }
 
-// Band Cholesky factors of ns samples and the inverses of their diagonal
-// blocks, which the sweeps read.  zem: with zero-energy modes.
+// Band Cholesky factors of ns samples, their diagonal blocks replaced by the
+// inverses, which the sweeps read.  zem: with zero-energy modes.
 int band_factor(msa_batch *b, const ClassDev *cp, int n, int W, int ns, bool zem = false)
 {
     hipStream_t s = b->ctx->stream;

@@ -5088,41 +5088,47 @@ __global__ void k_mg_load(const ClassDev *__restrict__ cp, const double *__restr
 
 // Dense inverse X = (L L^T)^-1 of every sample's band Cholesky factor
 // (coarsest multigrid levels, bn <= kDenseMax): one wavefront per column j
-// of one sample; forward L y = e_j and backward L^T x = y with the column
-// in LDS, each row's band sum split over the 64 lanes and reduced by
-// shuffles.  X is symmetric: column j is written as row j (contiguous).
+// of one sample; forward L y = e_j and backward L^T x = y by 64-row blocks
+// (lane = row) with the column in LDS, each block by its inverse, which the
+// factor holds in the block's place.  X is symmetric: column j is written as
+// row j (contiguous).
 __global__ __launch_bounds__(64) void k_band_inverse(const ClassDev *__restrict__ cp)
 {
-    __shared__ double y[kDenseMax];
+    __shared__ double y[kDenseMax], tb[kBandNB];
     const ClassDev &C = *cp;
     const int smp = blockIdx.y, j = blockIdx.x, lane = threadIdx.x;
-    const int n = C.bn, W = C.bW;
+    const int n = C.bn, W = C.bW, nblk = (n + kBandNB - 1) / kBandNB;
     const MSA_GLOBAL double *L = gbl(C.band + (size_t)smp * C.band_ss);
-    for (int i = lane; i < n; i += 64) y[i] = 0.0;
+    for (int i = lane; i < kDenseMax; i += 64) y[i] = 0.0;
     __syncthreads();
-    // forward: y_i = (delta_ij - sum_{k in [max(j, i-W+1), i)} L_ik y_k) / L_ii
-    for (int i = j; i < n; i++) {
-        double part = 0.0;
-        for (int k2 = max(j, i - W + 1) + lane; k2 < i; k2 += 64)
-            part += L[(size_t)k2 * W + (i - k2)] * y[k2];
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) part += __shfl_xor(part, off, 64);
-        const double yi = ((i == j ? 1.0 : 0.0) - part) / L[(size_t)i * W];
+    for (int kb = j / kBandNB; kb < nblk; kb++) {
+        const int k0 = kb * kBandNB, i = k0 + lane;
+        double v = i == j ? 1.0 : 0.0;
+#pragma unroll 8
+        for (int k2 = j; k2 < k0; k2++)
+            v -= (i < n && i - k2 < W ? L[(size_t)k2 * W + (i - k2)] : 0.0) * y[k2];
+        tb[lane] = v;
         __syncthreads();
-        if (lane == 0) y[i] = yi;
+        double yi = 0.0;
+#pragma unroll 8
+        for (int c = 0; c < kBandNB; c++)
+            yi += (i < n && c <= lane ? L[(size_t)(k0 + c) * W + (lane - c)] : 0.0) * tb[c];
+        if (i < n) y[i] = yi;
         __syncthreads();
     }
-    // backward: x_i = (y_i - sum_{k in (i, min(n, i+W))} L_ki x_k) / L_ii
-    for (int i = n - 1; i >= 0; i--) {
-        double part = 0.0;
-        const int kend = min(n, i + W);
-        for (int k2 = i + 1 + lane; k2 < kend; k2 += 64)
-            part += L[(size_t)i * W + (k2 - i)] * y[k2];
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) part += __shfl_xor(part, off, 64);
-        const double xi = (y[i] - part) / L[(size_t)i * W];
+    for (int kb = nblk - 1; kb >= 0; kb--) {
+        const int k0 = kb * kBandNB, i = k0 + lane;
+        double v = i < n ? y[i] : 0.0;
+#pragma unroll 8
+        for (int k2 = k0 + kBandNB; k2 < n; k2++)
+            v -= (i < n && k2 - i < W ? L[(size_t)i * W + (k2 - i)] : 0.0) * y[k2];
+        tb[lane] = v;
         __syncthreads();
-        if (lane == 0) y[i] = xi;
+        double xi = 0.0;
+#pragma unroll 8
+        for (int r = 0; r < kBandNB; r++)
+            xi += (k0 + r < n && r >= lane ? L[(size_t)i * W + (r - lane)] : 0.0) * tb[r];
+        if (i < n) y[i] = xi;
         __syncthreads();
     }
     MSA_GLOBAL double *X = gbl(C.binvd + (size_t)smp * n * n + (size_t)j * n);

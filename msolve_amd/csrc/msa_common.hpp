@@ -206,8 +206,6 @@ struct ClassDev {
                           // sample uses the one factor at band (first-sample preconditioner)
     double *by;           // [nsamp][bn] right-hand side / solution in band order
     double *bx;           // [nsamp][bn] second buffer of the sweeps of wide bands (null: narrow)
-    double *linv;         // [nsamp][blocks][2][64*64] inverted diagonal blocks, by row and by column
-    long long linv_ss;    // doubles between two samples' (0: one shared factor)
     int *bfail;           // [nsamp] non-positive pivot met
     // zero-energy modes of the direct solver's factorization (zv null: off):
     // a pivot of magnitude under zem_tol is set to 1 and its row and column

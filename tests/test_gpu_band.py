@@ -113,3 +113,23 @@ def test_zero_energy_modes_of_a_wide_band(ctx):
         assert np.abs(b.spmv(0, 0, Z[j])).max() <= 1e-9 * scale * np.abs(Z[j]).max()
     b.close()
     mesh.close()
+
+
+@pytest.mark.parametrize("shape,ns", [((4, 4, 4), 5), ((12, 3, 3), 2), ((9, 8, 8), 3)])
+def test_factor_memory(ctx, shape, ns):
+    """A factorization takes the band storage msa_batch_direct_info reports
+    (n W doubles a sample) and a few vectors beside it (right-hand side, the
+    second buffer of wide bands, the two permutations)."""
+    model = msa.cantilever(*shape, load=-100.0)
+    mesh = msa.Mesh(ctx, model.xyz, model.conn, model.dof, model.n_free)
+    b = msa.Batch(ctx, [mesh], [ns], L.MSA_FP64, 1)
+    b.set_modulus(0, np.full((ns, model.conn.shape[0]), 2.1e5))
+    b.set_rhs(0, model.f)
+    b.assemble(0.3)
+    before, info = b.device_bytes, b.direct_info(0)
+    b.factorize()
+    extra = b.device_bytes - before - ns * info["bytes_per_sample"]
+    print(f"\n[case] {shape} width {info['width']}: {extra / ns / info['n']:.1f} bytes a row beside the band")
+    assert 0 <= extra <= ns * info["n"] * 24 + 4096
+    b.close()
+    mesh.close()
