@@ -2765,10 +2765,15 @@ int newmark_head(msa_batch *b, const DynCoef &dc, double tol, int max_it)
     const bool mx = is_mixed(b);
     const int T = b->T, ni = (int)b->items.size(), ncol = max_colours(b);
     MSA_TRY(timed(b, KK_OTHER, [&] { return launch_dyn_prep(s, mx, T, b->d_cls, b->d_items, ni, dc); }));
-    // box grids of equal cells matrix-free (64 samples of 48x48x24: 2.4 ms
-    // per step for the 8 colours), the element scatter for the others
-    const bool mfres = mf_residual(b);
-    const bool mfrhs = mx ? mfres : b->n_items_mf > 0;
+    // grids of equal cells matrix-free (64 samples of 48x48x24: 2.4 ms per
+    // step for the 8 colours of the right-hand side; box grids only), the
+    // element scatter for the others
+    bool mfres = false, mfrhs = !mx && b->n_items_mf > 0;
+    for (auto &C : b->cls) {
+        const bool e = mx && C.dev.mf_r && C.dev.mf_exact;
+        mfres = mfres || e;
+        mfrhs = mfrhs || (e && C.dev.mf_box);
+    }
     if (mfrhs)
         MSA_TRY(timed(b, KK_RES64, [&] {
             return launch_dyn_rhs_mf(s, dc.betaR != 0.0, b->d_cls, mx ? b->mf_box_items : b->d_items_mf,

@@ -135,8 +135,10 @@ def test_what_keeps_the_stored_product(ctx):
                                   dict(shape=(8, 4, 6), roller=True)])
 def test_newmark_step_forms(ctx, grid, beta, precision):
     """A Newmark run on a grid of equal cells (right-hand side and first
-    residual matrix-free) against the same grid with one plane moved by
-    1e-12, which keeps the element-by-element kernels: steps solved to 1e-11
+    residual matrix-free, one launch each) against the same grid with one
+    plane moved by 1e-12, which keeps the element-by-element kernels (one
+    launch per colour; the MIXED replacements, here every second iteration,
+    are matrix-free on both): steps solved to 1e-11
     agree to that, amplified over the steps."""
     xyz, conn, dof, nf, f = block(**grid)
     bent = xyz.copy()
@@ -158,6 +160,15 @@ def test_newmark_step_forms(ctx, grid, beta, precision):
         b.assemble(0.3)
         b.newmark(acc, 1, 1e-11, 20000, 8)
         out.append([(b.history(0, s), *b.dynamic_state(0, s)[:3]) for s in (0, ns - 1)])
+        per = 1 if x is xyz else mesh.info["colours"]
+        b.set_kernel_timing(True)
+        b.newmark(acc[:1], 1, 1e-8, 20000, 8)
+        n = {k: v["launches"] for k, v in b.kernel_timing().items()}
+        b.set_kernel_timing(False)
+        if precision == L.MSA_FP64:
+            assert n["residual64"] == per
+        else:
+            assert n["residual64"] == 2 * per + n["spmv_dot"] // 2
         b.close()
         mesh.close()
     for a, c in zip(*out):
