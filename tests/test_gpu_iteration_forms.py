@@ -59,6 +59,15 @@ def test_partial_hierarchy_equals_separate_batches(ctx, precision, method, graph
     assert both[odd][0].min() > 2 * both[cube][0].max()  # the cycle was left out for a while
 
 
+def launches(b, run):
+    """Launches of run() by kernel kind (timed, so eager)."""
+    b.set_kernel_timing(True)
+    run()
+    t = b.kernel_timing()
+    b.set_kernel_timing(False)
+    return {k: v["launches"] for k, v in t.items()}
+
+
 @pytest.mark.parametrize("dyn", [False, True])
 @pytest.mark.parametrize("shape,lengths,roller", [((5, 4, 3), (5.0, 4.0, 3.0), False),
                                                   ((70, 2, 2), (35.0, 1.5, 1.0), True),
@@ -66,7 +75,8 @@ def test_partial_hierarchy_equals_separate_batches(ctx, precision, method, graph
 def test_mixed_residual_without_hierarchy(ctx, shape, lengths, roller, dyn):
     """Jacobi MIXED batches from 128 chunks on form the FP64 residual
     matrix-free: the first samples against a batch of those alone (too few
-    chunks: the coloured residual).  Both stop at a true relative residual of
+    chunks: the coloured residual).  A replacement every 8 iterations is one
+    launch there, one per colour here.  Both stop at a true relative residual of
     1e-11; the blocks' condition is below 1e4 (70 x 2 x 2: clamped along the
     side)."""
     xyz, conn = box_mesh(*shape, *lengths)
@@ -90,7 +100,13 @@ def test_mixed_residual_without_hierarchy(ctx, shape, lengths, roller, dyn):
         b.solve(tol=1e-11, max_it=5000, graph_iters=8)
         assert (b.stats(0)["status"] == msa.MSA_OK).all()
         u = [b.solution(0, s) for s in range(3)]
+        per = 1 if ns == 130 else mesh.info["colours"]
+        n = launches(b, lambda: b.solve(tol=1e-11, max_it=5000, graph_iters=8))
+        assert n["spmv_dot"] >= 8 and n["residual64"] == per * (n["spmv_dot"] // 8)
         if dyn:
+            n = launches(b, lambda: b.newmark(np.ones(1), 0, 1e-8, 5000, 8))
+            # the step's right-hand side and first residual too
+            assert n["residual64"] == per * (2 + n["spmv_dot"] // 8)
             b.newmark(np.linspace(1.0, 0.5, 4), acc_dir=0, tol=1e-11, max_it=5000, graph_iters=8)
             u += [v for s in range(3) for v in b.dynamic_state(0, s)[:3]]
         out.append(u)

@@ -260,3 +260,18 @@ def test_grids_off_the_origin(ctx, offset, free):
     assert outer >= 2 and (k < 8 * outer if free else k % 8 == 0)
     b.close()
     mesh.close()
+
+
+@pytest.mark.parametrize("ns", [830, 1700])
+def test_product_over_runs_of_chunks(ctx, ns):
+    """Large batches give a workgroup of the FP64 product runs of chunks (5
+    chunks a sample: from 4096 of them runs of 2, 2 and 1, from 8192 of 4 and
+    1).  The persistent launch takes one chunk at a time: the same bits."""
+    blk = block((10, 10, 10))
+    E = 2.1e5 * np.exp(0.3 * np.random.default_rng(8).standard_normal((ns, blk[1].shape[0])))
+    ua, ia, fa = solve(ctx, blk, ns, E, "matrix_free")
+    up, ip, fp = solve(ctx, blk, ns, E, "matrix_free", persistent=True)
+    assert (fa, fp) == ("matrix_free", "matrix_free")
+    assert np.array_equal(ia, ip)
+    for a, c in zip(ua, up):
+        assert np.array_equal(a, c)
