@@ -27,15 +27,21 @@
 // the update 23 -> 10.6 us (matrix cores instead of 4 x 4 register tiles
 // through LDS).
 //
-// Measured, sweeps (with the factorization before that change): the first-sample preconditioner on 8
-// samples of 12^3 (6084 rows, width 576, 22 applications) 525 -> 37.5 ms,
-// the sweeps of a 16^3 direct solve (13872 rows) 48 -> 1.6 ms, against a
-// launch pair per block and sweep with 64-step substitutions.  Both sweeps
-// in one launch and one workgroup take 4.5 us per block at width 576, what
-// one CU can load; a launch per block 3.6 us whatever the width.  So wide
-// bands take the launches (37.5 against 42 ms at width 576), and narrow ones
-// the one launch, which also costs an idle multigrid cycle next to nothing
-// (17 ragged samples, coarsest level of width 384: 85 against 203 ms).
+// Measured, sweeps: against a launch pair per block and sweep with 64-step
+// substitutions, eight first-sample solves of 12^3 (6084 rows, width 576, 22
+// applications) 525 -> 37.5 ms, the sweeps of a 16^3 direct solve (13872 rows)
+// 48 -> 1.6 ms.  Wide bands take a launch per block, narrow ones both sweeps
+// in one launch and one workgroup, whose CU then loads the whole panel (width
+// 512: 62 GB/s).  us a block and sweep, with an iteration's other kernels:
+//   samples, width     1, 576   8, 320   8, 512   8, 576   64, 320   64, 512   64, 576
+//   launch per block     12.3     3.66     3.71     3.59      3.78      4.57      4.63
+//   one launch            4.8     4.06     4.26     4.51      4.06      4.22      4.42
+// (one sample: the first application, which is not captured).  The line lies
+// at width 512: up to there a launch per block gains at most 15%, and loses 8%
+// with many samples, while in one launch an idle multigrid cycle costs next to
+// nothing (17 ragged samples, width 384: 85 against 203 ms, when cycles still
+// ran idle) and uncaptured launches a third; wider, few samples lose 25% in
+// one launch, and eight waves of 64 rows end it at 576 anyway.
 #include <hip/hip_runtime.h>
 
 #include "msa_common.hpp"
@@ -550,7 +556,7 @@ __global__ __launch_bounds__(64 * kSweepWaves) void k_band_sweep_one(const Class
 // Coarsest multigrid levels, all classes of the batch at once: items are
 // (class, sample), one workgroup each, which also moves the level's
 // right-hand side into band order and the solution back.  A sample's sweeps
-// are a serial chain of 2.8 us a block, so a batch's classes one after the
+// are a serial chain of 3.3 us a block and sweep, so a batch's classes one after the
 // other waited for the sum of their chains instead of the longest: 17 samples
 // over four meshes (coarsest chains of 53, 23 and 9 blocks) 31.1 -> 26.4 ms.
 template <typename real>

@@ -649,9 +649,9 @@ bool part_hierarchy(const msa_batch *b)
 // Whether the iterations apply their reductions inside the product and the
 // update (reduced_state): one-sample tiles, no preconditioner launches between
 // update and reduction, at most kFoldChunks chunks a sample.  An iteration of
-// short launches is then two instead of four: 10^3 FP64 (5 chunks) 20.7 -> 16
-// us an iteration, 32 mixed 24^3 samples (59 chunks) 47.5 -> 43.4 ms, 64 FP64
-// 32^3 (137 chunks) 139 -> 134 ms.  Samples of more chunks keep k_reduce, two
+// short launches is then two instead of four: one FP64 10^3 solve (19 one-slice
+// chunks) 3.69 -> 2.69 ms, 17 ragged mixed samples 27.8 -> 26.4, 32 mixed 24^3
+// (59 chunks) 40.3 -> 37.5, 64 FP64 32^3 (137 chunks) 134.6 -> 133.6.  Samples of more chunks keep k_reduce, two
 // 5 us launches of an iteration of 100 us and up (64^3: 1057 chunks), where
 // every workgroup would read more partials than rows.
 bool fold_reductions(const msa_batch *b, bool cycle)
